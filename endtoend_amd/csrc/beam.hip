@@ -727,7 +727,10 @@ struct PvcsArgs {
     v3 bev_lo, bev_hi;          // dilated crop box (BEV index units)
 };
 
-// One lane per PVCS voxel, 16x4x4 voxel tiles in XCD-aware order.  Voxels outside the dilated
+// One lane per PVCS voxel, 16x4x4 voxel tiles in XCD-aware order, each wave a 4x4x4 cube of the
+// tile: the gathers are bound by the number of different cache lines per load, and the cones run in
+// every direction, so the shape with the least projected area (24 voxels on average, against 42 for a
+// 16x4x1 slab) touches the fewest REV lines.  Voxels outside the dilated
 // crop box receive nothing from any cone and leave at once; the others sum every cone's trilinear
 // REV dose (compact store, REV2XYZdose's fetch) in a register and add it to the dose volume once.
 __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
@@ -739,7 +742,7 @@ __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
     const int txi = (int)(tile % (uint32_t)a.tx);
     const int tyi = (int)((tile / (uint32_t)a.tx) % (uint32_t)a.ty);
     const int tzi = (int)(tile / ((uint32_t)a.tx * (uint32_t)a.ty));
-    const int X = txi * 16 + (tid & 15), Y = tyi * 4 + ((tid >> 4) & 3), Z = tzi * 4 + (tid >> 6);
+    const int X = txi * 16 + (tid >> 6) * 4 + (tid & 3), Y = tyi * 4 + ((tid >> 2) & 3), Z = tzi * 4 + ((tid >> 4) & 3);
     if (X >= a.sx || Y >= a.sy || Z >= a.sz) return;
     const int gx = a.x0 + X, gy = a.y0 + Y, gz = a.z0 + Z;
     const v3 g = mk3((float)gx, (float)gy, (float)gz);
@@ -777,33 +780,19 @@ __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
             if (!(ub > -1.f && vb > -1.f && wb > -1.f && ub < (float)c.nx && vb < (float)c.ny && wb < (float)c.nz))
                 continue;
             const float fu = floorf(ub), fv = floorf(vb), fw = floorf(wb);
-            const int i = (int)fu, j = (int)fv, k = (int)fw;
             ok[u] = true;
-            di[u] = i;
+            di[u] = (int)fu;
             fa[u] = ub - fu;
             fb[u] = vb - fv;
             fc[u] = wb - fw;
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int jj = j + (t & 1), kk = k + (t >> 1);
-                if (jj >= 0 && jj < c.ny && kk >= 0 && kk < c.nz)
-                    mt[u][t] = a.lines[c.line0 + (uint64_t)jj + (uint64_t)c.ny * kk];
-            }
+            meta_pairs(a.lines, c.line0, c.ny, c.nz, (int)fv, (int)fw, mt[u]);
         }
 #pragma unroll
         for (int u = 0; u < kPvcsGroup; u++) {
             if (!ok[u]) continue;
             float tv[4];
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const LineMeta m = mt[u][t];
-                const int d = di[u] - m.i0;
-                const bool vlo = d >= 0 && d < m.len, vhi = d + 1 >= 0 && d + 1 < m.len;
-                const float x0 = a.rev[vlo ? m.off + (uint32_t)d : 0u];
-                const float x1 = a.rev[vhi ? m.off + (uint32_t)(d + 1) : 0u];
-                const float lo = vlo ? x0 : 0.f, hi = vhi ? x1 : 0.f;
-                tv[t] = lo + fa[u] * (hi - lo);
-            }
+            for (int t = 0; t < 4; t++) tv[t] = rev_lerp(a.rev, mt[u][t], di[u], fa[u]);
             const float e0 = tv[0] + fb[u] * (tv[1] - tv[0]);
             const float e1 = tv[2] + fb[u] * (tv[3] - tv[2]);
             sum += e0 + fc[u] * (e1 - e0);
@@ -1229,7 +1218,8 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     ConeDev* d_cones = nullptr;
     LineMeta* d_lines = nullptr;
     CCCS_TRY(S.get(ctx->cones, kMaxRays, &d_cones));
-    CCCS_TRY(S.get(ctx->lines, g.total_lines, &d_lines));
+    CCCS_TRY(S.get(ctx->lines, g.total_lines + 2 * kRevPad, &d_lines));
+    d_lines += kRevPad;
     ConeDev* hc = S.host_cones;
     dm33 bfwd = dm_beam_fwd(b.azimuth, b.zenith, b.coll);
     dm33 binv = dm_beam_inv(b.azimuth, b.zenith, b.coll);
@@ -1344,7 +1334,8 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     uint32_t cls_n[kConeClasses];
     std::memcpy(cls_n, S.host_small + 4, sizeof(cls_n));
     const uint64_t stored = (uint64_t)last.off + (uint64_t)last.len;
-    CCCS_TRY(S.get(ctx->rev, stored, &ca.rev));
+    CCCS_TRY(S.get(ctx->rev, stored + 2 * kRevPad, &ca.rev));
+    ca.rev += kRevPad;
     // pass 2: per-line resample + walks into the compact store, one workgroup per listed line
     ca.ramp_min = ctx->sched.cone_ramp_min;
     int tok = prof_begin(ctx, K_CONE);

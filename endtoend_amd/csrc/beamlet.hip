@@ -1570,6 +1570,10 @@ BlArgs base_args(cccs_ctx* ctx) {
     return a;
 }
 
+// Line table and REV store with the pads of rev_fetch's pair loads.
+inline size_t line_bytes(uint64_t n) { return sizeof(LineMeta) * (size_t)(n + 2 * kRevPad); }
+inline size_t rev_bytes(uint64_t n) { return sizeof(float) * (size_t)(n + 2 * kRevPad); }
+
 inline unsigned grid_for(uint64_t n, unsigned block) { return (unsigned)std::min<uint64_t>((n + block - 1) / block, 1u << 20); }
 
 // `while_busy` (may be empty) runs on the host once every launch of the job's first pass is
@@ -1592,8 +1596,8 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     uint8_t* d = ctx->bl_tab.as<uint8_t>();
     CCCS_HIP(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, ctx->stream));
     CCCS_TRY(ctx->bl_pdose.ensure(sizeof(float) * std::max<uint64_t>(1, J.pdose)));
-    CCCS_TRY(ctx->lines.ensure(sizeof(LineMeta) * std::max<uint64_t>(1, J.max_lines)));
-    CCCS_TRY(ctx->rev.ensure(sizeof(float) * std::max<uint64_t>(1, J.max_rev)));
+    CCCS_TRY(ctx->lines.ensure(line_bytes(J.max_lines)));
+    CCCS_TRY(ctx->rev.ensure(rev_bytes(J.max_rev)));
     CCCS_TRY(ctx->bl_h.ensure(sizeof(float) * std::max<uint64_t>(1, J.max_rev)));
     CCCS_TRY(ctx->bl_qcnt.ensure(sizeof(uint32_t) * (size_t)std::max(1, nrays)));
     CCCS_TRY(ctx->h_small.ensure(sizeof(uint32_t) * kMaxRays + 64));
@@ -1605,8 +1609,8 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     BlArgs a = base_args(ctx);
     a.batches = reinterpret_cast<const BatchDev*>(d);
     a.beamlets = reinterpret_cast<const BeamletDev*>(d + o_l);
-    a.lines = ctx->lines.as<LineMeta>();
-    a.rev = ctx->rev.as<float>();
+    a.lines = ctx->lines.as<LineMeta>() + kRevPad;
+    a.rev = ctx->rev.as<float>() + kRevPad;
     a.pdose = ctx->bl_pdose.as<float>();
     a.nbatch = nb;
     CCCS_TRY(ctx->bl_tiles.ensure(sizeof(uint32_t) * std::max<uint32_t>(1, J.tiles)));
@@ -1635,8 +1639,8 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     }
     for (int k = 0; k < nset; k++) CCCS_TRY(set_cone[k]->ensure(sizeof(uint32_t) * std::max<uint64_t>(1, J.max_lines)));
     for (int k = 1; k < nset; k++) {
-        CCCS_TRY(set_lines[k]->ensure(sizeof(LineMeta) * std::max<uint64_t>(1, J.max_lines)));
-        CCCS_TRY(set_rev[k]->ensure(sizeof(float) * std::max<uint64_t>(1, J.max_rev)));
+        CCCS_TRY(set_lines[k]->ensure(line_bytes(J.max_lines)));
+        CCCS_TRY(set_rev[k]->ensure(rev_bytes(J.max_rev)));
         CCCS_TRY(set_h[k]->ensure(sizeof(float) * std::max<uint64_t>(1, J.max_rev)));
     }
     for (int attempt = 0; attempt < 3; attempt++) {
@@ -1665,9 +1669,9 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
             // the helpers (line scan, profiling events) enqueue on ctx->stream and use ctx->scan
             ctx->stream = S[k];
             std::swap(ctx->scan, *set_scan[k]);
-            a.lines = set_lines[k]->as<LineMeta>();
+            a.lines = set_lines[k]->as<LineMeta>() + kRevPad;
             a.line_cone = set_cone[k]->as<uint32_t>();
-            a.rev = set_rev[k]->as<float>();
+            a.rev = set_rev[k]->as<float>() + kRevPad;
             float* H = set_h[k]->as<float>();
             TermaReq* q = set_q[k]->as<TermaReq>();
             do {
@@ -1843,14 +1847,14 @@ int run_plain_batch(cccs_ctx* ctx, const std::vector<BeamPlan>& plans, const Bat
     }
     if (max_rev > 0xffffffffULL) return set_error(CCCS_EGEOM, "REV grid exceeds 2^32 samples");
     CCCS_TRY(ctx->bl_pdose.ensure(sizeof(float) * std::max<uint64_t>(1, J.pdose)));
-    CCCS_TRY(ctx->lines.ensure(sizeof(LineMeta) * std::max<uint64_t>(1, max_lines)));
-    CCCS_TRY(ctx->rev.ensure(sizeof(float) * std::max<uint64_t>(1, max_rev)));
+    CCCS_TRY(ctx->lines.ensure(line_bytes(max_lines)));
+    CCCS_TRY(ctx->rev.ensure(rev_bytes(max_rev)));
     CCCS_TRY(ctx->bl_h.ensure(sizeof(float) * 2 * std::max<uint64_t>(1, max_rev)));
     BlArgs a = base_args(ctx);
     a.batches = reinterpret_cast<const BatchDev*>(d);
     a.beamlets = reinterpret_cast<const BeamletDev*>(d + o_l);
-    a.lines = ctx->lines.as<LineMeta>();
-    a.rev = ctx->rev.as<float>();
+    a.lines = ctx->lines.as<LineMeta>() + kRevPad;
+    a.rev = ctx->rev.as<float>() + kRevPad;
     a.pdose = ctx->bl_pdose.as<float>();
     a.nbatch = 1;
     float* dd = ctx->bl_h.as<float>();

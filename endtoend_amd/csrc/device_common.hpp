@@ -63,14 +63,58 @@ __device__ __forceinline__ LineMeta line_of_lane(const LineMeta& m, int lane) {
     return r;
 }
 
+// Entries kept before and after a line table and a REV store, so that a pair load at an end stays
+// inside the allocation (128 bytes of the store: lines keep their alignment).
+constexpr int kRevPad = 32;
+
+// Two consecutive entries as one load (the address is a multiple of the entry, not of the pair).
+typedef float pair_f32 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t pair_meta __attribute__((ext_vector_type(4), aligned(8)));
+
+__device__ __forceinline__ LineMeta meta_of(uint32_t off, uint32_t w, bool in) {
+    LineMeta r;
+    r.off = off;
+    r.i0 = (int16_t)(w & 0xffffu);
+    r.len = in ? (int16_t)(w >> 16) : (int16_t)0;
+    return r;
+}
+
+// Records of lines (j, k), (j+1, k), (j, k+1), (j+1, k+1) of a grid of ny x nz lines, j in [-1, ny-1],
+// k in [-1, nz-1]; lines outside the grid get length 0.
+__device__ __forceinline__ void meta_pairs(const LineMeta* __restrict__ meta, uint64_t line0, int ny, int nz, int j, int k,
+                                           LineMeta m[4]) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int kk = k + h;
+        const bool row = kk >= 0 && kk < nz;
+        const LineMeta* p = meta + line0 + (uint64_t)(row ? kk : 0) * (uint64_t)ny + (int64_t)j;
+        const pair_meta r = *reinterpret_cast<const pair_meta*>(p);
+        m[2 * h] = meta_of(r.x, r.y, row && j >= 0);
+        m[2 * h + 1] = meta_of(r.z, r.w, row && j + 1 < ny);
+    }
+}
+
+// Samples i and i+1 of a stored line (zero outside its interval), interpolated at fraction a.
+__device__ __forceinline__ float rev_lerp(const float* __restrict__ rev, const LineMeta& m, int i, float a) {
+    const int d = i - m.i0;
+    const bool vlo = d >= 0 && d < m.len, vhi = d + 1 >= 0 && d + 1 < m.len;
+    const pair_f32 x = *reinterpret_cast<const pair_f32*>(rev + (vlo || vhi ? (int64_t)m.off + (int64_t)d : (int64_t)0));
+    const float lo = vlo ? x.x : 0.f, hi = vhi ? x.y : 0.f;
+    return lo + a * (hi - lo);
+}
+
 // Trilinear fetch from a compactly stored REV grid (nx samples per line, ny x nz lines) at texture
 // coordinates (u, v, w) = (sample, line y, line z), texel centres at +0.5, border 0: the same
 // operation sequence as tex3_border on the dense grid, so both give identical results.
 //
-// The loads are branch-free and issued in two rounds: the four line records together, then the
-// eight samples together, so a lane waits for two memory round trips instead of one per tap.  A
-// tap outside the grid reads the grid's first record and a sample outside its line's stored
-// interval reads sample 0 of the store (both valid addresses); either is then replaced by zero.
+// The loads are branch-free and issued in two rounds: the line records together, then the samples
+// together, so a lane waits for two memory round trips instead of one per tap.  Neighbouring taps
+// are neighbours in memory (lines j and j+1 of the table, samples i and i+1 of a line), so a pair is
+// one load: two for the four records and four for the eight samples.  A gather of lanes on different
+// lines costs the L1 one lookup per lane and load, so halving the loads halves the stage's bound
+// (with the 4x4x4-voxel waves of pvcs_kernel: 472 -> 277 us per 4-cone pass of a 256x256x180 beam).  A
+// tap outside the grid or outside its line's stored interval is replaced by zero; its pair may read
+// one entry before or after the table or the store (kRevPad entries on both sides).
 __device__ __forceinline__ float rev_fetch(const LineMeta* __restrict__ meta, const float* __restrict__ rev,
                                            uint64_t line0, int nx, int ny, int nz, float u, float v, float w) {
     if (ny <= 0 || nz <= 0) return 0.f;
@@ -80,23 +124,10 @@ __device__ __forceinline__ float rev_fetch(const LineMeta* __restrict__ meta, co
     const int i = (int)fu, j = (int)fv, k = (int)fw;
     const float a = ub - fu, b = vb - fv, c = wb - fw;
     LineMeta m[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int jj = j + (q & 1), kk = k + (q >> 1);
-        const bool in = jj >= 0 && jj < ny && kk >= 0 && kk < nz;
-        m[q] = meta[in ? line0 + (uint64_t)jj + (uint64_t)ny * (uint64_t)kk : line0];
-        if (!in) m[q].len = 0;
-    }
+    meta_pairs(meta, line0, ny, nz, j, k, m);
     float t[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int d = i - m[q].i0;
-        const bool vlo = d >= 0 && d < m[q].len, vhi = d + 1 >= 0 && d + 1 < m[q].len;
-        const float x0 = rev[vlo ? m[q].off + (uint32_t)d : 0u];
-        const float x1 = rev[vhi ? m[q].off + (uint32_t)(d + 1) : 0u];
-        const float lo = vlo ? x0 : 0.f, hi = vhi ? x1 : 0.f;
-        t[q] = lo + a * (hi - lo);
-    }
+    for (int q = 0; q < 4; q++) t[q] = rev_lerp(rev, m[q], i, a);
     const float e0 = t[0] + b * (t[1] - t[0]);
     const float e1 = t[2] + b * (t[3] - t[2]);
     return e0 + c * (e1 - e0);
