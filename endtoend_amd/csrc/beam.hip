@@ -311,16 +311,22 @@ __device__ __forceinline__ void line_interval(const ConeArgs& a, const ConeDev& 
 //  * the radiological distance from destination j to sample k is a difference of the line's
 //    radiological coordinates: rho_k = P - c_k backward (P = boundary between j-1 and j, c_k the
 //    centre of sample k) and c_k - P forward (P = boundary between j and j+1);
-//  * the cumulative kernel C is linear on each radial interval (R_{s-1}, R_s]:
-//    C(rho) = beta_s + sigma_s * rho;
 //  * summing by parts, sum_k T_k (C(rho_k) - C(rho_{k+1})) = sum_k (T_k - T_{k-1}) C(rho_k) + one
-//    end term, so a run of samples in one interval contributes
-//    (beta_s + sigma_s P)(T_hi - T_{lo-1}) - sigma_s (E[hi+1] - E[lo]) with E the prefix sum of
-//    (T_k - T_{k-1}) c_k (FP64).
-// The samples of each interval are found by a lookup in a uniform table over the radiological
-// coordinate.  The walk's exits (distance beyond the last radius, entering the last interval) become
-// the first/last sample of the sum.  Same result as the sequential walk up to FP32 rounding of the
-// accumulated distance.
+//    end term, with C the cumulative kernel;
+//  * C is linear on each radial interval (R_{s-1}, R_s] with slope sigma_s and C(0) = 0, so it is a
+//    sum of ramps: C(rho) = sum_s sigma_s (max(rho - R_{s-1}, 0) - max(rho - R_s, 0)).
+// Hence the backward sum is sum_s sigma_s (F(P - R_{s-1}) - F(P - R_s)) with
+// F(y) = sum_{c_k < y} (T_k - T_{k-1}) (y - c_k) = T_{q-1} y - E[q], q the first sample with c_q >= y
+// and E the FP64 prefix sum of (T_k - T_{k-1}) c_k; the forward sum is its mirror image.  F is
+// continuous, so a tie in the search for q does not matter, and one evaluation of F per radius is
+// all that a destination costs: a lookup in a uniform table over the radiological coordinate, one
+// probe of two centres, one multiply-add.  The walk's exits (distance beyond the last radius,
+// entering the last interval) end the sum at one sample a: F(c_a) is then the constant that F
+// starts from; a line that fits into the radii has no such end.  Same result as the sequential walk
+// up to FP32 rounding of the accumulated distance.  The cone kernel issues VALU instructions in 92-98 %
+// of its cycles, so a walk is as fast as its instructions are few: interval sums with a search loop per
+// interval (about 55 per radius and direction) took 11.8 ms of a 256x256x180 request, this form (28)
+// 8.9 ms.
 struct RampLine {
     const float* c;       // centres, radiological cm from the segment start; c[n..n+3] = +inf
     const double* E;      // E[k]  = sum_{m<k} (T_m - T_{m-1}) c_m   (T_{-1} = 0), k in [0, n]
@@ -331,16 +337,27 @@ struct RampLine {
     float c0, cn, invD;
 };
 
-// first k with c_k >= y
-CCCS_HD int ramp_lb(const RampLine& L, float y) {
-    if (!(y > L.c0)) return 0;
-    if (y > L.cn) return L.n;
+// The search for the first k with c_k >= y (y <= c_{n-1}): a table lookup and two probes (one LDS
+// load), no branch.  A cell holds at most one centre where the density is at least half the line's
+// mean; `more` says that both probed centres lie below y, so that ramp_more has to go on from k.
+struct RampPos {
+    int u, k;
+    bool more;
+};
+CCCS_HD RampPos ramp_probe(const RampLine& L, float y) {
+    RampPos p;
     // biased by 1% of a cell so that the cell's threshold never exceeds y after rounding
-    int u = (int)((y - L.c0) * L.invD - 0.01f);
-    u = min(max(u, 0), L.U - 1);
-    int k = L.lb[u];
-    if (L.lb[u + 1] - k > 8) {  // a crowded cell (low density): bisect up to the next cell's end
-        int hi = L.lb[u + 2];
+    p.u = min(max((int)((y - L.c0) * L.invD - 0.01f), 0), L.U - 1);
+    const int k = L.lb[p.u];
+    const float ca = L.c[k], cb = L.c[k + 1];
+    p.more = cb < y;
+    p.k = k + (ca < y ? 1 : 0) + (p.more ? 1 : 0);
+    return p;
+}
+CCCS_HD int ramp_more(const RampLine& L, float y, const RampPos& p) {
+    int k = p.k;
+    if (L.lb[p.u + 1] - k > 8) {  // a crowded cell (low density): bisect up to the next cell's end
+        int hi = L.lb[p.u + 2];
         while (k < hi) {
             const int mid = (k + hi) >> 1;
             if (L.c[mid] < y) k = mid + 1; else hi = mid;
@@ -349,85 +366,100 @@ CCCS_HD int ramp_lb(const RampLine& L, float y) {
     while (L.c[k] < y) k++;
     return k;
 }
+CCCS_HD int ramp_lb(const RampLine& L, float y) {
+    const RampPos p = ramp_probe(L, y);
+    return p.more ? ramp_more(L, y, p) : p.k;
+}
 
-// first k with c_k > y
+// first k with c_k > y, for y < c_{n-1}
 CCCS_HD int ramp_ub(const RampLine& L, float y) {
-    if (y < L.c0) return 0;
-    if (!(y < L.cn)) return L.n;
-    int u = (int)((y - L.c0) * L.invD - 0.01f);
-    u = min(max(u, 0), L.U - 1);
-    int k = L.lb[u];
-    if (L.lb[u + 1] - k > 8) {
-        int hi = L.lb[u + 2];
-        while (k < hi) {
-            const int mid = (k + hi) >> 1;
-            if (L.c[mid] <= y) k = mid + 1; else hi = mid;
-        }
-    }
+    int k = y < L.c0 ? 0 : ramp_lb(L, y);
     while (L.c[k] <= y) k++;
     return k;
 }
 
-// Backward walk of destination j (toward lower indices), kernel row given as sigma/beta.
-CCCS_HD double ramp_back(const RampLine& L, int j, const double* __restrict__ sig,
-                                            const double* __restrict__ beta, const float* __restrict__ R, int nr,
-                                            uint32_t& iters) {
-    if (j == 0) return 0.0;
-    const float2 ep = L.s[j - 1];
-    const double P = (double)L.c[j - 1] + (double)ep.x;
-    const int nlast = ramp_lb(L, (float)(P - (double)R[nr - 1]));
-    const int nprev = ramp_lb(L, (float)(P - (double)R[nr - 2]));
-    const int a = max(nlast, nprev - 1);  // last sample the walk reaches
-    if (a >= j) return 0.0;
-    double sum = 0.0, Thi = (double)ep.y, Ehi = L.E[j];
-    int hiend = j;
-    for (int s = 0; s < nr; s++) {
-        int ns = s == nr - 1 ? nlast : (s == nr - 2 ? nprev : ramp_lb(L, (float)(P - (double)R[s])));
-        ns = max(ns, a);
-        if (ns < hiend) {  // samples [ns, hiend) lie in interval s
-            const double Tlo = ns > 0 ? (double)L.s[ns - 1].y : 0.0;
-            const double Elo = L.E[ns];
-            sum += (beta[s] + sig[s] * P) * (Thi - Tlo) - sig[s] * (Ehi - Elo);
-            if (ns == a) sum += Tlo * (beta[s] + sig[s] * (P - (double)L.c[a]));
-            hiend = ns;
-            Thi = Tlo;
-            Ehi = Elo;
-            iters++;
+// The backward (toward lower indices) and / or forward walk of destination j, the kernel rows given
+// by their slopes.  Both directions step through the radii together, so that their lookups (two
+// dependent LDS trips each) overlap.
+template <bool kBack, bool kFwd>
+CCCS_HD double ramp_walk(const RampLine& L, int j, const double* __restrict__ sigb, const double* __restrict__ sigf,
+                         const float* __restrict__ R, int nr, uint32_t& iters) {
+    // F starts at the boundary of the destination and ends, at Fa / Eb, at the centre ya / yb of the
+    // last sample that the walk reaches; a walk without samples ends at once.  (Forward, F is taken
+    // without its constant: E2[q] + T_q y.)
+    double Pb = 0.0, Pf = 0.0, Fb = 0.0, Ff = 0.0, Fa = 0.0, Eb = 0.0;
+    float ya = INFINITY, yb = -INFINITY;
+    const bool exits = L.cn - L.c0 > R[nr - 2];
+    if (kBack && j > 0) {
+        const float2 e = L.s[j - 1];
+        Pb = (double)L.c[j - 1] + (double)e.x;
+        int a = 0;
+        if (exits) {
+            const float yl = (float)(Pb - (double)R[nr - 1]), yp = (float)(Pb - (double)R[nr - 2]);
+            a = max(yl > L.c0 ? ramp_lb(L, yl) : 0, (yp > L.c0 ? ramp_lb(L, yp) : 0) - 1);
         }
-        if (hiend == a) break;
+        if (a < j) {
+            ya = L.c[a];
+            if (a > 0) Fa = fma((double)L.s[a - 1].y, (double)ya, -L.E[a]);
+            Fb = fma((double)e.y, Pb, -L.E[j]);
+        }
+    }
+    if (kFwd && j < L.n - 1) {
+        const float2 e = L.s[j + 1];
+        Pf = (double)L.c[j + 1] - (double)e.x;
+        int b = L.n - 1;
+        if (exits) {
+            const float yl = (float)(Pf + (double)R[nr - 1]), yp = (float)(Pf + (double)R[nr - 2]);
+            const int ml = yl < L.cn ? ramp_ub(L, yl) - 1 : b, mp = yp < L.cn ? ramp_ub(L, yp) - 1 : b;
+            b = min(ml, mp + 1);
+        }
+        if (b > j) {
+            yb = L.c[b];
+            Eb = L.E2[b + 1];
+            if (b < L.n - 1) Eb = fma((double)L.s[b + 1].y, (double)yb, Eb);
+            Ff = fma((double)e.y, Pf, L.E2[j + 1]);
+        }
+    }
+    double sum = 0.0;
+    for (int s = 0; s < nr; s++) {
+        const double r = (double)R[s];
+        const double y0 = Pb - r, y1 = Pf + r;
+        const bool in0 = kBack && (float)y0 > ya, in1 = kFwd && (float)y1 < yb;
+        const float z0 = in0 ? (float)y0 : L.c0, z1 = in1 ? (float)y1 : L.c0;
+        RampPos p0{0, 0, false}, p1{0, 0, false};
+        if (kBack) p0 = ramp_probe(L, z0);
+        if (kFwd) p1 = ramp_probe(L, z1);
+        if (p0.more || p1.more) {
+            if (p0.more) p0.k = ramp_more(L, z0, p0);
+            if (p1.more) p1.k = ramp_more(L, z1, p1);
+        }
+        if (kBack) {
+            const int q = max(p0.k, 1);
+            const double Fs = fma((double)L.s[q - 1].y, y0, -L.E[q]);
+            const double d = in0 ? Fs : Fa;
+            sum = fma(sigb[s], Fb - d, sum);
+            Fb = d;
+        }
+        if (kFwd) {
+            const double Fs = fma((double)L.s[p1.k].y, y1, L.E2[p1.k]);
+            const double d = in1 ? Fs : Eb;
+            sum = fma(sigf[s], d - Ff, sum);
+            Ff = d;
+        }
+        iters++;
+        if (!in0 && !in1) break;
     }
     return sum;
 }
 
-// Forward walk of destination j (toward higher indices).
-CCCS_HD double ramp_fwd(const RampLine& L, int j, const double* __restrict__ sig,
-                                           const double* __restrict__ beta, const float* __restrict__ R, int nr,
-                                           uint32_t& iters) {
-    if (j >= L.n - 1) return 0.0;
-    const float2 en = L.s[j + 1];
-    const double P = (double)L.c[j + 1] - (double)en.x;
-    const int mlast = ramp_ub(L, (float)(P + (double)R[nr - 1])) - 1;
-    const int mprev = ramp_ub(L, (float)(P + (double)R[nr - 2])) - 1;
-    const int b = min(mlast, mprev + 1);  // last sample the walk reaches
-    if (b <= j) return 0.0;
-    double sum = 0.0, Tlo = (double)en.y, Elo = L.E2[j + 1];
-    int lo = j + 1;
-    for (int s = 0; s < nr; s++) {
-        int ms = s == nr - 1 ? mlast : (s == nr - 2 ? mprev : ramp_ub(L, (float)(P + (double)R[s])) - 1);
-        ms = min(ms, b);
-        if (ms >= lo) {  // samples [lo, ms] lie in interval s
-            const double Thi = ms + 1 < L.n ? (double)L.s[ms + 1].y : 0.0;
-            const double Ehi = L.E2[ms + 1];
-            sum += (beta[s] - sig[s] * P) * (Tlo - Thi) + sig[s] * (Ehi - Elo);
-            if (ms == b) sum += Thi * (beta[s] + sig[s] * ((double)L.c[b] - P));
-            lo = ms + 1;
-            Tlo = Thi;
-            Elo = Ehi;
-            iters++;
-        }
-        if (lo > b) break;
-    }
-    return sum;
+// One direction alone, for a caller that also holds the rows' intercepts (the line checks).
+CCCS_HD double ramp_back(const RampLine& L, int j, const double* sig, const double*, const float* R, int nr,
+                         uint32_t& iters) {
+    return ramp_walk<true, false>(L, j, sig, nullptr, R, nr, iters);
+}
+CCCS_HD double ramp_fwd(const RampLine& L, int j, const double* sig, const double*, const float* R, int nr,
+                        uint32_t& iters) {
+    return ramp_walk<false, true>(L, j, nullptr, sig, R, nr, iters);
 }
 
 // First cell u in [0, nu] whose threshold c0 + u * D exceeds v (nu when none does): an estimate
@@ -506,7 +538,7 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     constexpr int NW = NT / 64;
     extern __shared__ double s_dyn[];
     __shared__ float sR[kMaxRadii], sIW[kMaxRadii], sF[kMaxRadii], sB[kMaxRadii];
-    __shared__ double sSig[2][kMaxRadii], sBeta[2][kMaxRadii];
+    __shared__ double sSig[2][kMaxRadii];
     __shared__ double s_tot[NW];
     __shared__ int s_red[NW][3];
     __shared__ uint32_t s_cnt[NW];
@@ -612,14 +644,11 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
             if (j < vlo || j > vhi) out[j] = 0.f;
         const int n = vhi - vlo + 1;
         if (n >= a.ramp_min && nvalid == n) {
-            // kernel rows as C(rho) = beta_s + sigma_s * rho on (R_{s-1}, R_s]
+            // slopes of the kernel rows on (R_{s-1}, R_s]
             if (tid < 2 * nr) {
                 const int d = tid / nr, q = tid - d * nr;
                 const float* row = d == 0 ? sF : sB;
-                const float prev = q == 0 ? 0.f : row[q - 1];
-                const float sg = (row[q] - prev) * sIW[q];
-                sSig[d][q] = (double)sg;
-                sBeta[d][q] = (double)prev - (double)sg * (q == 0 ? 0.0 : (double)sR[q - 1]);
+                sSig[d][q] = (double)((row[q] - (q == 0 ? 0.f : row[q - 1])) * sIW[q]);
             }
             const float2* sv = s_line + vlo;
             // radiological centres (FP64 scan) and the two FP64 prefix sums, one chunk per thread
@@ -678,8 +707,7 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
             __syncthreads();
             {
                 for (int j = tid; j < n; j += NT) {
-                    const double v = ramp_back(L, j, sSig[0], sBeta[0], sR, nr, iters) +
-                                     ramp_fwd(L, j, sSig[1], sBeta[1], sR, nr, iters);
+                    const double v = ramp_walk<true, true>(L, j, sSig[0], sSig[1], sR, nr, iters);
                     out[vlo + j] = (float)v / nphi_f;
                 }
             }

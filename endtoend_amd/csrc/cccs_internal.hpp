@@ -157,9 +157,11 @@ CCCS_HD float2 tex3_pair(const float2* __restrict__ v, int nx, int ny, int nz, f
     if (i >= 0 && j >= 0 && k >= 0 && i + 1 < nx && j + 1 < ny && k + 1 < nz) {
         // volumes below 2^31 voxels (checked by the caller): 32-bit tap offsets
         const uint32_t sy = (uint32_t)nx, sz = (uint32_t)nx * (uint32_t)ny;
+        // (each x pair is one 16-byte load: its second address is formed from the first)
         const float2* p = v + ((uint32_t)i + sy * (uint32_t)j + sz * (uint32_t)k);
-        c00 = p[0]; c10 = p[1]; c01 = p[sy]; c11 = p[sy + 1];
-        d00 = p[sz]; d10 = p[sz + 1]; d01 = p[sz + sy]; d11 = p[sz + sy + 1];
+        const float2 *py = p + sy, *pz = p + sz, *pyz = pz + sy;
+        c00 = p[0]; c10 = p[1]; c01 = py[0]; c11 = py[1];
+        d00 = pz[0]; d10 = pz[1]; d01 = pyz[0]; d11 = pyz[1];
     } else {
         c00 = fetch2_or0(v, nx, ny, nz, i, j, k); c10 = fetch2_or0(v, nx, ny, nz, i + 1, j, k);
         c01 = fetch2_or0(v, nx, ny, nz, i, j + 1, k); c11 = fetch2_or0(v, nx, ny, nz, i + 1, j + 1, k);
