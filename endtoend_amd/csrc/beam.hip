@@ -237,17 +237,31 @@ __global__ void __launch_bounds__(256) crop_final_kernel(const float* __restrict
     if (t < 7) out[t] = s[t][0];
 }
 
-// A class-list entry: the line, its cone and its record, so that a workgroup starts from one
-// 16-byte load instead of a list load, a record load and a search over the cones.
+// A class-list entry: all that a workgroup needs of its line, as one scalar load.  Samples
+// [ja, jb] of the stored interval lie inside the crop box, the calc_bbox and the interpolation range
+// by a margin that covers FP32 rounding; the others are tested one by one.
 struct ConeLine {
-    uint32_t line;
+    uint32_t line;     // global line index (profiling counters)
+    uint32_t off;      // first stored sample in the REV store
+    int16_t i0, len;   // stored interval
+    int16_t ja, jb;    // interior samples, relative to i0 (ja > jb: none)
+    uint16_t ty, tz;   // line of the cone's grid
     uint32_t cone;
-    LineMeta meta;
 };
+static_assert(sizeof(ConeLine) == 24, "six dwords");
+
+// Read-only data at wave-uniform addresses, loaded through the scalar unit.
+template <class T>
+using uniform_ptr = const __attribute__((address_space(4))) T*;
+template <class T>
+__device__ __forceinline__ uniform_ptr<T> as_uniform(const T* p) {
+    return (uniform_ptr<T>)p;
+}
 
 struct ConeArgs {
     const float2* dt;         // {density, TERMA (0 outside the calc_bbox)} over the CT grid
     const float* tables;      // kernel | radii | inverse widths
+    const RampStep* steps;    // [ntheta/2][nradii]
     const ConeDev* cones;
     LineMeta* lines;          // one entry per REV line of every cone
     float* rev;               // compact REV dose store
@@ -255,17 +269,15 @@ struct ConeArgs {
     int ncones;
     int ntheta, nradii, nphi;
     float delr;
-    uint32_t* counts;         // per-workgroup walk iteration counts (profiling) or nullptr
+    uint32_t* counts;         // per-workgroup walk step counts (profiling) or nullptr
     int ramp_min;             // valid segments at least this long use the segment-sum walk
     int maxn;                 // longest stored line of this launch (LDS sizing)
-    int len_lo, len_hi;       // this launch takes the lines whose stored length is in [len_lo, len_hi]
-    const ConeLine* list;     // the lines of this launch (one workgroup each), or nullptr: every line
+    const ConeLine* list;     // the lines of this launch, one workgroup each
     VolDesc vd;
     m33 binv;                 // PVCS <- BEV rotation (index units)
     v3 off;                   // (bevStart - start) / voxel
     v3 bev_size;              // crop-box size (index units)
     v3 bb0, bb1;              // calc_bbox bounds (PVCS index)
-    int bbx, bby, bbz;        // calc_bbox size
 };
 
 __device__ __forceinline__ int cone_of_line(const ConeDev* __restrict__ cones, int ncones, uint64_t line) {
@@ -325,8 +337,8 @@ __device__ __forceinline__ void line_interval(const ConeArgs& a, const ConeDev& 
 // starts from; a line that fits into the radii has no such end.  Same result as the sequential walk
 // up to FP32 rounding of the accumulated distance.  The cone kernel issues VALU instructions in 92-98 %
 // of its cycles, so a walk is as fast as its instructions are few: interval sums with a search loop per
-// interval (about 55 per radius and direction) took 11.8 ms of a 256x256x180 request, this form (28)
-// 8.9 ms.
+// interval (about 55 per radius and direction) took 11.8 ms of a 256x256x180 request, this form with
+// 28 8.9 ms, with 21 (no masks, no copies between the radii) 7.4 ms.
 struct RampLine {
     const float* c;       // centres, radiological cm from the segment start; c[n..n+3] = +inf
     const double* E;      // E[k]  = sum_{m<k} (T_m - T_{m-1}) c_m   (T_{-1} = 0), k in [0, n]
@@ -337,129 +349,171 @@ struct RampLine {
     float c0, cn, invD;
 };
 
-// The search for the first k with c_k >= y (y <= c_{n-1}): a table lookup and two probes (one LDS
-// load), no branch.  A cell holds at most one centre where the density is at least half the line's
-// mean; `more` says that both probed centres lie below y, so that ramp_more has to go on from k.
+// The search for the first k with c_k >= y (kUpper: c_k > y), c_0 <= y <= c_{n-1}: a table lookup and
+// two probes (one LDS load), no branch.  A cell holds at most one centre where the density is at
+// least half the line's mean; `more` says that both probed centres lie below y, so that ramp_more has
+// to go on from k.
+CCCS_HD double max_f64(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;  // (one instruction: the library form also quiets its operands)
+    __asm__("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return a > b ? a : b;
+#endif
+}
 struct RampPos {
     int u, k;
     bool more;
 };
+template <bool kUpper>
+CCCS_HD bool ramp_below(float c, float y) { return kUpper ? c <= y : c < y; }
+template <bool kUpper>
 CCCS_HD RampPos ramp_probe(const RampLine& L, float y) {
     RampPos p;
-    // biased by 1% of a cell so that the cell's threshold never exceeds y after rounding
-    p.u = min(max((int)((y - L.c0) * L.invD - 0.01f), 0), L.U - 1);
+    // biased by 2% of a cell so that the cell's threshold never exceeds y after rounding
+    p.u = (int)fmaf(y, L.invD, -0.02f - L.c0 * L.invD);
     const int k = L.lb[p.u];
     const float ca = L.c[k], cb = L.c[k + 1];
-    p.more = cb < y;
-    p.k = k + (ca < y ? 1 : 0) + (p.more ? 1 : 0);
+    p.more = ramp_below<kUpper>(cb, y);
+    p.k = k + (ramp_below<kUpper>(ca, y) ? 1 : 0) + (p.more ? 1 : 0);
     return p;
 }
+template <bool kUpper>
 CCCS_HD int ramp_more(const RampLine& L, float y, const RampPos& p) {
-    int k = p.k;
+    int k = min(p.k, L.n);
     if (L.lb[p.u + 1] - k > 8) {  // a crowded cell (low density): bisect up to the next cell's end
         int hi = L.lb[p.u + 2];
         while (k < hi) {
             const int mid = (k + hi) >> 1;
-            if (L.c[mid] < y) k = mid + 1; else hi = mid;
+            if (ramp_below<kUpper>(L.c[mid], y)) k = mid + 1; else hi = mid;
         }
     }
-    while (L.c[k] < y) k++;
+    while (k < L.n && ramp_below<kUpper>(L.c[k], y)) k++;  // (bounded: y is infinite with an infinite density)
     return k;
 }
-CCCS_HD int ramp_lb(const RampLine& L, float y) {
-    const RampPos p = ramp_probe(L, y);
-    return p.more ? ramp_more(L, y, p) : p.k;
+template <bool kUpper>
+CCCS_HD int ramp_find(const RampLine& L, float y) {
+    if (y < L.c0) return 0;
+    const RampPos p = ramp_probe<kUpper>(L, y);
+    return p.more ? ramp_more<kUpper>(L, y, p) : p.k;
 }
+// Lines whose cells are too fine for FP32 lookups (the first half step dwarfs the rest of the line:
+// cells of less than 1/20 of the samples' mean share of c_{n-1}) keep one cell and search in it.
+CCCS_HD float ramp_cells(float c0, float cn, int U) { return cn - c0 > 0.05f * cn ? (float)U / (cn - c0) : 0.f; }
 
-// first k with c_k > y, for y < c_{n-1}
-CCCS_HD int ramp_ub(const RampLine& L, float y) {
-    int k = y < L.c0 ? 0 : ramp_lb(L, y);
-    while (L.c[k] <= y) k++;
-    return k;
-}
+// Lanes of a wave leave the walk together, so that its body runs without masks.
+struct RampWave {
+    static __device__ __forceinline__ bool any(bool x) { return __any(x); }
+};
+struct RampAlone {
+    static CCCS_HD bool any(bool x) { return x; }
+};
 
-// The backward (toward lower indices) and / or forward walk of destination j, the kernel rows given
-// by their slopes.  Both directions step through the radii together, so that their lookups (two
-// dependent LDS trips each) overlap.
-template <bool kBack, bool kFwd>
-CCCS_HD double ramp_walk(const RampLine& L, int j, const double* __restrict__ sigb, const double* __restrict__ sigf,
-                         const float* __restrict__ R, int nr, uint32_t& iters) {
-    // F starts at the boundary of the destination and ends, at Fa / Eb, at the centre ya / yb of the
-    // last sample that the walk reaches; a walk without samples ends at once.  (Forward, F is taken
-    // without its constant: E2[q] + T_q y.)
-    double Pb = 0.0, Pf = 0.0, Fb = 0.0, Ff = 0.0, Fa = 0.0, Eb = 0.0;
-    float ya = INFINITY, yb = -INFINITY;
-    const bool exits = L.cn - L.c0 > R[nr - 2];
+// The backward (toward lower indices) and / or forward walk of destination j.  Both directions step
+// through the radii together, so that their lookups (two dependent LDS trips each) overlap.  F starts
+// at the boundary of the destination and ends, at Fa / Eb, at the centre ya / yb of the last sample
+// that the walk reaches: there y is clamped (backward) or F taken as Eb (forward: the last cell may be
+// crowded, so the lookup goes to the first), and F's differences are zero.  (Forward, F is taken
+// without its constant: E2[q] + T_q y.)
+template <bool kBack, bool kFwd, class Lanes>
+CCCS_HD double ramp_walk(const RampLine& L, int j, const RampStep* steps, int nr, uint32_t& iters) {
+    double Pb = L.c0, Pf = L.cn, Fb = 0.0, Ff = 0.0, Fa = 0.0, Eb = 0.0, ya = L.c0, yb = L.cn;
+    const double rlast = steps[nr - 1].r, rprev = steps[nr - 2].r;
+    const bool exits = (double)L.cn - (double)L.c0 > rprev;
+    bool back = false, fwd = false;
     if (kBack && j > 0) {
         const float2 e = L.s[j - 1];
         Pb = (double)L.c[j - 1] + (double)e.x;
-        int a = 0;
-        if (exits) {
-            const float yl = (float)(Pb - (double)R[nr - 1]), yp = (float)(Pb - (double)R[nr - 2]);
-            a = max(yl > L.c0 ? ramp_lb(L, yl) : 0, (yp > L.c0 ? ramp_lb(L, yp) : 0) - 1);
-        }
-        if (a < j) {
-            ya = L.c[a];
-            if (a > 0) Fa = fma((double)L.s[a - 1].y, (double)ya, -L.E[a]);
+        const int a = exits ? max(ramp_find<false>(L, (float)(Pb - rlast)), ramp_find<false>(L, (float)(Pb - rprev)) - 1) : 0;
+        back = a < j;
+        if (back) {
+            ya = (double)L.c[a];
+            if (a > 0) Fa = fma((double)L.s[a - 1].y, ya, -L.E[a]);
             Fb = fma((double)e.y, Pb, -L.E[j]);
+            // F rises where there is TERMA: a difference of rounding size means none in the walk's reach
+            back = !exits || fabs(Fb - Fa) > 1e-14 * fabs(Fa);
         }
+        if (!back) Pb = ya;
     }
     if (kFwd && j < L.n - 1) {
         const float2 e = L.s[j + 1];
         Pf = (double)L.c[j + 1] - (double)e.x;
         int b = L.n - 1;
         if (exits) {
-            const float yl = (float)(Pf + (double)R[nr - 1]), yp = (float)(Pf + (double)R[nr - 2]);
-            const int ml = yl < L.cn ? ramp_ub(L, yl) - 1 : b, mp = yp < L.cn ? ramp_ub(L, yp) - 1 : b;
+            const float yl = (float)(Pf + rlast), yp = (float)(Pf + rprev);
+            const int ml = yl < L.cn ? ramp_find<true>(L, yl) - 1 : b, mp = yp < L.cn ? ramp_find<true>(L, yp) - 1 : b;
             b = min(ml, mp + 1);
         }
-        if (b > j) {
-            yb = L.c[b];
+        fwd = b > j;
+        if (fwd) {
+            yb = (double)L.c[b];
             Eb = L.E2[b + 1];
-            if (b < L.n - 1) Eb = fma((double)L.s[b + 1].y, (double)yb, Eb);
+            if (b < L.n - 1) Eb = fma((double)L.s[b + 1].y, yb, Eb);
             Ff = fma((double)e.y, Pf, L.E2[j + 1]);
+            fwd = !exits || fabs(Eb - Ff) > 1e-14 * fabs(Eb);
         }
+        if (!fwd) Pf = yb;
     }
-    double sum = 0.0;
-    for (int s = 0; s < nr; s++) {
-        const double r = (double)R[s];
-        const double y0 = Pb - r, y1 = Pf + r;
-        const bool in0 = kBack && (float)y0 > ya, in1 = kFwd && (float)y1 < yb;
-        const float z0 = in0 ? (float)y0 : L.c0, z1 = in1 ? (float)y1 : L.c0;
-        RampPos p0{0, 0, false}, p1{0, 0, false};
-        if (kBack) p0 = ramp_probe(L, z0);
-        if (kFwd) p1 = ramp_probe(L, z1);
+    const double span = fmax(Pb - ya, yb - Pf);
+    double sb = 0.0, sf = 0.0;
+    // one radius: F at distance r from the destination, gb and gf the slopes of the interval it ends
+    auto step = [&](const RampStep& st, double Fb0, double Ff0, double& Fb1, double& Ff1) {
+        const double y0 = max_f64(Pb - st.r, ya), y1 = Pf + st.r;
+        const bool in1 = y1 < yb;
+        const float z0 = (float)y0, z1 = in1 ? (float)y1 : L.c0;
+        RampPos p0{0, 1, false}, p1{0, 0, false};
+        if (kBack) p0 = ramp_probe<true>(L, z0);
+        if (kFwd) p1 = ramp_probe<false>(L, z1);
         if (p0.more || p1.more) {
-            if (p0.more) p0.k = ramp_more(L, z0, p0);
-            if (p1.more) p1.k = ramp_more(L, z1, p1);
+            if (p0.more) p0.k = ramp_more<true>(L, z0, p0);
+            if (p1.more) p1.k = ramp_more<false>(L, z1, p1);
         }
         if (kBack) {
-            const int q = max(p0.k, 1);
-            const double Fs = fma((double)L.s[q - 1].y, y0, -L.E[q]);
-            const double d = in0 ? Fs : Fa;
-            sum = fma(sigb[s], Fb - d, sum);
-            Fb = d;
+            Fb1 = fma((double)L.s[p0.k - 1].y, y0, -L.E[p0.k]);
+            sb = fma(st.sigb, Fb0 - Fb1, sb);
         }
         if (kFwd) {
             const double Fs = fma((double)L.s[p1.k].y, y1, L.E2[p1.k]);
-            const double d = in1 ? Fs : Eb;
-            sum = fma(sigf[s], d - Ff, sum);
-            Ff = d;
+            Ff1 = in1 ? Fs : Eb;
+            sf = fma(st.sigf, Ff1 - Ff0, sf);
         }
-        iters++;
-        if (!in0 && !in1) break;
+    };
+    int s = 0;
+    while (s < nr && Lanes::any(steps[s].r < span)) {  // two radii a round: no copies between them
+        double Fb1 = 0.0, Ff1 = 0.0;
+        step(steps[s], Fb, Ff, Fb1, Ff1);
+        if (++s < nr && Lanes::any(steps[s].r < span)) {
+            step(steps[s], Fb1, Ff1, Fb, Ff);
+            s++;
+        } else {
+            Fb = Fb1;
+            Ff = Ff1;
+            break;
+        }
     }
-    return sum;
+    if (s < nr) {  // the interval in which the last of the lanes ends
+        if (kBack) sb = fma(steps[s].sigb, Fb - Fa, sb);
+        if (kFwd) sf = fma(steps[s].sigf, Eb - Ff, sf);
+    }
+    iters += (uint32_t)s;
+    return (back ? sb : 0.0) + (fwd ? sf : 0.0);
 }
 
-// One direction alone, for a caller that also holds the rows' intercepts (the line checks).
+// One direction alone with a row's slopes in an array (the line checks).
+template <bool kBack>
+CCCS_HD double ramp_one(const RampLine& L, int j, const double* sig, const float* R, int nr, uint32_t& iters) {
+    RampStep st[kMaxRadii];
+    for (int q = 0; q < nr; q++) st[q] = RampStep{(double)R[q], sig[q], sig[q], 0.0};
+    return ramp_walk<kBack, !kBack, RampAlone>(L, j, st, nr, iters);
+}
 CCCS_HD double ramp_back(const RampLine& L, int j, const double* sig, const double*, const float* R, int nr,
                          uint32_t& iters) {
-    return ramp_walk<true, false>(L, j, sig, nullptr, R, nr, iters);
+    return ramp_one<true>(L, j, sig, R, nr, iters);
 }
 CCCS_HD double ramp_fwd(const RampLine& L, int j, const double* sig, const double*, const float* R, int nr,
                         uint32_t& iters) {
-    return ramp_walk<false, true>(L, j, nullptr, sig, R, nr, iters);
+    return ramp_one<false>(L, j, sig, R, nr, iters);
 }
 
 // First cell u in [0, nu] whose threshold c0 + u * D exceeds v (nu when none does): an estimate
@@ -473,23 +527,13 @@ CCCS_HD int ramp_cell_after(float c0, float D, float invD, int nu, float v) {
     return u;
 }
 
-// Exclusive prefix sum over the 64 lanes of a wave.
-__device__ __forceinline__ double wave_excl_sum(double v) {
-    const int lane = threadIdx.x & 63;
-    double x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const double u = __shfl_up(x, o, 64);
-        if (lane >= o) x += u;
-    }
-    const double e = __shfl_up(x, 1, 64);
-    return lane == 0 ? 0.0 : e;
-}
-
 // LDS bytes of the cone kernel for lines of up to maxn samples (with the segment-sum arrays).
 inline size_t cone_lds_bytes(uint32_t maxn, bool ramp) {
-    if (!ramp) return sizeof(float2) * maxn;
+    // (the sequential walk's rows take the place of the lookup table)
+    const size_t rows = sizeof(float) * 4 * kMaxRadii;
+    if (!ramp) return sizeof(float2) * maxn + rows;
     const size_t n1 = (size_t)maxn + 1, nc = ((size_t)maxn + 4 + 1) & ~(size_t)1;
-    return 2 * sizeof(double) * n1 + sizeof(float) * nc + sizeof(float2) * maxn + sizeof(uint16_t) * (2 * maxn + 2);
+    return 2 * sizeof(double) * n1 + sizeof(float) * nc + sizeof(float2) * maxn + std::max(sizeof(uint16_t) * (2 * (size_t)maxn + 4), rows);
 }
 
 // Pass 1 of the cone pipeline: the stored interval of every REV line (offsets come from a scan).
@@ -508,61 +552,133 @@ __global__ void __launch_bounds__(256) line_interval_kernel(ConeArgs a) {
     a.lines[line] = m;
 }
 
-// Pass 2: one wave per REV line of any cone (XCD-aware order).  The stored interval of the line is
-// resampled (density and TERMA, trilinear) into LDS with the exact per-sample test of
-// cudaRaytrace; then every valid sample runs both collapsed-cone walks from LDS and the interval's
-// cone dose is written to the compact REV store.
-// Workgroup-wide exclusive prefix sum of one double per thread (NT/64 waves; s_tot holds NT/64
-// doubles).  Contains barriers: every thread of the workgroup must call it.
+// v moved across lanes by a DPP control; lanes outside the rows of the mask or without a source get 0.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kCtrl, kRows, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kCtrl, kRows, 0xf, false);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// Inclusive prefix sum over the 64 lanes of a wave: three instructions a step and no LDS trip.
+__device__ __forceinline__ double wave_incl_sum(double x) {
+    x += dpp_f64<0x111, 0xf>(x);  // row_shr 1, 2, 4, 8 (rows of 16 lanes)
+    x += dpp_f64<0x112, 0xf>(x);
+    x += dpp_f64<0x114, 0xf>(x);
+    x += dpp_f64<0x118, 0xf>(x);
+    x += dpp_f64<0x142, 0xa>(x);  // row_bcast 15 into rows 1 and 3
+    x += dpp_f64<0x143, 0xc>(x);  // row_bcast 31 into rows 2 and 3
+    return x;
+}
+// Workgroup-wide exclusive prefix sums of one or two doubles per thread (NT/64 waves; s_tot holds
+// 2 * NT/64 doubles).  Contains barriers: every thread of the workgroup must call it.
 template <int NT>
-__device__ __forceinline__ double block_excl_sum(double v, double* s_tot) {
+__device__ __forceinline__ void block_excl_sum2(double& v, double& w, double* s_tot) {
+    const double x = wave_incl_sum(v), y = wave_incl_sum(w);
+    v = dpp_f64<0x138, 0xf>(x);  // wave_shr 1
+    w = dpp_f64<0x138, 0xf>(y);
+    if (NT == 64) return;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    double x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const double u = __shfl_up(x, o, 64);
-        if (lane >= o) x += u;
+    if (lane == 63) {
+        s_tot[2 * wid] = x;
+        s_tot[2 * wid + 1] = y;
     }
-    double e = __shfl_up(x, 1, 64);
-    e = lane == 0 ? 0.0 : e;
-    if (NT == 64) return e;
-    if (lane == 63) s_tot[wid] = x;
     __syncthreads();
-    double base = 0.0;
-    for (int w = 0; w < wid; w++) base += s_tot[w];
+    for (int q = 0; q < wid; q++) {
+        v += s_tot[2 * q];
+        w += s_tot[2 * q + 1];
+    }
     __syncthreads();
-    return base + e;
 }
 
+// Narrows [t0, t1] to the parameters where o + t*d lies in [lo, hi], for |t| <= 1024 (approximate
+// reciprocal: the caller's bounds carry a margin).
+__device__ __forceinline__ void keep_slab(float o, float d, float lo, float hi, float& t0, float& t1) {
+    if (fabsf(d) < 1e-6f) {
+        if (!(o >= lo && o <= hi)) { t0 = 1.f; t1 = 0.f; }
+        return;
+    }
+    const float id = __builtin_amdgcn_rcpf(d), ta = (lo - o) * id, tb = (hi - o) * id;
+    t0 = fmaxf(t0, fminf(ta, tb));
+    t1 = fminf(t1, fmaxf(ta, tb));
+}
+
+// Interior samples [ja, jb] of a stored line (ConeLine).  The margin is far above the rounding of
+// the exact per-sample chain and of the affine form (both a few 1e-4 index units at most), so inside it
+// the exact test cannot fail and all eight taps exist.
+__device__ __forceinline__ void line_interior(const ConeArgs& a, const ConeDev& c, int tY, int tZ, int i0, int len,
+                                              int& ja, int& jb) {
+    constexpr float m = 0.01f;
+    const v3 b0 = c.kinv(mk3(c.rs.x + (float)tZ, c.rs.y, c.rs.z + (float)tY));
+    const v3 kd = mk3(c.kinv.m[1], c.kinv.m[4], c.kinv.m[7]);
+    const v3 g0 = c.g0 + (float)tY * c.gy + (float)tZ * c.gz;
+    float t0 = (float)i0, t1 = (float)(i0 + len - 1);
+    keep_slab(b0.x, kd.x, m, a.bev_size.x - m, t0, t1);
+    keep_slab(b0.y, kd.y, m, a.bev_size.y - m, t0, t1);
+    keep_slab(b0.z, kd.z, m, a.bev_size.z - m, t0, t1);
+    keep_slab(g0.x, c.gx.x, a.bb0.x + m, fminf(a.bb1.x, (float)(a.vd.nx - 1)) - m, t0, t1);
+    keep_slab(g0.y, c.gx.y, a.bb0.y + m, fminf(a.bb1.y, (float)(a.vd.ny - 1)) - m, t0, t1);
+    keep_slab(g0.z, c.gx.z, a.bb0.z + m, fminf(a.bb1.z, (float)(a.vd.nz - 1)) - m, t0, t1);
+    ja = len;
+    jb = -1;
+    // the interior's tap index is formed with 24-bit products: rows below 2^24
+    if (!(t0 <= t1) || (int64_t)a.vd.ny * a.vd.nz >= (1 << 24) || a.vd.nx >= (1 << 24)) return;
+    ja = (int)ceilf(t0) - i0;
+    jb = (int)floorf(t1) - i0;
+    if (ja > jb) {
+        ja = len;
+        jb = -1;
+    }
+}
+
+__device__ __forceinline__ float lerp1(float a, float b, float t) { return fmaf(t, b - a, a); }
+
+// {density, TERMA} at an interior point (all eight taps inside): four 16-byte loads.
+__device__ __forceinline__ float2 interior_pair(const float2* __restrict__ dt, uint32_t nx, uint32_t ny, v3 g) {
+    typedef float quad __attribute__((ext_vector_type(4), aligned(8)));
+    const float fx = floorf(g.x), fy = floorf(g.y), fz = floorf(g.z);
+    const float ax = g.x - fx, ay = g.y - fy, az = g.z - fz;
+    const uint32_t row = __umul24((uint32_t)(int)fz, ny) + (uint32_t)(int)fy;
+    const float2* p = dt + (__umul24(row, nx) + (uint32_t)(int)fx);
+    const size_t sz = (size_t)nx * ny;
+    const quad q0 = *reinterpret_cast<const quad*>(p), q1 = *reinterpret_cast<const quad*>(p + nx);
+    const quad q2 = *reinterpret_cast<const quad*>(p + sz), q3 = *reinterpret_cast<const quad*>(p + sz + nx);
+    float2 r;
+    r.x = lerp1(lerp1(lerp1(q0.x, q0.z, ax), lerp1(q1.x, q1.z, ax), ay),
+                lerp1(lerp1(q2.x, q2.z, ax), lerp1(q3.x, q3.z, ax), ay), az);
+    r.y = lerp1(lerp1(lerp1(q0.y, q0.w, ax), lerp1(q1.y, q1.w, ax), ay),
+                lerp1(lerp1(q2.y, q2.w, ax), lerp1(q3.y, q3.w, ax), ay), az);
+    return r;
+}
+
+// Pass 2: one workgroup (one or more waves) per listed REV line of any cone, in XCD-aware order.  The
+// stored interval of the line is resampled (density and TERMA, trilinear) into LDS; then every valid
+// sample runs both collapsed-cone walks from LDS and the interval's cone dose is written to the
+// compact REV store.  Interior samples take their position as one multiply-add per axis along the
+// line and interpolate without tests; the few samples near a face of the crop box or the grid run
+// the exact test of cudaRaytrace.  The line's entry, the cone's constants and the radial steps are
+// scalar loads.
 template <int NT>
 __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     constexpr int NW = NT / 64;
     extern __shared__ double s_dyn[];
-    __shared__ float sR[kMaxRadii], sIW[kMaxRadii], sF[kMaxRadii], sB[kMaxRadii];
-    __shared__ double sSig[2][kMaxRadii];
-    __shared__ double s_tot[NW];
+    __shared__ RampStep s_steps[kMaxRadii];
+    __shared__ double s_tot[2 * NW];
     __shared__ int s_red[NW][3];
     __shared__ uint32_t s_cnt[NW];
-    const uint64_t slot = xcd_remap(blockIdx.x, gridDim.x);
-    uint64_t line;
-    uint32_t cone;
-    LineMeta meta;
-    if (a.list) {
-        const ConeLine e = a.list[slot];
-        line = e.line;
-        cone = e.cone;
-        meta = e.meta;
-    } else {
-        line = slot;
-        meta = a.lines[line];
-        cone = (uint32_t)cone_of_line(a.cones, a.ncones, line);
-    }
+    const uint32_t slot = xcd_remap(blockIdx.x, gridDim.x);
+    const uniform_ptr<ConeLine> en = as_uniform(a.list) + slot;
+    const uint32_t line = en->line, off = en->off;
+    const int i0 = en->i0, m = en->len, ja = en->ja, jb = en->jb, tY = en->ty, tZ = en->tz;
+    const uniform_ptr<ConeDev> c = as_uniform(a.cones) + en->cone;
+    const int rowf = c->rowf;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const bool mine = meta.len >= a.len_lo && meta.len <= a.len_hi;
+    const int nr = a.nradii;
     uint32_t iters = 0;
-    if (mine) {
-        const ConeDev& c = a.cones[cone];
-        const int nr = a.nradii;
-        const int m = meta.len;
+    // the radial steps go to LDS past the resample, so their latency overlaps the gathers
+    RampStep step{};
+    if (tid < nr) step = a.steps[(size_t)rowf * nr + tid];
+    {
         const bool ramp_lds = a.ramp_min <= a.maxn;
         // LDS: [E | E2 | c | line | lb] with the segment-sum arrays, else [line]
         const int n1 = a.maxn + 1, nc = (a.maxn + 5) & ~1;
@@ -571,65 +687,69 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
         float* rc = reinterpret_cast<float*>(rE2 + n1);
         float2* s_line = ramp_lds ? reinterpret_cast<float2*>(rc + nc) : reinterpret_cast<float2*>(s_dyn);
         uint16_t* rlb = reinterpret_cast<uint16_t*>(s_line + a.maxn);
-        // the kernel rows' loads are issued before the resample's and land in LDS after it, so
-        // their latency overlaps the density / TERMA fetches
-        float tR = 0.f, tIW = 0.f, tF = 0.f, tB = 0.f;
-        if (tid < nr) {
-            const float* K = a.tables;
-            const float* R = a.tables + (size_t)a.ntheta * nr;
-            tR = R[tid];
-            tIW = R[nr + tid];
-            tF = K[(size_t)c.rowf * nr + tid];
-            tB = K[(size_t)c.rowb * nr + tid];
+        float* out = a.rev + off;
+        // interior (a negative or undefined density makes a sample invalid, as outside)
+        bool bad = false;
+        if (ja <= jb) {
+            const float fY = (float)tY, fZ = (float)tZ;
+            const v3 gx = mk3(c->gx.x, c->gx.y, c->gx.z);
+            const v3 g0 = mk3(fmaf(fZ, c->gz.x, fmaf(fY, c->gy.x, c->g0.x)), fmaf(fZ, c->gz.y, fmaf(fY, c->gy.y, c->g0.y)),
+                              fmaf(fZ, c->gz.z, fmaf(fY, c->gy.z, c->g0.z)));
+            for (int j = ja + tid; j <= jb; j += NT) {
+                const float t = (float)(i0 + j);
+                const float2 dt = interior_pair(a.dt, (uint32_t)a.vd.nx, (uint32_t)a.vd.ny,
+                                                mk3(fmaf(t, gx.x, g0.x), fmaf(t, gx.y, g0.y), fmaf(t, gx.z, g0.z)));
+                const float h = 0.5f * (a.delr * dt.x);
+                bad = bad || !(h >= 0.f);
+                s_line[j] = make_float2(h, dt.y);
+            }
         }
-        const uint64_t l = line - c.line0;
-        const int tY = (int)(l % (uint64_t)c.ny);
-        const int tZ = (int)(l / (uint64_t)c.ny);
-        const int i0 = meta.i0;
-        float* out = a.rev + meta.off;
-        for (int j = tid; j < m; j += NT) {
-            const int i = i0 + j;
-            float2 e = make_float2(-1.f, 0.f);
-            v3 bev = c.kinv(mk3(c.rs.x + (float)tZ, c.rs.y + (float)i, c.rs.z + (float)tY));
-            if (bev.x >= 0.f && bev.y >= 0.f && bev.z >= 0.f && bev.x < a.bev_size.x && bev.y < a.bev_size.y &&
-                bev.z < a.bev_size.z) {
-                v3 g = a.binv(bev) + a.off;
-                if (g.x >= a.bb0.x && g.x < a.bb1.x && g.y >= a.bb0.y && g.y < a.bb1.y && g.z >= a.bb0.z &&
-                    g.z < a.bb1.z) {
-                    const float2 dt = tex3_pair(a.dt, a.vd.nx, a.vd.ny, a.vd.nz, g.x + 0.5f, g.y + 0.5f, g.z + 0.5f);
-                    e.x = 0.5f * (a.delr * dt.x);
-                    e.y = dt.y;
+        const int nbad = __any(bad) ? 1 : 0;  // (per wave)
+        // the other samples, exactly; the valid segment is the interior and the valid ones among these
+        // (contiguous: the crop box and the calc_bbox are convex)
+        int vlo = ja <= jb ? ja : m, vhi = jb, nvalid = 0;
+        const int nhead = min(ja, m), nedge = m - (ja <= jb ? jb - ja + 1 : 0);
+        if (nedge > 0) {
+            m33 kinv;
+            for (int q = 0; q < 9; q++) kinv.m[q] = c->kinv.m[q];
+            const v3 rs = mk3(c->rs.x, c->rs.y, c->rs.z);
+            for (int e0 = 64 * wid; e0 < nedge; e0 += NT) {
+                const int e = e0 + lane;
+                float2 v = make_float2(-1.f, 0.f);
+                if (e < nedge) {
+                    const int j = e < nhead ? e : jb + 1 + (e - nhead);
+                    const v3 bev = kinv(mk3(rs.x + (float)tZ, rs.y + (float)(i0 + j), rs.z + (float)tY));
+                    if (bev.x >= 0.f && bev.y >= 0.f && bev.z >= 0.f && bev.x < a.bev_size.x && bev.y < a.bev_size.y &&
+                        bev.z < a.bev_size.z) {
+                        const v3 g = a.binv(bev) + a.off;
+                        if (g.x >= a.bb0.x && g.x < a.bb1.x && g.y >= a.bb0.y && g.y < a.bb1.y && g.z >= a.bb0.z &&
+                            g.z < a.bb1.z) {
+                            const float2 dt = tex3_pair(a.dt, a.vd.nx, a.vd.ny, a.vd.nz, g.x + 0.5f, g.y + 0.5f, g.z + 0.5f);
+                            v.x = 0.5f * (a.delr * dt.x);
+                            v.y = dt.y;
+                        }
+                    }
+                    s_line[j] = v;
+                }
+                // (j rises with e, so the first and the last valid lane give the extremes)
+                const uint64_t ok = __ballot(v.x >= 0.f);
+                if (ok) {
+                    const int ef = e0 + __builtin_ctzll(ok), el = e0 + 63 - __builtin_clzll(ok);
+                    vlo = min(vlo, ef < nhead ? ef : jb + 1 + (ef - nhead));
+                    vhi = max(vhi, el < nhead ? el : jb + 1 + (el - nhead));
+                    nvalid += __popcll(ok);
                 }
             }
-            s_line[j] = e;
         }
-        if (tid < nr) {
-            sR[tid] = tR;
-            sIW[tid] = tIW;
-            sF[tid] = tF;
-            sB[tid] = tB;
+        nvalid -= nbad;
+        if (tid < nr) s_steps[tid] = step;
+        if (NW > 1 && lane == 0) {
+            s_red[wid][0] = vlo;
+            s_red[wid][1] = vhi;
+            s_red[wid][2] = nvalid;
         }
         __syncthreads();
-        // valid segment of the line (contiguous: the crop box and the calc_bbox are convex)
-        int vlo = m, vhi = -1, nvalid = 0;
-        for (int j = tid; j < m; j += NT)
-            if (s_line[j].x >= 0.f) {
-                vlo = min(vlo, j);
-                vhi = max(vhi, j);
-                nvalid++;
-            }
-        for (int o = 32; o > 0; o >>= 1) {
-            vlo = min(vlo, __shfl_xor(vlo, o, 64));
-            vhi = max(vhi, __shfl_xor(vhi, o, 64));
-            nvalid += __shfl_xor(nvalid, o, 64);
-        }
         if (NW > 1) {
-            if (lane == 0) {
-                s_red[wid][0] = vlo;
-                s_red[wid][1] = vhi;
-                s_red[wid][2] = nvalid;
-            }
-            __syncthreads();
             vlo = s_red[0][0];
             vhi = s_red[0][1];
             nvalid = s_red[0][2];
@@ -639,49 +759,41 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
                 nvalid += s_red[w][2];
             }
         }
+        nvalid += m - nedge;  // (below the segment's length where the interior has an invalid sample)
+        vlo = __builtin_amdgcn_readfirstlane(vlo);
+        vhi = __builtin_amdgcn_readfirstlane(vhi);
+        nvalid = __builtin_amdgcn_readfirstlane(nvalid);
         const float nphi_f = (float)a.nphi;
         for (int j = tid; j < m; j += NT)
             if (j < vlo || j > vhi) out[j] = 0.f;
         const int n = vhi - vlo + 1;
         if (n >= a.ramp_min && nvalid == n) {
-            // slopes of the kernel rows on (R_{s-1}, R_s]
-            if (tid < 2 * nr) {
-                const int d = tid / nr, q = tid - d * nr;
-                const float* row = d == 0 ? sF : sB;
-                sSig[d][q] = (double)((row[q] - (q == 0 ? 0.f : row[q - 1])) * sIW[q]);
-            }
             const float2* sv = s_line + vlo;
-            // radiological centres (FP64 scan) and the two FP64 prefix sums, one chunk per thread
+            // radiological centres (FP64 scan), then the two FP64 prefix sums and the lookup table, one
+            // chunk of samples per thread; a sample's neighbours roll through registers
             const int per = (n + NT - 1) / NT;
             const int ca = min(n, tid * per), cb = min(n, ca + per);
-            double loc = 0.0;
-            for (int k = ca; k < cb; k++) loc += 2.0 * (double)sv[k].x;
-            double P = block_excl_sum<NT>(loc, s_tot);
-            double le = 0.0, le2 = 0.0;
-            for (int k = ca; k < cb; k++) {
-                const float2 e = sv[k];
-                const float ck = (float)(P + (double)e.x);
-                rc[k] = ck;
-                P += 2.0 * (double)e.x;
-                const double tp = k > 0 ? (double)sv[k - 1].y : 0.0, tn = k + 1 < n ? (double)sv[k + 1].y : 0.0;
-                le += ((double)e.y - tp) * (double)ck;
-                le2 += ((double)e.y - tn) * (double)ck;
+            double P = 0.0, unused = 0.0;
+            for (int k = ca; k < cb; k++) P += 2.0 * (double)sv[k].x;
+            block_excl_sum2<NT>(P, unused, s_tot);
+            double e1 = 0.0, e2 = 0.0;
+            const float tfirst = ca > 0 && ca < cb ? sv[ca - 1].y : 0.f;
+            {
+                float tp = tfirst;
+                float2 e = ca < cb ? sv[ca] : make_float2(0.f, 0.f);
+                for (int k = ca; k < cb; k++) {
+                    const float2 nx = k + 1 < n ? sv[k + 1] : make_float2(0.f, 0.f);
+                    const float ck = (float)(P + (double)e.x);
+                    rc[k] = ck;
+                    P += 2.0 * (double)e.x;
+                    e1 = fma((double)e.y - (double)tp, (double)ck, e1);
+                    e2 = fma((double)e.y - (double)nx.y, (double)ck, e2);
+                    tp = e.y;
+                    e = nx;
+                }
             }
-            double e1 = block_excl_sum<NT>(le, s_tot);
-            double e2 = block_excl_sum<NT>(le2, s_tot);
-            for (int k = ca; k < cb; k++) {
-                const double ck = (double)rc[k], t = (double)sv[k].y;
-                const double tp = k > 0 ? (double)sv[k - 1].y : 0.0, tn = k + 1 < n ? (double)sv[k + 1].y : 0.0;
-                rE[k] = e1;
-                rE2[k] = e2;
-                e1 += (t - tp) * ck;
-                e2 += (t - tn) * ck;
-            }
-            if (ca < cb && cb == n) {
-                rE[n] = e1;
-                rE2[n] = e2;
-                for (int q = 0; q < 4; q++) rc[n + q] = INFINITY;  // lookups probe up to 3 past n
-            }
+            if (tid < 4) rc[n + tid] = INFINITY;  // lookups probe past n
+            block_excl_sum2<NT>(e1, e2, s_tot);
             __syncthreads();
             // lookup table: lb[u] = first k with c_k >= c0 + u * D, U = 2n cells over [c0, c_{n-1}]
             RampLine L;
@@ -695,23 +807,49 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
             L.c0 = rc[0];
             L.cn = rc[n - 1];
             const float range = L.cn - L.c0;
-            const float D = range > 0.f ? range / (float)L.U : 0.f;
-            L.invD = range > 0.f ? (float)L.U / range : 0.f;
+            L.invD = ramp_cells(L.c0, L.cn, L.U);
+            const float D = L.invD > 0.f ? range / (float)L.U : 0.f;
             // sample k owns the cells whose threshold lies in (c_{k-1}, c_k] (c_{-1} = -inf, c_n =
-            // +inf): each of the U + 2 entries is written by exactly one sample
-            for (int k = tid; k <= n; k += NT) {
-                const int u0 = k == 0 ? 0 : ramp_cell_after(L.c0, D, L.invD, L.U + 2, rc[k - 1]);
-                const int u1 = k == n ? L.U + 2 : ramp_cell_after(L.c0, D, L.invD, L.U + 2, rc[k]);
-                for (int u = u0; u < u1; u++) rlb[u] = (uint16_t)k;
-            }
-            __syncthreads();
-            {
-                for (int j = tid; j < n; j += NT) {
-                    const double v = ramp_walk<true, true>(L, j, sSig[0], sSig[1], sR, nr, iters);
-                    out[vlo + j] = (float)v / nphi_f;
+            // +inf): each of the U + 2 entries is written by exactly one sample, the two past them by the
+            // last chunk (a lookup may round one cell up)
+            if (ca < cb) {
+                float tp = tfirst;
+                float2 e = sv[ca];
+                int u = ca == 0 ? 0 : ramp_cell_after(L.c0, D, L.invD, L.U + 2, rc[ca - 1]);
+                for (int k = ca; k < cb; k++) {
+                    const float2 nx = k + 1 < n ? sv[k + 1] : make_float2(0.f, 0.f);
+                    const float ck = rc[k];
+                    rE[k] = e1;
+                    rE2[k] = e2;
+                    e1 = fma((double)e.y - (double)tp, (double)ck, e1);
+                    e2 = fma((double)e.y - (double)nx.y, (double)ck, e2);
+                    const int u1 = ramp_cell_after(L.c0, D, L.invD, L.U + 2, ck);
+                    for (; u < u1; u++) rlb[u] = (uint16_t)k;
+                    tp = e.y;
+                    e = nx;
+                }
+                if (cb == n) {
+                    rE[n] = e1;
+                    rE2[n] = e2;
+                    for (; u < L.U + 4; u++) rlb[u] = (uint16_t)n;
                 }
             }
+            __syncthreads();
+            for (int j = tid; j < n; j += NT)
+                out[vlo + j] = (float)ramp_walk<true, true, RampWave>(L, j, s_steps, nr, iters) / nphi_f;
         } else {
+            // short segments: the sequential walk, its rows in LDS past the line
+            float* sR = reinterpret_cast<float*>(s_line + a.maxn);
+            float *sIW = sR + kMaxRadii, *sF = sIW + kMaxRadii, *sB = sF + kMaxRadii;
+            if (tid < nr) {
+                const float* K = a.tables;
+                const float* R = a.tables + (size_t)a.ntheta * nr;
+                sR[tid] = R[tid];
+                sIW[tid] = R[nr + tid];
+                sF[tid] = K[(size_t)rowf * nr + tid];
+                sB[tid] = K[(size_t)(a.ntheta - 1 - rowf) * nr + tid];
+            }
+            __syncthreads();
             for (int base = vlo; base <= vhi; base += NT) {
                 const int j = base + tid;
                 const bool act = j <= vhi && s_line[min(j, vhi)].x >= 0.f;
@@ -720,9 +858,8 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
             }
         }
     }
-    // every line's slot is written by exactly one of the length-class launches (empty lines' slots
-    // by the class-list pass when the launches take lists)
-    if (a.counts && (mine || (!a.list && meta.len == 0 && a.len_lo == 1))) {
+    // (empty lines' slots are zeroed by the class-list pass)
+    if (a.counts) {
         for (int o = 32; o > 0; o >>= 1) iters += __shfl_xor(iters, o, 64);
         if (NW == 1) {
             if (tid == 0) a.counts[line] = iters;
@@ -745,7 +882,6 @@ struct PvcsArgs {
     const LineMeta* lines;
     const float* rev;
     float* dose;
-    int ncones;
     int q0, q1;                 // cones of this pass
     int nx, ny;                 // full volume dims (x, y)
     int x0, y0, z0, sx, sy, sz; // PVCS index box
@@ -762,10 +898,7 @@ struct PvcsArgs {
 // crop box receive nothing from any cone and leave at once; the others sum every cone's trilinear
 // REV dose (compact store, REV2XYZdose's fetch) in a register and add it to the dose volume once.
 __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
-    __shared__ ConeDev sc[kMaxRays];
     const int tid = threadIdx.x;
-    for (int q = tid; q < a.ncones; q += 256) sc[q] = a.cones[q];
-    __syncthreads();
     const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
     const int txi = (int)(tile % (uint32_t)a.tx);
     const int tyi = (int)((tile / (uint32_t)a.tx) % (uint32_t)a.ty);
@@ -800,12 +933,15 @@ __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
             for (int t = 0; t < 4; t++) mt[u][t] = LineMeta{0u, 0, 0};
             const int q = q0 + u;
             if (q >= a.q1) continue;
-            const ConeDev& c = sc[q];
-            const v3 r = c.a(g) + c.t;
-            if (r.y >= (float)c.nx || r.z >= (float)c.ny || r.x >= (float)c.nz || r.x < 0.f || r.y < 0.f || r.z < 0.f)
+            const uniform_ptr<ConeDev> c = as_uniform(a.cones) + q;
+            m33 ca;
+            for (int w = 0; w < 9; w++) ca.m[w] = c->a.m[w];
+            const int nx = c->nx, ny = c->ny, nz = c->nz;
+            const v3 r = ca(g) + mk3(c->t.x, c->t.y, c->t.z);
+            if (r.y >= (float)nx || r.z >= (float)ny || r.x >= (float)nz || r.x < 0.f || r.y < 0.f || r.z < 0.f)
                 continue;
             const float ub = (r.y + 0.5f) - 0.5f, vb = (r.z + 0.5f) - 0.5f, wb = (r.x + 0.5f) - 0.5f;
-            if (!(ub > -1.f && vb > -1.f && wb > -1.f && ub < (float)c.nx && vb < (float)c.ny && wb < (float)c.nz))
+            if (!(ub > -1.f && vb > -1.f && wb > -1.f && ub < (float)nx && vb < (float)ny && wb < (float)nz))
                 continue;
             const float fu = floorf(ub), fv = floorf(vb), fw = floorf(wb);
             ok[u] = true;
@@ -813,7 +949,7 @@ __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
             fa[u] = ub - fu;
             fb[u] = vb - fv;
             fc[u] = wb - fw;
-            meta_pairs(a.lines, c.line0, c.ny, c.nz, (int)fv, (int)fw, mt[u]);
+            meta_pairs(a.lines, c->line0, ny, nz, (int)fv, (int)fw, mt[u]);
         }
 #pragma unroll
         for (int u = 0; u < kPvcsGroup; u++) {
@@ -1143,9 +1279,7 @@ struct ClassArgs {
     int ncls;
     uint32_t* bcnt;        // [blocks][kConeClasses]: counts, then the blocks' list offsets
     uint32_t* tot;         // [kConeClasses]: lines per class
-    ConeLine* list;        // lines with their cone and record, class by class
-    const ConeDev* cones;  // the beam's cones (the entries' cone indices)
-    int ncones;
+    ConeLine* list;        // the lines' entries, class by class
     uint32_t* counts;      // profiling: the slots of empty lines are zeroed here (or nullptr)
 };
 
@@ -1200,7 +1334,7 @@ __global__ void __launch_bounds__(kClassBlock) class_scan_kernel(ClassArgs a, ui
     }
 }
 
-__global__ void __launch_bounds__(kClassBlock) class_scatter_kernel(ClassArgs a) {
+__global__ void __launch_bounds__(kClassBlock) class_scatter_kernel(ClassArgs a, ConeArgs ca) {
     __shared__ uint32_t s[kClassBlock / 64][kConeClasses];
     const uint64_t i = (uint64_t)blockIdx.x * kClassBlock + threadIdx.x;
     const int cls = i < a.n ? class_of_line(a, a.lines[i].len) : -1;
@@ -1216,10 +1350,22 @@ __global__ void __launch_bounds__(kClassBlock) class_scatter_kernel(ClassArgs a)
     if (cls >= 0) {
         uint32_t off = a.bcnt[(size_t)blockIdx.x * kConeClasses + cls] + rank;
         for (int q = 0; q < w; q++) off += s[q][cls];
+        const LineMeta meta = a.lines[i];
+        const int q = cone_of_line(ca.cones, ca.ncones, i);
+        const ConeDev& c = ca.cones[q];
+        const uint32_t l = (uint32_t)(i - c.line0), tz = l / (uint32_t)c.ny, ty = l - tz * (uint32_t)c.ny;
+        int ja, jb;
+        line_interior(ca, c, (int)ty, (int)tz, meta.i0, meta.len, ja, jb);
         ConeLine e;
         e.line = (uint32_t)i;
-        e.cone = (uint32_t)cone_of_line(a.cones, a.ncones, i);
-        e.meta = a.lines[i];
+        e.off = meta.off;
+        e.i0 = meta.i0;
+        e.len = meta.len;
+        e.ja = (int16_t)ja;
+        e.jb = (int16_t)jb;
+        e.ty = (uint16_t)ty;
+        e.tz = (uint16_t)tz;
+        e.cone = (uint32_t)q;
         a.list[off] = e;
     }
 }
@@ -1254,7 +1400,7 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     v3 rv = mk3(p.rev_latspacing, p.rev_longspacing, p.rev_latspacing);
     v3 off = mk3((g.lim_min.x - p.start[0]) / p.voxel[0], (g.lim_min.y - p.start[1]) / p.voxel[1],
                  (g.lim_min.z - p.start[2]) / p.voxel[2]);
-    uint64_t line0 = 0, roff = 0;
+    uint64_t line0 = 0;
     const int half = (int)p.ntheta / 2;
     for (int r = 0; r < g.nrays; r++) {
         float th = ctx->theta[r] * 3.14159265358979323846f / 180.f;
@@ -1272,11 +1418,14 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
         c.ny = (int)g.rev_size[r][1];
         c.nz = (int)g.rev_size[r][2];
         c.rowf = r % half;
-        c.rowb = (int)p.ntheta - 1 - (r % half);
         c.line0 = line0;
-        c.off = roff;
         line0 += (uint64_t)c.ny * c.nz;
-        roff += (uint64_t)c.nx * c.ny * c.nz;
+        // PVCS index along the grid's axes (lines run along REV y, tY counts along z, tZ along x)
+        dm33 gm = dm_mul(binv, ki);
+        c.g0 = dm_apply_f(gm, c.rs) + off;
+        c.gx = mk3((float)gm.m[1], (float)gm.m[4], (float)gm.m[7]);
+        c.gy = mk3((float)gm.m[2], (float)gm.m[5], (float)gm.m[8]);
+        c.gz = mk3((float)gm.m[0], (float)gm.m[3], (float)gm.m[6]);
     }
     CCCS_HIP(hipMemcpyAsync(d_cones, hc, sizeof(ConeDev) * g.nrays, hipMemcpyHostToDevice, ctx->stream));
     // the host staging may be the caller's stack (no-allocation entry point): the copy completes first
@@ -1289,6 +1438,7 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     ca.list = nullptr;
     ca.dt = d_dt;
     ca.tables = ctx->d_tables;
+    ca.steps = ctx->d_steps;
     ca.cones = d_cones;
     ca.lines = d_lines;
     ca.rev = nullptr;
@@ -1305,13 +1455,13 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     ca.bev_size = mk3((float)g.bev_size[0], (float)g.bev_size[1], (float)g.bev_size[2]);
     ca.bb0 = ldu3(p.bbox_start);
     ca.bb1 = ca.bb0 + ldu3(p.bbox_size);
-    ca.bbx = (int)p.bbox_size[0]; ca.bby = (int)p.bbox_size[1]; ca.bbz = (int)p.bbox_size[2];
     if (g.total_lines == 0) return CCCS_OK;
     {
         dim3 blk(64, 4, 1), grd((unsigned)((p.size[0] + 63) / 64), (unsigned)((p.size[1] + 3) / 4), p.size[2]);
         hipLaunchKernelGGL(pack_dt_kernel, grd, blk, 0, ctx->stream, (const float*)ctx->d_dens, d_terma,
                            (int)p.size[0], (int)p.size[1], (int)p.size[2], (int)p.bbox_start[0],
-                           (int)p.bbox_start[1], (int)p.bbox_start[2], ca.bbx, ca.bby, ca.bbz, d_dt);
+                           (int)p.bbox_start[1], (int)p.bbox_start[2], (int)p.bbox_size[0], (int)p.bbox_size[1],
+                           (int)p.bbox_size[2], d_dt);
         CCCS_HIP(hipGetLastError());
     }
     // pass 1: stored interval of every line, then offsets into the compact store
@@ -1325,11 +1475,10 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     // many short lines are not held to the occupancy of the longest
     uint32_t maxn = 1;
     for (int r = 0; r < g.nrays; r++) maxn = std::max(maxn, g.rev_size[r][0]);
-    int cls_lo[kConeClasses], cls_hi[kConeClasses], cls_threads[kConeClasses], ncls = 0;
+    int cls_hi[kConeClasses], cls_threads[kConeClasses], ncls = 0;
     for (int ci = 0, lo = 1; ci < kConeClasses && lo <= (int)maxn; ci++) {
         const int hi = ci == kConeClasses - 1 ? (int)maxn : std::min<int>(ctx->sched.cone_class_len[ci], (int)maxn);
         if (hi < lo) continue;
-        cls_lo[ncls] = lo;
         cls_hi[ncls] = hi;
         cls_threads[ncls] = ctx->sched.cone_class_threads[ci];
         ncls++;
@@ -1342,15 +1491,13 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     for (int c = 0; c < kConeClasses; c++) cl.hi[c] = c < ncls ? cls_hi[c] : 0;
     cl.ncls = ncls;
     cl.counts = ca.counts;
-    cl.cones = d_cones;
-    cl.ncones = g.nrays;
     const uint64_t ncb = (g.total_lines + kClassBlock - 1) / kClassBlock;
     CCCS_TRY(S.get(ctx->cls_cnt, (size_t)ncb * kConeClasses + kConeClasses, &cl.bcnt));
     cl.tot = cl.bcnt + (size_t)ncb * kConeClasses;
     CCCS_TRY(S.get(ctx->cls_list, g.total_lines, &cl.list));
     hipLaunchKernelGGL(class_count_kernel, dim3((unsigned)ncb), dim3(kClassBlock), 0, ctx->stream, cl);
     hipLaunchKernelGGL(class_scan_kernel, dim3(1), dim3(kClassBlock), 0, ctx->stream, cl, (uint32_t)ncb);
-    hipLaunchKernelGGL(class_scatter_kernel, dim3((unsigned)ncb), dim3(kClassBlock), 0, ctx->stream, cl);
+    hipLaunchKernelGGL(class_scatter_kernel, dim3((unsigned)ncb), dim3(kClassBlock), 0, ctx->stream, cl, ca);
     CCCS_HIP(hipGetLastError());
     CCCS_HIP(hipMemcpyAsync(S.host_small, ca.lines + (g.total_lines - 1), sizeof(LineMeta), hipMemcpyDeviceToHost,
                             ctx->stream));
@@ -1370,9 +1517,7 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     uint64_t list_off = 0;
     for (int c = 0; c < ncls; c++) {
         if (cls_n[c] == 0) continue;
-        ca.len_lo = cls_lo[c];
-        ca.len_hi = cls_hi[c];
-        ca.maxn = ca.len_hi;
+        ca.maxn = cls_hi[c];
         ca.list = cl.list + list_off;
         list_off += cls_n[c];
         const size_t lds = cone_lds_bytes((uint32_t)ca.maxn, ca.ramp_min <= ca.maxn);
@@ -1386,7 +1531,6 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     pa.lines = ca.lines;
     pa.rev = ca.rev;
     pa.dose = d_dose;
-    pa.ncones = g.nrays;
     pa.nx = (int)p.size[0];
     pa.ny = (int)p.size[1];
     pa.x0 = g.pvcs_lo[0]; pa.y0 = g.pvcs_lo[1]; pa.z0 = g.pvcs_lo[2];

@@ -298,7 +298,22 @@ extern "C" int cccs_ctx_create(const cccs_problem* p, int device, cccs_ctx** out
         for (uint32_t r = 0; r < nr; r++) MIW[r] = 1.0f / (r == 0 ? MR[0] : (MR[r] - MR[r - 1]));
         if (hipMalloc((void**)&c->d_tables, tab.size() * sizeof(float)) != hipSuccess) { st = set_error(CCCS_ENOMEM, "tables"); break; }
         if (hipMemcpy(c->d_tables, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) { st = set_error(CCCS_EDEVICE, "tables copy"); break; }
-        c->resident = nv * sizeof(float) + tab.size() * sizeof(float);
+        // radial steps of each kernel row pair (row q walks toward lower, ntheta-1-q toward higher indices)
+        const uint32_t half = p->ntheta / 2;
+        std::vector<RampStep> steps((size_t)half * nr);
+        for (uint32_t q = 0; q < half; q++)
+            for (uint32_t r = 0; r < nr; r++) {
+                const float* kb = p->kernel + (size_t)q * nr;
+                const float* kf = p->kernel + (size_t)(p->ntheta - 1 - q) * nr;
+                RampStep& e = steps[(size_t)q * nr + r];
+                e.r = (double)R[r];
+                e.sigb = (double)((kb[r] - (r == 0 ? 0.f : kb[r - 1])) * IW[r]);
+                e.sigf = (double)((kf[r] - (r == 0 ? 0.f : kf[r - 1])) * IW[r]);
+                e.pad = 0.0;
+            }
+        if (hipMalloc((void**)&c->d_steps, steps.size() * sizeof(RampStep)) != hipSuccess) { st = set_error(CCCS_ENOMEM, "tables"); break; }
+        if (hipMemcpy(c->d_steps, steps.data(), steps.size() * sizeof(RampStep), hipMemcpyHostToDevice) != hipSuccess) { st = set_error(CCCS_EDEVICE, "tables copy"); break; }
+        c->resident = nv * sizeof(float) + tab.size() * sizeof(float) + steps.size() * sizeof(RampStep);
         uint64_t h = 1469598103934665603ull;
         const uint32_t* bits = reinterpret_cast<const uint32_t*>(p->density);
         for (size_t i = 0; i < nv; i++) h = (h ^ bits[i]) * 1099511628211ull;
@@ -323,6 +338,7 @@ extern "C" int cccs_ctx_destroy(cccs_ctx* c) {
     if (c->cstream) (void)hipStreamSynchronize(c->cstream);
     if (c->d_dens) (void)hipFree(c->d_dens);
     if (c->d_tables) (void)hipFree(c->d_tables);
+    if (c->d_steps) (void)hipFree(c->d_steps);
     c->terma.release(); c->fmap.release(); c->partial.release(); c->rev.release(); c->cones.release();
     c->dose.release(); c->col.release(); c->lines.release(); c->scan.release(); c->dt.release();
     c->cls_cnt.release(); c->cls_list.release();

@@ -36,16 +36,22 @@ constexpr int kMaxRays = 48;      // ntheta/2 * nphi <= 48 cone lines per beam i
 constexpr int kMaxLine = 1024;    // REV line limit of the reference (nvbbRayConvolve_host.cu:567)
 constexpr int kMaxRadii = 32;
 
-// Per-cone constants of the plain beam path, consumed by the cone and PVCS kernels.
+// Per-cone constants of the plain beam path, consumed by the cone and PVCS kernels (as scalar loads:
+// every wave works on one cone at a time).
 struct ConeDev {
-    m33 kinv;          // BEV <- REV (index units)
     m33 a;             // REV <- PVCS index: kernel_fwd * beam_fwd
-    v3 rs;             // REV origin in REV index units (revStart / rev spacing)
     v3 t;              // REV coordinate of PVCS index (0,0,0)
     int nx, ny, nz;    // line length, lines along y, lines along z
-    int rowf, rowb;    // kernel rows of the forward / backward walk
+    int rowf;          // kernel row of the forward walk (the backward row mirrors it)
     uint64_t line0;    // first global line index of this cone
-    uint64_t off;      // float offset of this cone's REV dose grid
+    m33 kinv;          // BEV <- REV (index units)
+    v3 rs;             // REV origin in REV index units (revStart / rev spacing)
+    v3 g0, gx, gy, gz; // PVCS index of REV sample (i, tY, tZ): g0 + i gx + tY gy + tZ gz
+};
+
+// One radial interval (R_{s-1}, R_s] of a kernel row pair: its end and the rows' slopes in it.
+struct RampStep {
+    double r, sigb, sigf, pad;
 };
 
 struct BeamGeom {
@@ -97,8 +103,9 @@ constexpr int kRaySets = 4;  // most cone directions of the beamlet pipeline in 
 // which samples contribute.
 struct Schedule {
     // plain-path cone lines whose valid segment has at least this many samples use the
-    // segment-sum walk (O(nradii) per destination) instead of the sequential walk (O(line))
-    int cone_ramp_min = 64;
+    // segment-sum walk (O(nradii) per destination) instead of the sequential walk (O(line)); 24, 32 and
+    // 40 run the 128^3 water beam in 1241, 1235 and 1241 us, 64 in 1391
+    int cone_ramp_min = 32;
     // cones per pass of the PVCS resample (each pass adds its cones' dose to the volume); 0: from
     // the size of the beam's REV data
     int pvcs_pass_cones = 0;
@@ -143,6 +150,7 @@ struct cccs_ctx {
     uint32_t max_rev_beam[3] = {0, 0, 0};
     int nrays = 0;
     float* d_dens = nullptr;
+    cccs::RampStep* d_steps = nullptr;  // [ntheta/2][nradii] radial steps of the cone walks
     float* d_tables = nullptr;  // kernel (ntheta*nradii) | radii | inverse widths | mean radii | inverse widths
     size_t resident = 0;
     cccs::DevBuf terma, fmap, partial, rev, cones, dose, col, lines, scan, dt;
