@@ -20,6 +20,16 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb) {
     return x * per + (x < rem ? x : rem) + idx;
 }
 
+// The same with chunks of `chunk` consecutive work items going to the XCDs in turn: neighbours still
+// share an L2, and work that is unevenly spread over the items (voxels outside the field, lines of
+// different lengths) still reaches every XCD.  A bijection on [0, nb).
+__device__ __forceinline__ uint32_t xcd_chunks(uint32_t b, uint32_t nb, uint32_t chunk) {
+    const uint32_t super = 8 * chunk, s0 = b / super * super;
+    if (super > nb - s0) return b;  // the incomplete last round
+    const uint32_t r = b - s0;
+    return s0 + (r % 8) * chunk + r / 8;
+}
+
 // Sums one uint32 per thread over the workgroup (LDS tree, <= 256 threads) into part[slot].
 // Sums one uint32 per lane over a 64-lane workgroup into part[slot] (no LDS).
 __device__ __forceinline__ void wave_count(uint32_t v, uint32_t* __restrict__ part, size_t slot) {
