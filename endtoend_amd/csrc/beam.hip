@@ -681,7 +681,7 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     __shared__ double s_tot[2 * NW];
     __shared__ int s_red[NW][3];
     __shared__ uint32_t s_cnt[NW];
-    const uint32_t slot = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t slot = xcd_chunks(blockIdx.x, gridDim.x, 64);
     const uniform_ptr<ConeLine> en = as_uniform(a.list) + slot;
     const uint32_t line = en->line, off = en->off;
     const int i0 = en->i0, m = en->len, ja = en->ja, jb = en->jb, tY = en->ty, tZ = en->tz;
@@ -914,7 +914,7 @@ struct PvcsArgs {
 // REV dose (compact store, REV2XYZdose's fetch) in a register and add it to the dose volume once.
 __global__ void __launch_bounds__(256) pvcs_kernel(PvcsArgs a) {
     const int tid = threadIdx.x;
-    const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_chunks(blockIdx.x, gridDim.x, 64);
     const int txi = (int)(tile % (uint32_t)a.tx);
     const int tyi = (int)((tile / (uint32_t)a.tx) % (uint32_t)a.ty);
     const int tzi = (int)(tile / ((uint32_t)a.tx * (uint32_t)a.ty));

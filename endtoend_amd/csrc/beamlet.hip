@@ -772,7 +772,7 @@ __device__ __forceinline__ bool bl_gather_hit(const BatchDev& B, const BlConeDev
 constexpr int kGatherX = 4;  // the tile's depth along pX
 constexpr int kGatherY = 4;  // pY voxels per lane
 __global__ void __launch_bounds__(64) bl_gather_kernel(BlArgs a, uint32_t ntiles) {
-    const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_chunks(blockIdx.x, gridDim.x, 64);
     if (tile >= ntiles) return;
     const int lo = a.tile_batch ? (int)a.tile_batch[tile] : 0;
     const BatchDev& B = a.batches[lo];

@@ -22,7 +22,9 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb) {
 
 // The same with chunks of `chunk` consecutive work items going to the XCDs in turn: neighbours still
 // share an L2, and work that is unevenly spread over the items (voxels outside the field, lines of
-// different lengths) still reaches every XCD.  A bijection on [0, nb).
+// different lengths) still reaches every XCD.  A bijection on [0, nb).  Against one range per XCD, chunks
+// of 64: PVCS 276 -> 174 us per pass and cone kernel -4 % (thorax beam), beamlet gather 199 -> 187 us
+// (thorax, 3 beams); chunks of 16 and 256 are within 2 %.
 __device__ __forceinline__ uint32_t xcd_chunks(uint32_t b, uint32_t nb, uint32_t chunk) {
     const uint32_t super = 8 * chunk, s0 = b / super * super;
     if (super > nb - s0) return b;  // the incomplete last round
