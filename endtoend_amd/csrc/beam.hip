@@ -252,18 +252,18 @@ __global__ void __launch_bounds__(256) crop_final_kernel(const float* __restrict
     if (t < 7) out[t] = s[t][0];
 }
 
-// A class-list entry: all that a workgroup needs of its line, as one scalar load.  Samples
+// A class-list entry: all that a workgroup needs of its line, as one 16-byte scalar load.  Samples
 // [ja, jb] of the stored interval lie inside the crop box, the calc_bbox and the interpolation range
-// by a margin that covers FP32 rounding; the others are tested one by one.
+// by a margin that covers FP32 rounding (relative to i0; ja > jb: none); the others are tested one by
+// one.
 struct ConeLine {
-    uint32_t line;     // global line index (profiling counters)
-    uint32_t off;      // first stored sample in the REV store
-    int16_t i0, len;   // stored interval
-    int16_t ja, jb;    // interior samples, relative to i0 (ja > jb: none)
-    uint16_t ty, tz;   // line of the cone's grid
-    uint32_t cone;
+    uint32_t off;   // first stored sample in the REV store
+    uint32_t tyz;   // line of the cone's grid: ty | tz << ConeDev::tybits (a cone has < 2^31 lines)
+    uint32_t seg;   // i0 | (len - 1) << 10 | ja << 20 (lines have at most 1024 samples)
+    uint32_t last;  // jb + 1 | cone << 11
 };
-static_assert(sizeof(ConeLine) == 24, "six dwords");
+static_assert(kMaxLine <= 1024 && kMaxRays <= 64, "fields of a class-list entry");
+static_assert(sizeof(ConeLine) == 16, "four dwords");
 
 // Read-only data at wave-uniform addresses, loaded through the scalar unit.
 template <class T>
@@ -683,9 +683,11 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     __shared__ uint32_t s_cnt[NW];
     const uint32_t slot = xcd_chunks(blockIdx.x, gridDim.x, 64);
     const uniform_ptr<ConeLine> en = as_uniform(a.list) + slot;
-    const uint32_t line = en->line, off = en->off;
-    const int i0 = en->i0, m = en->len, ja = en->ja, jb = en->jb, tY = en->ty, tZ = en->tz;
-    const uniform_ptr<ConeDev> c = as_uniform(a.cones) + en->cone;
+    const uint32_t off = en->off, tyz = en->tyz, seg = en->seg, last = en->last;
+    const int i0 = (int)(seg & 1023u), m = (int)(seg >> 10 & 1023u) + 1, ja = (int)(seg >> 20);
+    const int jb = (int)(last & 2047u) - 1;
+    const uniform_ptr<ConeDev> c = as_uniform(a.cones) + (last >> 11);
+    const int tY = (int)(tyz & ((1u << c->tybits) - 1u)), tZ = (int)(tyz >> c->tybits);
     const int rowf = c->rowf;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int nr = a.nradii;
@@ -875,6 +877,7 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     }
     // (empty lines' slots are zeroed by the class-list pass)
     if (a.counts) {
+        const size_t line = (size_t)c->line0 + (uint32_t)tZ * (uint32_t)c->ny + (uint32_t)tY;
         for (int o = 32; o > 0; o >>= 1) iters += __shfl_xor(iters, o, 64);
         if (NW == 1) {
             if (tid == 0) a.counts[line] = iters;
@@ -1262,7 +1265,9 @@ int context_scratch(cccs_ctx* ctx, BeamScratch& S) {
 int run_crop(BeamScratch& S, const float* d_terma, const cccs_beam& b, float* red_host) {
     cccs_ctx* ctx = S.ctx;
     float* part = nullptr;
+    const size_t used = S.used;
     CCCS_TRY(S.get(ctx->partial, kCropBlocks * 8 + 8, &part));
+    S.used = used;  // the partials are read back below: what follows in a fixed array takes their place
     Rot2 rot = rot2_beam_fwd(b.azimuth, b.zenith, b.coll);
     const cccs_problem& p = ctx->prob;
     size_t n = bbox_voxels(ctx);
@@ -1372,15 +1377,10 @@ __global__ void __launch_bounds__(kClassBlock) class_scatter_kernel(ClassArgs a,
         int ja, jb;
         line_interior(ca, c, (int)ty, (int)tz, meta.i0, meta.len, ja, jb);
         ConeLine e;
-        e.line = (uint32_t)i;
         e.off = meta.off;
-        e.i0 = meta.i0;
-        e.len = meta.len;
-        e.ja = (int16_t)ja;
-        e.jb = (int16_t)jb;
-        e.ty = (uint16_t)ty;
-        e.tz = (uint16_t)tz;
-        e.cone = (uint32_t)q;
+        e.tyz = ty | tz << c.tybits;
+        e.seg = (uint32_t)meta.i0 | (uint32_t)(meta.len - 1) << 10 | (uint32_t)ja << 20;
+        e.last = (uint32_t)(jb + 1) | (uint32_t)q << 11;
         a.list[off] = e;
     }
 }
@@ -1434,6 +1434,8 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
         c.nz = (int)g.rev_size[r][2];
         c.rowf = r % half;
         c.line0 = line0;
+        c.tybits = 0;
+        while ((uint64_t(1) << c.tybits) < (uint64_t)c.ny) c.tybits++;
         line0 += (uint64_t)c.ny * c.nz;
         // PVCS index along the grid's axes (lines run along REV y, tY counts along z, tZ along x)
         dm33 gm = dm_mul(binv, ki);

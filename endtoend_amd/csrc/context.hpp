@@ -43,6 +43,7 @@ struct ConeDev {
     v3 t;              // REV coordinate of PVCS index (0,0,0)
     int nx, ny, nz;    // line length, lines along y, lines along z
     int rowf;          // kernel row of the forward walk (the backward row mirrors it)
+    int tybits;        // bits of a line index along y (class-list entries)
     uint64_t line0;    // first global line index of this cone
     m33 kinv;          // BEV <- REV (index units)
     v3 rs;             // REV origin in REV index units (revStart / rev spacing)
