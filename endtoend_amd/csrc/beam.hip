@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(256) crop_partial_kernel(const float* __restri
             int x = (int)(v % bx);
             int y = (int)((v / bx) % by);
             int z = (int)(v / ((size_t)bx * by));
-            v3 b = rot2(rot, mk3((float)x, (float)y, (float)z));
+            v3 b = rot_fwd(rot, mk3((float)x, (float)y, (float)z));
             mn0 = fminf(mn0, b.x); mn1 = fminf(mn1, b.y); mn2 = fminf(mn2, b.z);
             mx0 = fmaxf(mx0, b.x); mx1 = fmaxf(mx1, b.y); mx2 = fmaxf(mx2, b.z);
             cnt += 1.f;
@@ -264,14 +264,6 @@ struct ConeLine {
 };
 static_assert(kMaxLine <= 1024 && kMaxRays <= 64, "fields of a class-list entry");
 static_assert(sizeof(ConeLine) == 16, "four dwords");
-
-// Read-only data at wave-uniform addresses, loaded through the scalar unit.
-template <class T>
-using uniform_ptr = const __attribute__((address_space(4))) T*;
-template <class T>
-__device__ __forceinline__ uniform_ptr<T> as_uniform(const T* p) {
-    return (uniform_ptr<T>)p;
-}
 
 struct ConeArgs {
     const float2* dt;         // {density, TERMA (0 outside the calc_bbox)} over the CT grid
@@ -1030,7 +1022,7 @@ __global__ void __launch_bounds__(64) projection_kernel(const float* __restrict_
         const int sx = sr % 3 - 1, sz = sr / 3 - 1;
         const v3 fcs = mk3(b.bsx * ((float)rx + 0.5f * (float)sx - (float)b.fx * 0.5f + 0.5f), 0.f,
                            b.bsy * ((float)rz + 0.5f * (float)sz - (float)b.fy * 0.5f + 0.5f));
-        v3 ctr = rot2(b.inv, fcs) + b.iso;
+        v3 ctr = rot_inv(b.inv, fcs) + b.iso;
         ctr = ctr + 1e-9f;
         const v3 sd = ctr - b.src;
         const v3 sink = b.src + 3.f * sd;

@@ -38,10 +38,10 @@ struct Rot1 {
     v3 a;
     float s, c;
 };
-CCCS_HD v3 rot1(const Rot1& R, v3 p) { return rodrigues(p, R.a, R.s, R.c); }
-
 // invRotateBeamlet / rotateBeamlet (CudaUtilities/geometry.cu:99-115): a rotation about
 // (sin(-phi), 0, cos(-phi)) by -theta (beamlet frame -> BEV) or +theta (BEV -> beamlet frame).
+// Both axes lie in the x-z plane.
+CCCS_HD v3 rot1(const Rot1& R, v3 p) { return rot_xz(p, R.a.x, R.a.z, R.s, R.c); }
 static Rot1 beamlet_rot(float theta, float phi, bool to_bev) {
     Rot1 r;
     float s, c;
@@ -118,6 +118,7 @@ struct BlArgs {
     float delr;
     v3 rvs, rrv;                // REV spacings (lat, long, lat) and reciprocals
     VolDesc vd;
+    v3 ivoxel;                  // 1 / vd.voxel
     SpecDev spec;
     float bhc;
     uint32_t* line_cone;        // grid (= batch) of every line, written by the interval pass
@@ -138,7 +139,7 @@ CCCS_HD int find_cone(const BlConeDev* __restrict__ c, int n, uint64_t line) {
 // nvbbRayConvolve_device.cu:33-41).
 CCCS_HD v3 rev_to_packed(const BlConeDev& c, v3 rrv, int tX, int tY, int tZ) {
     v3 q = mk3(fmaf(c.minc.x, rrv.x, (float)tZ), fmaf(c.minc.y, rrv.y, (float)tX), fmaf(c.minc.z, rrv.z, (float)tY));
-    return rot2(c.kinv, q) + 0.5f;
+    return rot_inv(c.kinv, q) + 0.5f;
 }
 
 // Interval of stored samples of every line of one cone direction: the line clipped to the packed
@@ -242,15 +243,16 @@ CCCS_HD PillarRec pillar_rec(const BeamletDev& d) {
 
 // PVCS point [cm] where the sample's TERMA is evaluated (device.cu:170-180).
 CCCS_HD v3 bl_terma_point(const BlArgs& a, const BatchDev& B, const PillarRec& bl, v3 inp) {
-    const v3 g = rot2(B.beam_inv, rot1(bl.inv, inp));
+    const v3 g = rot_inv(B.beam_inv, rot1(bl.inv, inp));
     return mk3(fmaf(g.x, a.rvs.x, bl.pst.x), fmaf(g.y, a.rvs.y, bl.pst.y), fmaf(g.z, a.rvs.z, bl.pst.z));
 }
 
 // Density at the sample (device.cu:213-223): trilinear, border 0.
-__device__ __forceinline__ float bl_density(const BlArgs& a, const BatchDev& B, const PillarRec& bl, v3 inp) {
-    const v3 g2 = rot2(B.beam_inv, rot1(bl.inv, inp * a.rvs)) + bl.pst;
-    const v3 gi = (g2 - a.vd.start) / a.vd.voxel;
-    return tex3_border(a.dens, a.vd.nx, a.vd.ny, a.vd.nz, gi.x + 0.5f, gi.y + 0.5f, gi.z + 0.5f);
+__device__ __forceinline__ float bl_density(const BlArgs& a, const MarchVol& vol, const BatchDev& B, const PillarRec& bl,
+                                            v3 inp) {
+    const v3 g2 = rot_inv(B.beam_inv, rot1(bl.inv, inp * a.rvs)) + bl.pst;
+    const v3 gi = div_by(g2 - a.vd.start, a.vd.voxel, a.ivoxel);
+    return tex3_march(vol, gi.x + 0.5f, gi.y + 0.5f, gi.z + 0.5f);
 }
 
 // Cumulative kernel of one row, linear between radii (the reference's clamped linear texture
@@ -262,282 +264,334 @@ __device__ __forceinline__ float kc_at(float r, const float4* __restrict__ tab, 
     return iv.y + (r - iv.x) * iv.z;
 }
 
-// The grid and batch fields the mapping reads sit in LDS; this compiler-only barrier keeps their
-// reads inside each pass iteration (next to their use) instead of holding ~50 of them in VGPRs
-// across the pass.
-__device__ __forceinline__ void lds_reload_fence() { __asm__ volatile("" ::: "memory"); }
-
 constexpr int kStagePillars = 64;  // footprint pillars of one line whose beamlet data sits in LDS
 
-// Stage 1 of a cone direction, one wave per REV line: pillar mapping of every stored sample and
-// the beamlet-footprint test (fluence cell of the sample == its beamlet).  A line without footprint
+__device__ __forceinline__ int lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ float lane_f(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// A record at a wave-uniform address, through the scalar unit; only the fields that are used load.
+template <class T>
+__device__ __forceinline__ T uniform_copy(const T* p) {
+    static_assert(sizeof(T) % 4 == 0, "whole dwords");
+    uint32_t w[sizeof(T) / 4];
+    const uniform_ptr<uint32_t> s = as_uniform(reinterpret_cast<const uint32_t*>(p));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); i++) w[i] = s[i];
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
+// Stage 1 of a cone direction, one wave per stride of REV lines: pillar mapping of every stored sample
+// and the beamlet-footprint test (fluence cell of the sample == its beamlet).  A line without footprint
 // samples carries no TERMA, so all its cone dose is zero: it is marked empty.  Otherwise the half
 // steps (0.5 * delr * density, -1 for walls) go to H, TERMA slots are zeroed, and the footprint
 // samples are queued for their Siddon TERMA.
 //
-// The per-sample work is a chain of dependent memory trips (line record, grid tables, beamlet
-// record, density taps), so the kernel keeps each chain short: the line's grid comes from the line
-// table built by the interval pass (no search), its grid and batch tables load together, and the
-// beamlet data of the line's footprint pillars is staged in LDS once, while the pillar
-// classification runs, instead of being read per sample by the density pass.
+// Most stored samples are far from every footprint (1 to 2 % are candidates, 7 to 15 % reach the exact
+// mapping), and most lines have a handful of candidates, so the kernel's time is its instructions per
+// line.  A wave takes the records of 64 lines at once, one per lane (line record, grid indices and
+// affine start cost once per 64 lines), culls the samples line by line (pass A.1: one multiply-add, a
+// fraction and a compare per axis and sample), and collects the candidates of consecutive lines
+// until the list is full, so that the exact test (pass A.2) runs on full waves.  Lines with footprint
+// samples then take passes B.1 and B.2.  The grid's and batch's fields come through the scalar
+// unit.
 __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restrict__ H, TermaReq* __restrict__ q,
                                                        uint32_t subcap, uint32_t* __restrict__ qcnt) {
-    __shared__ uint8_t s_fp[kMaxLine];            // bit 0: footprint sample, bit 1: on the exact list
-    __shared__ short s_list[kMaxLine];            // compacted work list of the current pass
-    __shared__ uint32_t s_pil[kPillarBits / 32];  // pillars with footprint samples on this line
+    __shared__ uint16_t s_cand[kMaxLine];         // candidates: lane of the line << 10 | sample
+    __shared__ uint16_t s_cpil[kMaxLine];         // footprint samples among them: their pillar, else kNoPil
+    __shared__ uint16_t s_list[kMaxLine];         // one line's samples for pass B.2
+    __shared__ uint32_t s_foot[kMaxLine / 32];    // one line's footprint samples
+    __shared__ uint64_t s_exact[kMaxLine / 64];   // one line's samples on s_list
+    __shared__ uint32_t s_pil[kPillarBits / 32];  // pillars with footprint samples on the line
     __shared__ uint16_t s_rank[kPillarBits / 32]; // footprint pillars in the words before each word
     __shared__ PillarRec s_rec[kStagePillars];    // their beamlet data, in pillar order
-    __shared__ BlConeDev s_cone;                  // the line's grid and batch records
-    __shared__ BatchDev s_batch;
-    static_assert(sizeof(BlConeDev) % 8 == 0 && sizeof(BatchDev) % 8 == 0 &&
-                      (sizeof(BlConeDev) + sizeof(BatchDev)) / 8 <= 64, "one 8-byte word per lane");
-    uint32_t stored = 0;
-    uint32_t staged = 0xffffffffu;  // grid whose records sit in LDS
-    for (uint64_t line = xcd_remap(blockIdx.x, gridDim.x); line < a.nlines; line += gridDim.x) {
-    const LineMeta meta = a.lines[line];
-    const uint32_t ci = a.line_cone[line];
-    if (meta.len <= 0) continue;
-    // the lane id is opaque per line, so that the lane arithmetic is redone per line rather than
-    // hoisted out of the line loop into registers held for the whole kernel
-    int tid = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid));
+    constexpr uint16_t kNoPil = 0xffff;
+    const int tid = threadIdx.x;
     const uint64_t lt = (1ull << tid) - 1ull;
-    // each wave walks a stride of lines; a line's TERMA requests go to one of kSubQueues queues,
-    // chosen by its run of 64 consecutive lines: the Siddon stage then marches neighbouring
-    // lines' rays side by side (shared cache lines; -26 % stage time against one queue per wave),
-    // and the lines in flight still spread over every counter
-    const uint32_t sq = (uint32_t)((line >> 6) % kSubQueues);
-    TermaReq* qs = q + (size_t)sq * subcap;
-    // grid ci of a direction belongs to batch ci; both records go to LDS when the line's grid
-    // changes, so the passes below read their fields there instead of from global memory
-    if (ci != staged) {
-        constexpr int nc = (int)(sizeof(BlConeDev) / 8), nb = (int)(sizeof(BatchDev) / 8);
-        if (tid < nc) reinterpret_cast<uint64_t*>(&s_cone)[tid] = reinterpret_cast<const uint64_t*>(a.cones + ci)[tid];
-        else if (tid < nc + nb)
-            reinterpret_cast<uint64_t*>(&s_batch)[tid - nc] = reinterpret_cast<const uint64_t*>(a.batches + ci)[tid - nc];
-        staged = ci;
-        __syncthreads();
+    const MarchVol vol = march_vol(a.dens, a.vd.nx, a.vd.ny, a.vd.nz);
+    uint32_t stored = 0;
+    const uint64_t G = gridDim.x;
+    for (uint64_t base = xcd_remap(blockIdx.x, gridDim.x); base < a.nlines; base += 64 * G) {
+    // this lane's line
+    const uint64_t my_line = base + (uint64_t)tid * G;
+    LineMeta mine{};
+    int my_ci = 0, my_y = 0, my_z = 0;
+    v3 my_p0 = mk3(0.f, 0.f, 0.f);
+    if (my_line < a.nlines) {
+        mine = a.lines[my_line];
+        my_ci = (int)a.line_cone[my_line];
+        const BlConeDev& c = a.cones[my_ci];
+        const uint64_t l = my_line - c.line0;
+        my_z = (int)(l / (uint64_t)c.ny);
+        my_y = (int)(l - (uint64_t)my_z * (uint64_t)c.ny);
+        // affine form of the packed coordinate along the line (matrix rotation): used only to skip
+        // samples that are far from every footprint or inside pillars without footprint samples; the
+        // exact mapping decides every other sample
+        my_p0 = c.kinv_m(mk3(fmaf(c.minc.x, a.rrv.x, (float)my_z), c.minc.y * a.rrv.y,
+                             fmaf(c.minc.z, a.rrv.z, (float)my_y))) + 0.5f;
+        if (mine.len > 0) stored += (uint32_t)mine.len;  // summed over the wave's lanes by wave_count
     }
-    const BlConeDev& c = s_cone;
-    const BatchDev& B = s_batch;
-    const uint64_t l = line - c.line0;
-    const int tY = (int)(l % (uint64_t)c.ny), tZ = (int)(l / (uint64_t)c.ny);
-    const int i0 = meta.i0, m = meta.len;
-    if (tid == 0) stored += (uint32_t)m;  // summed over the wave's lanes by wave_count
-    // affine form of the packed coordinate along the line (matrix rotation): used only to skip
-    // samples that are far from every footprint or inside pillars without footprint samples;
-    // the exact mapping decides every other sample.  Pass A.1 keeps a sample only inside the
-    // footprint half-width fw and inside the batch's depth-linear footprint bounds (cb).
-    const v3 q0 = mk3(fmaf(c.minc.x, a.rrv.x, (float)tZ), c.minc.y * a.rrv.y, fmaf(c.minc.z, a.rrv.z, (float)tY));
-    const v3 p0 = c.kinv_m(q0) + 0.5f;
-    const v3 dl = mk3(c.kinv_m.m[1], c.kinv_m.m[4], c.kinv_m.m[7]);
-    const float pdx = (float)B.pd[0], pdz = (float)B.pd[2], ipdx = 1.f / pdx, ipdz = 1.f / pdz;
-    const float cull = B.fw + 0.05f;
-    const v3 ipd = mk3(ipdx, 1.f / (float)B.pd[1], ipdz);
-    const bool track = B.n <= (int)kPillarBits;
-    for (int k = tid; k < (int)(kPillarBits / 32); k += 64) s_pil[k] = 0u;
-    // pass A.1: affine cull of every sample, candidates compacted into s_list
-    int ncand = 0;
-    for (int base = 0; base < m; base += 64) {
-        const int j = base + tid;
-        bool cand = false;
-        if (j < m) {
-            const float t = (float)(i0 + j);
-            const float px = p0.x + t * dl.x, pz = p0.z + t * dl.z, py = p0.y + t * dl.y;
-            const float xl = px - floorf(px * ipdx) * pdx, zl = pz - floorf(pz * ipdz) * pdz;
-            cand = fabsf(xl - B.fc[0]) <= cull && fabsf(zl - B.fc[1]) <= cull && xl >= B.cb[0] + B.cb[1] * py &&
-                   xl <= B.cb[2] + B.cb[3] * py && zl >= B.cb[4] + B.cb[5] * py && zl <= B.cb[6] + B.cb[7] * py;
-            s_fp[j] = 0;
-        }
-        const uint64_t mask = __ballot(cand);
-        if (cand) s_list[ncand + __popcll(mask & lt)] = (short)j;
-        ncand += __popcll(mask);
-    }
-    if (ncand == 0) {
-        if (tid == 0) a.lines[line].len = 0;
-        __syncthreads();
-        continue;
-    }
-    __syncthreads();
-    // pass A.2: exact pillar mapping and fluence-cell test of the candidates, full waves
-    bool any = false;
-    uint32_t nfoot = 0;  // footprint samples of the line: exactly its TERMA requests below
-    for (int r = 0; r < ncand; r += 64) {
-        lds_reload_fence();
-        bool fp = false;
-        if (r + tid < ncand) {
-            const int j = s_list[r + tid];
-            int pidx;
-            v3 inp;
-            if (bl_locate(a, c, B, ipd, i0 + j, tY, tZ, pidx, inp) && fabsf(inp.x - B.fc[0]) <= B.fw &&
-                fabsf(inp.z - B.fc[1]) <= B.fw) {
-                // point_fluence(...) > 0 without its map load: a job beamlet's own cell has a
-                // positive weight (plan_beam keeps only those), so the cell test decides alone
-                const PillarRec bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
-                const v3 tp = bl_terma_point(a, B, bl, inp);
-                lds_reload_fence();
-                fp = fluence_cell(tp, B.beam) == bl.fidx;
-                if (fp) {
-                    s_fp[j] = 1;
-                    if (track) atomicOr(&s_pil[pidx >> 5], 1u << (pidx & 31));
+    uint64_t todo = __ballot(mine.len > 0);
+    while (todo) {
+        // pass A.1: affine cull of consecutive lines of one grid, candidates to s_cand
+        const int ci = lane_i(my_ci, __builtin_ctzll(todo));
+        const BlConeDev* pc = a.cones + ci;
+        const BatchDev* pB = a.batches + ci;  // grid ci of a direction belongs to batch ci
+        uint64_t lines_in = 0, with_cand = 0;
+        int my_c0 = 0, my_c1 = 0, ncand = 0;
+        {
+            const BlConeDev c = uniform_copy(pc);
+            const BatchDev B = uniform_copy(pB);
+            const v3 dl = mk3(c.kinv_m.m[1], c.kinv_m.m[4], c.kinv_m.m[7]);
+            const float pdx = (float)B.pd[0], pdz = (float)B.pd[2], ipdx = 1.f / pdx, ipdz = 1.f / pdz;
+            const float cull = B.fw + 0.05f;
+            // the distance from the nearest beamlet axis in pillars (0.05 samples wider than the cull)
+            const float dux = dl.x * ipdx, duz = dl.z * ipdz, cx = (cull + 0.05f) * ipdx, cz = (cull + 0.05f) * ipdz;
+            while (todo) {
+                const int k = __builtin_ctzll(todo);
+                const int m = lane_i((int)mine.len, k);
+                if (lane_i(my_ci, k) != ci || ncand + m > kMaxLine) break;
+                todo &= todo - 1ull;
+                lines_in |= 1ull << k;
+                const float px0 = lane_f(my_p0.x, k), py0 = lane_f(my_p0.y, k), pz0 = lane_f(my_p0.z, k);
+                const float t0 = (float)(lane_i((int)mine.i0, k) + tid);
+                const float ux0 = fmaf(px0 - B.fc[0], ipdx, 0.5f), uz0 = fmaf(pz0 - B.fc[1], ipdz, 0.5f);
+                const int c0 = ncand;
+                for (int j0 = 0; j0 < m; j0 += 64) {
+                    const float t = t0 + (float)j0;
+                    const float ux = fmaf(t, dux, ux0), uz = fmaf(t, duz, uz0);
+                    bool cand = tid < m - j0 && fabsf((ux - floorf(ux)) - 0.5f) <= cx &&
+                                fabsf((uz - floorf(uz)) - 0.5f) <= cz;
+                    if (!__ballot(cand)) continue;
+                    // the footprint half-width fw and the batch's depth-linear footprint bounds (cb)
+                    const float px = px0 + t * dl.x, pz = pz0 + t * dl.z, py = py0 + t * dl.y;
+                    const float xl = px - floorf(px * ipdx) * pdx, zl = pz - floorf(pz * ipdz) * pdz;
+                    cand = cand && fabsf(xl - B.fc[0]) <= cull && fabsf(zl - B.fc[1]) <= cull &&
+                           xl >= B.cb[0] + B.cb[1] * py && xl <= B.cb[2] + B.cb[3] * py &&
+                           zl >= B.cb[4] + B.cb[5] * py && zl <= B.cb[6] + B.cb[7] * py;
+                    const uint64_t mask = __ballot(cand);
+                    if (cand) s_cand[ncand + __popcll(mask & lt)] = (uint16_t)(k << 10 | (j0 + tid));
+                    ncand += __popcll(mask);
+                }
+                if (ncand > c0) {
+                    with_cand |= 1ull << k;
+                    if (tid == k) {
+                        my_c0 = c0;
+                        my_c1 = ncand;
+                    }
                 }
             }
         }
-        const uint64_t fm = __ballot(fp);
-        any = any || fm != 0ull;
-        nfoot += (uint32_t)__popcll(fm);
-    }
-    if (!any) {
-        if (tid == 0) a.lines[line].len = 0;
+        if ((lines_in & ~with_cand) >> tid & 1ull) a.lines[my_line].len = 0;
         __syncthreads();
-        continue;
-    }
-    // one reservation per line in the sub-queue (its latency overlaps pass B.1): every footprint
-    // sample, and no other, queues one TERMA request in pass B.2
-    uint32_t qres = 0;
-    if (tid == 0) qres = atomicAdd(qcnt + sq * kCntStride, nfoot);
-    __syncthreads();
-    // the beamlet data of the footprint pillars into LDS (its loads overlap pass B.1): word w of
-    // s_pil is lane w's (w < 64) or lane w-64's; a pillar's slot is its rank among the set bits
-    if (track) {
-        const uint32_t w0 = s_pil[tid], w1 = s_pil[tid + 64];
-        const uint32_t c0 = (uint32_t)__popc(w0), c1 = (uint32_t)__popc(w1);
-        uint32_t i0s = c0, i1s = c1;  // inclusive scans over the lanes
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u0 = __shfl_up(i0s, o, 64), u1 = __shfl_up(i1s, o, 64);
-            if (tid >= o) { i0s += u0; i1s += u1; }
-        }
-        const uint32_t tot0 = __shfl(i0s, 63, 64);
-        const uint32_t r0 = i0s - c0, r1 = tot0 + i1s - c1;
-        s_rank[tid] = (uint16_t)r0;
-        s_rank[tid + 64] = (uint16_t)r1;
-        uint32_t w = w0, slot = r0;
-        for (int h = 0; h < 2; h++) {
-            const int wbase = (h == 0 ? tid : tid + 64) * 32;
-            for (; w != 0u && slot < (uint32_t)kStagePillars; slot++) {
-                const int b = __ffs(w) - 1;
-                w &= w - 1u;
-                s_rec[slot] = pillar_rec(a.beamlets[B.beamlet0 + wbase + b]);
+        // pass A.2: exact pillar mapping and fluence-cell test of the candidates, full waves
+        if (ncand > 0) {
+            const BlConeDev c = uniform_copy(pc);
+            const BatchDev B = uniform_copy(pB);
+            const v3 ipd = mk3(1.f / (float)B.pd[0], 1.f / (float)B.pd[1], 1.f / (float)B.pd[2]);
+            for (int r = 0; r < ncand; r += 64) {
+                const bool in = r + tid < ncand;
+                const int e = in ? (int)s_cand[r + tid] : 0, k = e >> 10;
+                const int i = __shfl((int)mine.i0, k, 64) + (e & 1023), y = __shfl(my_y, k, 64), z = __shfl(my_z, k, 64);
+                if (in) {
+                    int pidx;
+                    v3 inp;
+                    bool fp = false;
+                    if (bl_locate(a, c, B, ipd, i, y, z, pidx, inp) && fabsf(inp.x - B.fc[0]) <= B.fw &&
+                        fabsf(inp.z - B.fc[1]) <= B.fw) {
+                        // point_fluence(...) > 0 without its map load: a job beamlet's own cell has a
+                        // positive weight (plan_beam keeps only those), so the cell test decides alone
+                        const PillarRec bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
+                        fp = fluence_cell(bl_terma_point(a, B, bl, inp), B.beam) == bl.fidx;
+                    }
+                    s_cpil[r + tid] = !fp ? kNoPil : (uint16_t)(B.n <= (int)kPillarBits ? pidx : 0);
+                }
             }
-            w = w1;
-            slot = r1;
         }
-    }
-    // pass B.1: a pillar without footprint samples on this line gets no dose on it, so its samples
-    // act as walls (a pillar crossing is exactly one segment of the walk).  Samples confidently
-    // in such pillars (or outside the grid's pillars) are walls; the others go to the exact list
-    // (and are marked with bit 1 of s_fp).  Only the walls between the first and the last listed
-    // sample are written: the line is trimmed to its non-wall span below, so no stage reads the
-    // others.
-    float* T = a.rev + meta.off;
-    float* Hl = H + meta.off;
-    int nex = 0;
-    for (int base = 0; base < m; base += 64) {
-        const int j = base + tid;
-        bool exact = false;
-        if (j < m) {
-            exact = true;
+        __syncthreads();
+        while (with_cand) {
+            const int k = __builtin_ctzll(with_cand);
+            with_cand &= with_cand - 1ull;
+            const uint64_t line = base + (uint64_t)k * G;
+            const int c0 = lane_i(my_c0, k), c1 = lane_i(my_c1, k);
+            uint32_t nfoot = 0;  // footprint samples of the line: exactly its TERMA requests below
+            for (int e = c0; e < c1; e += 64)
+                nfoot += (uint32_t)__popcll(__ballot(e + tid < c1 && s_cpil[e + tid] != kNoPil));
+            if (nfoot == 0) {
+                if (tid == 0) a.lines[line].len = 0;
+                continue;
+            }
+            // a line's TERMA requests go to one of kSubQueues queues, chosen by its run of 64
+            // consecutive lines: the Siddon stage then marches neighbouring lines' rays side by side
+            // (shared cache lines; -26 % stage time against one queue per wave), and the lines in
+            // flight still spread over every counter.  One reservation per line (its latency overlaps
+            // pass B.1): every footprint sample, and no other, queues one TERMA request in pass B.2
+            const uint32_t sq = (uint32_t)((line >> 6) % kSubQueues);
+            TermaReq* qs = q + (size_t)sq * subcap;
+            uint32_t qres = 0;
+            if (tid == 0) qres = atomicAdd(qcnt + sq * kCntStride, nfoot);
+            const BatchDev B = uniform_copy(pB);
+            const BlConeDev c = uniform_copy(pc);
+            const bool track = B.n <= (int)kPillarBits;
+            if (tid < kMaxLine / 32) s_foot[tid] = 0u;
+            s_pil[tid] = 0u;
+            s_pil[tid + 64] = 0u;
+            __syncthreads();
+            for (int e = c0 + tid; e < c1; e += 64) {
+                const uint32_t pil = s_cpil[e], j = s_cand[e] & 1023u;
+                if (pil == kNoPil) continue;
+                atomicOr(&s_foot[j >> 5], 1u << (j & 31u));
+                if (track) atomicOr(&s_pil[pil >> 5], 1u << (pil & 31u));
+            }
+            __syncthreads();
+            // the beamlet data of the footprint pillars into LDS (its loads overlap pass B.1): word w of
+            // s_pil is lane w's (w < 64) or lane w-64's; a pillar's slot is its rank among the set bits
             if (track) {
-                const float t = (float)(i0 + j);
-                const float px = p0.x + t * dl.x, pz = p0.z + t * dl.z;
-                const float fx = floorf(px * ipdx), fz = floorf(pz * ipdz);
-                const float xl = px - fx * pdx, zl = pz - fz * pdz;
-                if (xl > 0.05f && xl < pdx - 0.05f && zl > 0.05f && zl < pdz - 0.05f) {
-                    const int pa = (int)fx + (int)fz * B.npx;
-                    exact = !(fx < 0.f || fz < 0.f || (int)fx >= B.npx || pa >= B.n ||
-                              !((s_pil[pa >> 5] >> (pa & 31)) & 1u));
+                uint32_t slot = 0;
+                for (int h = 0; h < 2; h++) {
+                    uint32_t w = s_pil[tid + 64 * h];
+                    uint32_t first = 0;
+                    for (uint64_t nz = __ballot(w != 0u); nz; nz &= nz - 1ull) {
+                        const int l = __builtin_ctzll(nz);
+                        if (tid == l) first = slot;
+                        slot += (uint32_t)__builtin_popcount((uint32_t)lane_i((int)w, l));
+                    }
+                    if (w) s_rank[tid + 64 * h] = (uint16_t)first;
+                    for (; w != 0u && first < (uint32_t)kStagePillars; first++) {
+                        const int b = __ffs(w) - 1;
+                        w &= w - 1u;
+                        s_rec[first] = pillar_rec(a.beamlets[B.beamlet0 + (tid + 64 * h) * 32 + b]);
+                    }
                 }
             }
-            if (exact) s_fp[j] |= 2;
-        }
-        const uint64_t mask = __ballot(exact);
-        if (exact) s_list[nex + __popcll(mask & lt)] = (short)j;
-        nex += __popcll(mask);
-    }
-    const uint32_t qbase = __shfl(qres, 0, 64);
-    if (nex == 0) {  // every sample is a wall: no dose on this line, and the reservation stays empty
-        if (tid == 0) a.lines[line].len = 0;
-        for (uint32_t k = (uint32_t)tid; k < nfoot; k += 64)
-            if (qbase + k < subcap) qs[qbase + k].slot = kNoSlot;
-        __syncthreads();
-        continue;
-    }
-    __syncthreads();
-    {
-        const int elo = s_list[0], ehi = s_list[nex - 1];
-        for (int j = elo + tid; j <= ehi; j += 64)
-            if (!(s_fp[j] & 2)) {
-                Hl[j] = -1.f;
-                T[j] = 0.f;
+            // pass B.1: a pillar without footprint samples on this line gets no dose on it, so its
+            // samples act as walls (a pillar crossing is exactly one segment of the walk).  Samples
+            // confidently in such pillars (or outside the grid's pillars) are walls; the others go to
+            // the list.  Only the walls between the first and the last listed sample are written: the
+            // line is trimmed to its non-wall span below, so no stage reads the others.
+            const int i0 = lane_i((int)mine.i0, k), m = lane_i((int)mine.len, k);
+            const uint32_t moff = (uint32_t)lane_i((int)mine.off, k);
+            float* T = a.rev + moff;
+            float* Hl = H + moff;
+            int nex = 0;
+            {
+                const float ipdx = 1.f / (float)B.pd[0], ipdz = 1.f / (float)B.pd[2];
+                const float ux0 = lane_f(my_p0.x, k) * ipdx, uz0 = lane_f(my_p0.z, k) * ipdz;
+                const float dux = c.kinv_m.m[1] * ipdx, duz = c.kinv_m.m[7] * ipdz;
+                // (inside the pillar by 0.05 samples on each side)
+                const float hx = 0.5f - 0.05f * ipdx, hz = 0.5f - 0.05f * ipdz;
+                for (int j0 = 0; j0 < m; j0 += 64) {
+                    const int j = j0 + tid;
+                    bool exact = j < m;
+                    if (track) {
+                        const float t = (float)(i0 + j);
+                        const float ux = fmaf(t, dux, ux0), uz = fmaf(t, duz, uz0);
+                        const float fx = floorf(ux), fz = floorf(uz);
+                        if (fabsf((ux - fx) - 0.5f) < hx && fabsf((uz - fz) - 0.5f) < hz) {
+                            const int px = (int)fx, pa = px + (int)fz * B.npx;
+                            const bool grid = (uint32_t)px < (uint32_t)B.npx && fz >= 0.f && pa < B.n;
+                            exact = exact && grid && (s_pil[grid ? pa >> 5 : 0] >> (pa & 31)) & 1u;
+                        }
+                    }
+                    const uint64_t mask = __ballot(exact);
+                    if (tid == 0) s_exact[j0 >> 6] = mask;
+                    if (exact) s_list[nex + __popcll(mask & lt)] = (uint16_t)j;
+                    nex += __popcll(mask);
+                }
             }
-    }
-    // pass B.2: exact mapping, density and TERMA request of the listed samples, full waves
-    int nlo = m, nhi = -1;  // first and last sample that is not a wall
-    uint32_t qdone = 0;
-    for (int r = 0; r < nex; r += 64) {
-        lds_reload_fence();
-        bool ok = false, need = false;
-        int j = 0, pidx = 0;
-        v3 inp;
-        PillarRec bl;
-        if (r + tid < nex) {
-            j = s_list[r + tid];
-            if (bl_locate(a, c, B, ipd, i0 + j, tY, tZ, pidx, inp) &&
-                (!track || ((s_pil[pidx >> 5] >> (pidx & 31)) & 1u))) {
-                ok = true;
-                const uint32_t slot = track ? (uint32_t)s_rank[pidx >> 5] +
-                                                  (uint32_t)__popc(s_pil[pidx >> 5] & ((1u << (pidx & 31)) - 1u))
-                                            : (uint32_t)kStagePillars;
-                if (slot < (uint32_t)kStagePillars) bl = s_rec[slot];
-                else bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
-                need = (s_fp[j] & 1) != 0;
+            const uint32_t qbase = (uint32_t)lane_i((int)qres, 0);
+            if (nex == 0) {  // every sample is a wall: no dose on this line, and the reservation stays empty
+                if (tid == 0) a.lines[line].len = 0;
+                for (uint32_t e = (uint32_t)tid; e < nfoot; e += 64)
+                    if (qbase + e < subcap) qs[qbase + e].slot = kNoSlot;
+                __syncthreads();
+                continue;
             }
-        }
-        // the TERMA requests first, then the density: the two rotations are not live together
-        const uint64_t mask = __ballot(need);
-        if (mask) {
-            if (need) {
-                const uint32_t pos = qbase + qdone + (uint32_t)__popcll(mask & lt);
-                const v3 gcs = bl_terma_point(a, B, bl, inp);
-                TermaReq rq;
-                rq.slot = (uint32_t)(meta.off + j);
-                rq.beamlet = (uint32_t)(B.beamlet0 + pidx);
-                rq.x = gcs.x; rq.y = gcs.y; rq.z = gcs.z;
-                if (pos < subcap) qs[pos] = rq;
+            __syncthreads();
+            {
+                const int elo = s_list[0], ehi = s_list[nex - 1];
+                for (int j0 = elo & ~63; j0 <= ehi; j0 += 64) {
+                    const int j = j0 + tid;
+                    if (j > elo && j < ehi && !(s_exact[j0 >> 6] >> tid & 1ull)) {
+                        Hl[j] = -1.f;
+                        T[j] = 0.f;
+                    }
+                }
             }
-            qdone += (uint32_t)__popcll(mask);
-        }
-        if (r + tid < nex) {
-            const float h = ok ? 0.5f * (a.delr * bl_density(a, B, bl, inp)) : -1.f;
-            Hl[j] = h;
-            T[j] = 0.f;
-            if (h >= 0.f) {
-                nlo = min(nlo, j);
-                nhi = max(nhi, j);
+            // pass B.2: exact mapping, density and TERMA request of the listed samples, full waves
+            int first = -1, last = -1;  // first and last listed sample that is not a wall
+            uint32_t qdone = 0;
+            const int tY = lane_i(my_y, k), tZ = lane_i(my_z, k);
+            const v3 ipd = mk3(1.f / (float)B.pd[0], 1.f / (float)B.pd[1], 1.f / (float)B.pd[2]);
+            for (int r = 0; r < nex; r += 64) {
+                bool ok = false, need = false;
+                int j = 0, pidx = 0;
+                v3 inp;
+                PillarRec bl;
+                if (r + tid < nex) {
+                    j = s_list[r + tid];
+                    if (bl_locate(a, c, B, ipd, i0 + j, tY, tZ, pidx, inp) &&
+                        (!track || ((s_pil[pidx >> 5] >> (pidx & 31)) & 1u))) {
+                        ok = true;
+                        const uint32_t slot = track ? (uint32_t)s_rank[pidx >> 5] +
+                                                          (uint32_t)__popc(s_pil[pidx >> 5] & ((1u << (pidx & 31)) - 1u))
+                                                    : (uint32_t)kStagePillars;
+                        if (slot < (uint32_t)kStagePillars) bl = s_rec[slot];
+                        else bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
+                        need = (s_foot[j >> 5] >> (j & 31)) & 1u;
+                    }
+                }
+                // the TERMA requests first, then the density: the two rotations are not live together
+                const uint64_t mask = __ballot(need);
+                if (mask) {
+                    if (need) {
+                        const uint32_t pos = qbase + qdone + (uint32_t)__popcll(mask & lt);
+                        const v3 gcs = bl_terma_point(a, B, bl, inp);
+                        TermaReq rq;
+                        rq.slot = moff + (uint32_t)j;
+                        rq.beamlet = (uint32_t)(B.beamlet0 + pidx);
+                        rq.x = gcs.x; rq.y = gcs.y; rq.z = gcs.z;
+                        if (pos < subcap) qs[pos] = rq;
+                    }
+                    qdone += (uint32_t)__popcll(mask);
+                }
+                float h = -1.f;
+                if (r + tid < nex) {
+                    if (ok) h = 0.5f * (a.delr * bl_density(a, vol, B, bl, inp));
+                    Hl[j] = h;
+                    T[j] = 0.f;
+                }
+                const uint64_t open = __ballot(h >= 0.f);
+                if (open) {
+                    if (first < 0) first = r + __builtin_ctzll(open);
+                    last = r + 63 - __builtin_clzll(open);
+                }
             }
+            // The reservation counted footprint samples of pass A.2; pass B.2 requests TERMA for those of
+            // them it maps to the same pillar again, so any shortfall is closed with empty entries.
+            for (uint32_t e = qdone + (uint32_t)tid; e < nfoot; e += 64) {
+                const uint32_t pos = qbase + e;
+                if (pos < subcap) qs[pos].slot = kNoSlot;
+            }
+            // Walls before the first and after the last non-wall sample bound no segment and receive no
+            // dose: the line's stored interval shrinks to the span between, so the walk and the gather
+            // skip them (the gather reads samples outside a line's interval as zero, the dose the walk
+            // gives a wall).
+            const int nlo = first < 0 ? m : (int)s_list[first], nhi = last < 0 ? -1 : (int)s_list[last];
+            if (tid == 0 && (nlo > 0 || nhi < m - 1)) {
+                LineMeta t;
+                t.off = nhi < nlo ? moff : moff + (uint32_t)nlo;
+                t.i0 = nhi < nlo ? (int16_t)i0 : (int16_t)(i0 + nlo);
+                t.len = nhi < nlo ? (int16_t)0 : (int16_t)(nhi - nlo + 1);
+                a.lines[line] = t;
+            }
+            __syncthreads();  // the next line reuses the LDS arrays
         }
+        __syncthreads();  // the next lines reuse the candidate list
     }
-    // The reservation counted footprint samples of pass A.2; pass B.2 requests TERMA for those of
-    // them it maps to the same pillar again, so any shortfall is closed with empty entries.
-    for (uint32_t k = qdone + (uint32_t)tid; k < nfoot; k += 64) {
-        const uint32_t pos = qbase + k;
-        if (pos < subcap) qs[pos].slot = kNoSlot;
-    }
-    // Walls before the first and after the last non-wall sample bound no segment and receive no
-    // dose: the line's stored interval shrinks to [nlo, nhi], so the walk and the gather skip them
-    // (the gather reads samples outside a line's interval as zero, the dose the walk gives a wall).
-    for (int o = 32; o > 0; o >>= 1) {
-        nlo = min(nlo, __shfl_xor(nlo, o, 64));
-        nhi = max(nhi, __shfl_xor(nhi, o, 64));
-    }
-    if (tid == 0 && (nlo > 0 || nhi < m - 1)) {
-        LineMeta t;
-        t.off = nhi < nlo ? meta.off : meta.off + (uint32_t)nlo;
-        t.i0 = nhi < nlo ? meta.i0 : (int16_t)(i0 + nlo);
-        t.len = nhi < nlo ? (int16_t)0 : (int16_t)(nhi - nlo + 1);
-        a.lines[line] = t;
-    }
-    __syncthreads();  // the next line reuses the LDS arrays
     }
     if (a.counts) wave_count(stored, a.counts, blockIdx.x);
 }
@@ -550,7 +604,6 @@ __global__ void __launch_bounds__(256) bl_siddon_kernel(BlArgs a, const TermaReq
     const uint32_t sq = blockIdx.x % kSubQueues, per = gridDim.x / kSubQueues;
     const uint32_t n = min(qcnt[sq * kCntStride], subcap);
     const TermaReq* qs = q + (size_t)sq * subcap;
-    const v3 ivox = mk3(1.f / a.vd.voxel.x, 1.f / a.vd.voxel.y, 1.f / a.vd.voxel.z);
     uint32_t steps = 0;
     for (uint32_t i = (blockIdx.x / kSubQueues) * 256 + threadIdx.x; i < n; i += per * 256) {
         const TermaReq r = qs[i];
@@ -558,7 +611,7 @@ __global__ void __launch_bounds__(256) bl_siddon_kernel(BlArgs a, const TermaReq
         const BeamletDev& bl = a.beamlets[r.beamlet];
         const BatchDev& B = a.batches[bl.batch];
         int it = 0;
-        a.rev[r.slot] = point_terma_rpl(mk3(r.x, r.y, r.z), B.fmap, B.beam, a.spec, a.vd, ivox, a.dens, a.bhc, bl.fidx,
+        a.rev[r.slot] = point_terma_rpl(mk3(r.x, r.y, r.z), B.fmap, B.beam, a.spec, a.vd, a.ivoxel, a.dens, a.bhc, bl.fidx,
                                         &it);
         steps += (uint32_t)it;
     }
@@ -827,7 +880,7 @@ struct UnpackArgs {
     float* arena;
     int nbeamlets;
     uint64_t narena;
-    v3 start, voxel, rvs;
+    v3 start, voxel, rvs, rrv;  // (rrv: 1 / rvs)
     int bbs[3];   // calc_bbox start
 };
 
@@ -852,7 +905,7 @@ __global__ void __launch_bounds__(256) bl_unpack_kernel(UnpackArgs a) {
     const v3 gc = mk3(((float)tX + (float)a.bbs[0]) * a.voxel.x + a.start.x,
                       ((float)tY + (float)a.bbs[1]) * a.voxel.y + a.start.y,
                       ((float)tZ + (float)a.bbs[2]) * a.voxel.z + a.start.z);
-    v3 pidx = rot1(bl.fwd, rot2(B.beam.beam_fwd, gc - bl.pst)) / a.rvs + 0.5f;
+    v3 pidx = div_by(rot1(bl.fwd, rot_fwd(B.beam.beam_fwd, gc - bl.pst)), a.rvs, a.rrv) + 0.5f;
     float v = 0.f;
     const float lo_f = (float)(kWall + kBuffer);
     if (!(pidx.x < lo_f || pidx.y < lo_f || pidx.z < lo_f || pidx.x >= (float)(B.pd[0] - kBuffer) ||
@@ -876,7 +929,7 @@ struct ColArgs {
     const BatchDev* batches;
     const BeamletDev* beamlets;
     const float* pdose;
-    v3 start, voxel, rvs;
+    v3 start, voxel, rvs, rrv;  // (rrv: 1 / rvs)
     int bbs[3];        // calc_bbox start
     int nx, ny;        // full volume dims (keys)
     float thresh;
@@ -893,7 +946,7 @@ __device__ __forceinline__ float pillar_value(const ColArgs& a, const BeamletDev
     const v3 gc = mk3(((float)tX + (float)a.bbs[0]) * a.voxel.x + a.start.x,
                       ((float)tY + (float)a.bbs[1]) * a.voxel.y + a.start.y,
                       ((float)tZ + (float)a.bbs[2]) * a.voxel.z + a.start.z);
-    v3 pidx = rot1(bl.fwd, rot2(B.beam.beam_fwd, gc - bl.pst)) / a.rvs + 0.5f;
+    v3 pidx = div_by(rot1(bl.fwd, rot_fwd(B.beam.beam_fwd, gc - bl.pst)), a.rvs, a.rrv) + 0.5f;
     const float lo_f = (float)(kWall + kBuffer);
     if (pidx.x < lo_f || pidx.y < lo_f || pidx.z < lo_f || pidx.x >= (float)(B.pd[0] - kBuffer) ||
         pidx.y >= (float)(B.pd[1] - kBuffer) || pidx.z >= (float)(B.pd[2] - kBuffer))
@@ -1092,7 +1145,7 @@ __global__ void __launch_bounds__(256) plain_ray_kernel(BlArgs a, float* __restr
     if (bl_locate(a, c, B, ipd, tX, tY, tZ, pidx, inp)) {
         const PillarRec bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
         t = point_terma(bl_terma_point(a, B, bl, inp), B.fmap, B.beam, a.spec, a.vd, a.dens, a.bhc, bl.fidx, nullptr);
-        d = bl_density(a, B, bl, inp);
+        d = bl_density(a, march_vol(a.dens, a.vd.nx, a.vd.ny, a.vd.nz), B, bl, inp);
     }
     dens[i] = d;
     terma[i] = t;
@@ -1566,6 +1619,7 @@ BlArgs base_args(cccs_ctx* ctx) {
     a.rvs = mk3(p.rev_latspacing, p.rev_longspacing, p.rev_latspacing);
     a.rrv = mk3(1.f / a.rvs.x, 1.f / a.rvs.y, 1.f / a.rvs.z);
     a.vd = ctx->vol;
+    a.ivoxel = mk3(1.f / a.vd.voxel.x, 1.f / a.vd.voxel.y, 1.f / a.vd.voxel.z);
     a.spec = ctx->spec;
     a.bhc = p.beamhard_correct;
     return a;
@@ -1777,6 +1831,7 @@ int run_job_unpack(cccs_ctx* ctx, const Job& J) {
     u.start = ld3(p.start);
     u.voxel = ld3(p.voxel);
     u.rvs = mk3(p.rev_latspacing, p.rev_longspacing, p.rev_latspacing);
+    u.rrv = mk3(1.f / u.rvs.x, 1.f / u.rvs.y, 1.f / u.rvs.z);
     for (int k = 0; k < 3; k++) u.bbs[k] = (int)p.bbox_start[k];
     if (J.arena == 0) return CCCS_OK;
     const uint64_t blocks = (J.arena + 255) / 256;
@@ -1928,6 +1983,7 @@ int run_plain_batch(cccs_ctx* ctx, const std::vector<BeamPlan>& plans, const Bat
     u.start = ld3(p.start);
     u.voxel = ld3(p.voxel);
     u.rvs = a.rvs;
+    u.rrv = a.rrv;
     for (int k = 0; k < 3; k++) u.bbs[k] = (int)p.bbox_start[k];
     for (int g0 = 0; g0 < nbl; g0 += G) {
         const int set = (g0 / G) % 2;
@@ -2412,6 +2468,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         ca.start = ld3(p.start);
         ca.voxel = ld3(p.voxel);
         ca.rvs = mk3(p.rev_latspacing, p.rev_longspacing, p.rev_latspacing);
+        ca.rrv = mk3(1.f / ca.rvs.x, 1.f / ca.rvs.y, 1.f / ca.rvs.z);
         for (int k = 0; k < 3; k++) ca.bbs[k] = (int)p.bbox_start[k];
         ca.nx = (int)p.size[0];
         ca.ny = (int)p.size[1];

@@ -65,6 +65,35 @@ CCCS_HD v3 rodrigues(v3 p, v3 r, float s, float c) {
                (-r.z * (-r.x * p.x - r.y * p.y - r.z * p.z)) * (1 - c) + p.z * c + (-r.y * p.x + r.x * p.y) * s);
 }
 CCCS_HD v3 rot2(const Rot2& R, v3 p) { return rodrigues(rodrigues(p, R.a1, R.s1, R.c1), R.a2, R.s2, R.c2); }
+
+// The same rotations about the axes that the builders below use: one of the two is +y, the other lies
+// in the x-z plane.  The terms of rodrigues() that those axes make zero are left out and the others
+// keep their order, so the results are equal for finite coordinates (a zero may differ in sign): 34
+// operations a Rot2 against 74, in kernels that are bound by their instruction count.
+CCCS_HD v3 rot_y(v3 p, float s, float c) {
+    return mk3(p.x * c + p.z * s, p.y * (1.f - c) + p.y * c, p.z * c - p.x * s);
+}
+CCCS_HD v3 rot_xz(v3 p, float rx, float rz, float s, float c) {
+    const float d = rx * p.x + rz * p.z, u = 1.f - c;
+    return mk3((rx * d) * u + p.x * c - (rz * p.y) * s, p.y * c + (rz * p.x - rx * p.z) * s,
+               (rz * d) * u + p.z * c + (rx * p.y) * s);
+}
+// rot2 of rot2_beam_fwd / rot2_kernel_fwd, and of rot2_beam_inv / rot2_kernel_inv
+CCCS_HD v3 rot_fwd(const Rot2& R, v3 p) { return rot_y(rot_xz(p, R.a1.x, R.a1.z, R.s1, R.c1), R.s2, R.c2); }
+CCCS_HD v3 rot_inv(const Rot2& R, v3 p) { return rot_xz(rot_y(p, R.s1, R.c1), R.a2.x, R.a2.z, R.s2, R.c2); }
+
+// x / y, correctly rounded, from iy = 1 / y correctly rounded: the first correction makes the quotient
+// faithful, and by Markstein's theorem a second one with an exact remainder then rounds it correctly
+// (P. Markstein, IBM J. Res. Dev. 34, 1990).  For quotients between 2^-100 and 2^100 and zero; smaller
+// ones may be off in their last bits, larger ones become NaN instead of infinity.  5 operations
+// against the 12 of a division.
+CCCS_HD float div_by(float x, float y, float iy) {
+    float q = x * iy;
+    q = fmaf(fmaf(-y, q, x), iy, q);
+    return fmaf(fmaf(-y, q, x), iy, q);
+}
+CCCS_HD v3 div_by(v3 x, v3 y, v3 iy) { return mk3(div_by(x.x, y.x, iy.x), div_by(x.y, y.y, iy.y), div_by(x.z, y.z, iy.z)); }
+
 // host builders (CudaUtilities/geometry.cu:69-75, 85-92, 126-131, 140-145)
 Rot2 rot2_beam_fwd(float theta, float phi, float coll);
 Rot2 rot2_beam_inv(float theta, float phi, float coll);
@@ -355,7 +384,9 @@ CCCS_HD int fluence_cell(v3 p, const BeamDev& b) {
     v3 projection = dot3(diff, b.dir_n) * b.dir_n;
     v3 rejection = diff - projection;
     float trad = len3(rejection) * fabsf(b.iso_dist / len3(projection));
-    v3 pf = rot2(b.beam_fwd, trad * norm3(rejection));
+    const v3 pr = trad * norm3(rejection);
+    // (a point level with the source has no finite radius: rot2 decides its NaN coordinates)
+    v3 pf = trad < 1e30f ? rot_fwd(b.beam_fwd, pr) : rot2(b.beam_fwd, pr);
     float fx = (pf.x / b.bsx) + ((float)b.fmx * 0.5f);
     float fz = (pf.z / b.bsy) + ((float)b.fmy * 0.5f);
     // a NaN coordinate (voxel on the central axis) passes these tests, as in the reference

@@ -52,6 +52,14 @@ __device__ __forceinline__ void block_count(uint32_t v, uint32_t* __restrict__ p
     if (t == 0) part[slot] = s_cnt[0];
 }
 
+// Read-only data at wave-uniform addresses, loaded through the scalar unit.
+template <class T>
+using uniform_ptr = const __attribute__((address_space(4))) T*;
+template <class T>
+__device__ __forceinline__ uniform_ptr<T> as_uniform(const T* p) {
+    return (uniform_ptr<T>)p;
+}
+
 // One REV line of a cone grid in the compact store: samples [i0, i0 + len) of the line are kept at
 // rev[off ...]; every other sample of the line is zero.
 struct LineMeta {
