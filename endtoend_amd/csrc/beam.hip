@@ -1000,25 +1000,124 @@ struct ProjBeam {
     uint32_t off;     // first beamlet of this beam in the output
 };
 
-// One lane per beamlet of any beam.  Nine sub-rays (offsets -1/0/+1 half beamlets along each
-// fluence axis) run from the source to three times the source-to-cell distance through the
-// trilinearly sampled mask with the TERMA path's Siddon march; the beamlet is 1 when any sub-ray
-// accumulates a positive path integral.
-__global__ void __launch_bounds__(64) projection_kernel(const float* __restrict__ mask, VolDesc vd,
-                                                        const ProjBeam* __restrict__ beams, int nbeams, uint32_t total,
-                                                        float* __restrict__ out) {
-    const uint32_t t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= total) return;
-    int lo = 0, hi = nbeams - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (beams[mid].off <= t) lo = mid; else hi = mid - 1;
+// Mask bytes to floats, and the index box {lo xyz, hi xyz} of the non-zero voxels (initialised by the
+// caller to {INT_MAX, -1}).  Four voxels per thread and step.
+__global__ void __launch_bounds__(256) mask_to_float_kernel(const uint8_t* __restrict__ m, float* __restrict__ f, size_t n,
+                                                            int nx, int ny, int* __restrict__ box) {
+    int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {-1, -1, -1};
+    const size_t n4 = (n + 3) / 4;
+    for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < n4; q += (size_t)gridDim.x * 256) {
+        uint32_t w = 0;
+        if (4 * q + 4 <= n) {
+            w = reinterpret_cast<const uint32_t*>(m)[q];
+            reinterpret_cast<float4*>(f)[q] =
+                make_float4((float)(w & 255u), (float)(w >> 8 & 255u), (float)(w >> 16 & 255u), (float)(w >> 24));
+        } else {
+            for (size_t i = 4 * q; i < n; i++) {
+                f[i] = (float)m[i];
+                w |= (uint32_t)m[i] << (8 * (i - 4 * q));
+            }
+        }
+        for (int e = 0; w != 0u; e++, w >>= 8) {
+            if (!(w & 255u)) continue;
+            const size_t i = 4 * q + (size_t)e, row = i / (size_t)nx;
+            const int c[3] = {(int)(i - row * (size_t)nx), (int)(row % (size_t)ny), (int)(row / (size_t)ny)};
+            for (int k = 0; k < 3; k++) {
+                lo[k] = min(lo[k], c[k]);
+                hi[k] = max(hi[k], c[k]);
+            }
+        }
     }
-    const ProjBeam& b = beams[lo];
-    const int pix = (int)(t - b.off);
-    const int rx = pix % b.fx, rz = pix / b.fx;
-    bool hit = false;
-    for (int sr = 0; sr < 9 && !hit; sr++) {
+    for (int k = 0; k < 3; k++) {
+        for (int o = 32; o > 0; o >>= 1) {
+            lo[k] = min(lo[k], __shfl_xor(lo[k], o, 64));
+            hi[k] = max(hi[k], __shfl_xor(hi[k], o, 64));
+        }
+        if ((threadIdx.x & 63) == 0 && hi[k] >= 0) {
+            atomicMin(box + k, lo[k]);
+            atomicMax(box + 3 + k, hi[k]);
+        }
+    }
+}
+
+// True if the path integral of a ray over the mask is positive: siddon_march's segments (its planes in
+// its order), ended at the first segment with a positive contribution.  The mask is not negative and
+// neither is its interpolation, so the sum of the segments can only grow.  A segment's taps can be
+// non-zero only if its midpoint lies within half a voxel cell of the mask's box; the midpoint
+// parameters for which it does form one interval [t0, t1] (widened far beyond the rounding of the
+// coordinates), so the others cost no fetch, and the march ends behind the interval.
+__device__ __forceinline__ bool mask_ray_hit(v3 sink, const VolDesc& vd, v3 ivoxel, v3 src, const float* __restrict__ mask,
+                                             const int* __restrict__ box) {
+    const v3 diff = sink - src, startdiff = vd.start - src, enddiff = vd.end - src;
+    const float ax0 = (startdiff.x - 0.5f * vd.voxel.x) / diff.x, ax1 = (enddiff.x + 0.5f * vd.voxel.x) / diff.x;
+    const float ay0 = (startdiff.y - 0.5f * vd.voxel.y) / diff.y, ay1 = (enddiff.y + 0.5f * vd.voxel.y) / diff.y;
+    const float az0 = (startdiff.z - 0.5f * vd.voxel.z) / diff.z, az1 = (enddiff.z + 0.5f * vd.voxel.z) / diff.z;
+    const float a_min = fmaxf(0.f, fmaxf(fmaxf(fminf(ax0, ax1), fminf(ay0, ay1)), fminf(az0, az1)));
+    const float a_max = fminf(1.f, fminf(fminf(fmaxf(ax0, ax1), fmaxf(ay0, ay1)), fmaxf(az0, az1)));
+    if (a_min >= a_max) return false;
+    float t0 = 0.f, t1 = 1.f;
+    const v3 o = (src - vd.start) * ivoxel, dd = diff * ivoxel;
+    const float oc[3] = {o.x, o.y, o.z}, dc[3] = {dd.x, dd.y, dd.z};
+    for (int k = 0; k < 3; k++) {
+        const float m = 0.05f + 4e-6f * (fabsf(oc[k]) + fabsf(dc[k]));
+        const float ta = ((float)box[k] - 0.5f - m - oc[k]) / dc[k], tb = ((float)box[3 + k] + 1.5f + m - oc[k]) / dc[k];
+        t0 = fmaxf(t0, fminf(ta, tb));
+        t1 = fminf(t1, fmaxf(ta, tb));
+    }
+    if (t0 > t1) return false;
+    const float d12 = len3(diff);
+    const float step_x = fabsf(vd.voxel.x / diff.x), step_y = fabsf(vd.voxel.y / diff.y), step_z = fabsf(vd.voxel.z / diff.z);
+    float alpha = a_min, ax = a_min, ay = a_min, az = a_min;
+    int iter = 0;
+    while (alpha < a_max && !(alpha > t1) && ++iter < 5000) {
+        // (the planes of one step: siddon_rpl)
+        const float m0 = fminf(fminf(ax, ay), az);
+        if (!(m0 < 1.0f)) break;
+        if (ax == m0) ax += step_x;
+        const float m1 = fminf(fminf(ax, ay), az);
+        const bool ty = ay == m1 && m1 < 1.0f;
+        if (ty) ay += step_y;
+        const float m2 = fminf(fminf(ax, ay), az);
+        const bool tz = az == m2 && m2 < 1.0f;
+        if (tz) az += step_z;
+        const float nextalpha = tz ? m2 : (ty ? m1 : m0);
+        const float inter = fabsf(d12 * (nextalpha - alpha));
+        const float am = (nextalpha + alpha) * 0.5f;
+        if (inter >= 0.001f && am >= t0 && am <= t1) {
+            const v3 f = div_by(mk3(src.x + am * diff.x - vd.start.x, src.y + am * diff.y - vd.start.y,
+                                    src.z + am * diff.z - vd.start.z), vd.voxel, ivoxel);
+            if (inter * tex3_border(mask, vd.nx, vd.ny, vd.nz, f.x, f.y, f.z) > 0.f) return true;
+        }
+        alpha = nextalpha;
+    }
+    return false;
+}
+
+// Nine sub-rays per beamlet of any beam (offsets -1/0/+1 half beamlets along each fluence axis) run
+// from the source to three times the source-to-cell distance through the trilinearly sampled mask with
+// the TERMA path's Siddon planes; the beamlet is 1 when any sub-ray accumulates a positive path
+// integral.  A workgroup takes 64 beamlets, each of its nine waves one sub-ray of them: with one lane
+// per beamlet the rays ran one after another and a 64-beam set filled one wave per SIMD.  With the
+// fetches and the march held to the mask's box: 5270 -> 145 us (64 beams of 40x40 beamlets, 200x200x160
+// mask).  What is left is the planes of the rays up to the box, a serial chain.
+constexpr int kSubRays = 9;
+__global__ void __launch_bounds__(64 * kSubRays) projection_kernel(const float* __restrict__ mask, VolDesc vd, v3 ivoxel,
+                                                        const int* __restrict__ box, const ProjBeam* __restrict__ beams,
+                                                        int nbeams, uint32_t total, float* __restrict__ out) {
+    __shared__ uint32_t s_hit[64];
+    const int lane = threadIdx.x & 63, sr = threadIdx.x >> 6;
+    const uint32_t t = blockIdx.x * 64 + lane;
+    if (sr == 0) s_hit[lane] = 0u;
+    __syncthreads();
+    if (t < total && box[3] >= 0) {
+        int lo = 0, hi = nbeams - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (beams[mid].off <= t) lo = mid; else hi = mid - 1;
+        }
+        const ProjBeam& b = beams[lo];
+        const int pix = (int)(t - b.off);
+        const int rx = pix % b.fx, rz = pix / b.fx;
         const int sx = sr % 3 - 1, sz = sr / 3 - 1;
         const v3 fcs = mk3(b.bsx * ((float)rx + 0.5f * (float)sx - (float)b.fx * 0.5f + 0.5f), 0.f,
                            b.bsy * ((float)rz + 0.5f * (float)sz - (float)b.fy * 0.5f + 0.5f));
@@ -1026,11 +1125,10 @@ __global__ void __launch_bounds__(64) projection_kernel(const float* __restrict_
         ctr = ctr + 1e-9f;
         const v3 sd = ctr - b.src;
         const v3 sink = b.src + 3.f * sd;
-        const float rpl = siddon_march(sink, vd.start, vd.end, vd.voxel, b.src, mask, vd.nx, vd.ny, vd.nz,
-                                       [](float, float, float, float) {}, nullptr);
-        hit = rpl > 0.f;
+        if (mask_ray_hit(sink, vd, ivoxel, b.src, mask, box)) s_hit[lane] = 1u;
     }
-    out[t] = hit ? 1.f : 0.f;
+    __syncthreads();
+    if (sr == 0 && t < total) out[t] = s_hit[lane] ? 1.f : 0.f;
 }
 
 // ---- fluence-map convolution (the FCBB lateral step; no reference source) --------------------
@@ -1068,11 +1166,6 @@ __global__ void __launch_bounds__(256) fluence_conv_kernel(const float* __restri
     for (int j = 0; j < kh; j++)
         for (int i = 0; i < kw; i++) acc += s_k[j * kw + i] * s_f[(bv + j) * sw + bu + i];
     out[(size_t)map * w * h + (size_t)y * w + x] = acc;
-}
-
-__global__ void mask_to_float_kernel(const uint8_t* __restrict__ m, float* __restrict__ f, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        f[i] = (float)m[i];
 }
 
 __global__ void add_kernel(float* __restrict__ dst, const float* __restrict__ src, size_t n) {
@@ -1924,17 +2017,25 @@ extern "C" int cccs_fluence_projection(cccs_ctx* ctx, const uint8_t* mask, const
     } release{{&mb, &mf, &tb, &ob}};
     CCCS_TRY(mb.ensure(nv));
     CCCS_TRY(mf.ensure(nv * sizeof(float)));
-    CCCS_TRY(tb.ensure(sizeof(ProjBeam) * pb.size()));
+    // beam table, then the mask's index box
+    const size_t box_at = (sizeof(ProjBeam) * pb.size() + 15) & ~size_t(15);
+    std::vector<uint8_t> tab(box_at + 6 * sizeof(int), 0);
+    std::memcpy(tab.data(), pb.data(), sizeof(ProjBeam) * pb.size());
+    const int box0[6] = {INT32_MAX, INT32_MAX, INT32_MAX, -1, -1, -1};
+    std::memcpy(tab.data() + box_at, box0, sizeof(box0));
+    CCCS_TRY(tb.ensure(tab.size()));
     CCCS_TRY(ob.ensure(sizeof(float) * total));
     CCCS_HIP(hipStreamSynchronize(ctx->stream));
     CCCS_HIP(hipMemcpy(mb.p, mask, nv, hipMemcpyHostToDevice));
-    CCCS_HIP(hipMemcpy(tb.p, pb.data(), sizeof(ProjBeam) * pb.size(), hipMemcpyHostToDevice));
+    CCCS_HIP(hipMemcpy(tb.p, tab.data(), tab.size(), hipMemcpyHostToDevice));
+    int* box = reinterpret_cast<int*>(tb.as<uint8_t>() + box_at);
     hipLaunchKernelGGL(mask_to_float_kernel, dim3(1024), dim3(256), 0, ctx->stream, (const uint8_t*)mb.p,
-                       mf.as<float>(), nv);
+                       mf.as<float>(), nv, ctx->vol.nx, ctx->vol.ny, box);
     CCCS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(projection_kernel, dim3((unsigned)((total + 63) / 64)), dim3(64), 0, ctx->stream,
-                       (const float*)mf.as<float>(), ctx->vol, (const ProjBeam*)tb.as<ProjBeam>(), nbeams,
-                       (uint32_t)total, ob.as<float>());
+    const v3 vox = ctx->vol.voxel;
+    hipLaunchKernelGGL(projection_kernel, dim3((unsigned)((total + 63) / 64)), dim3(64 * kSubRays), 0, ctx->stream,
+                       (const float*)mf.as<float>(), ctx->vol, mk3(1.f / vox.x, 1.f / vox.y, 1.f / vox.z), (const int*)box,
+                       (const ProjBeam*)tb.as<ProjBeam>(), nbeams, (uint32_t)total, ob.as<float>());
     CCCS_HIP(hipGetLastError());
     CCCS_HIP(hipStreamSynchronize(ctx->stream));
     CCCS_HIP(hipMemcpy(fluence, ob.p, sizeof(float) * total, hipMemcpyDeviceToHost));
