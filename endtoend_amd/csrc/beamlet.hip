@@ -918,12 +918,17 @@ __global__ void __launch_bounds__(256) bl_unpack_kernel(UnpackArgs a) {
 }
 
 // ---- sparse columns without an arena -------------------------------------------------------------
-// One workgroup per beamlet walks the calc_bbox rows (i, j) of its box in the emission order of
-// _sparsify (i outer, j, k inner).  The pillar's voxels along a row form one interval of k (the
+// Workgroups walk the calc_bbox rows (i, j) of a beamlet's box in the emission order of _sparsify (i
+// outer, j, k inner), 256 rows each.  The pillar's voxels along a row form one interval of k (the
 // pillar is a box in its own frame and the frame is affine in k), found by clipping the row
 // against the pillar's three slabs (matrix form, widened); inside it the exact unpack test and
 // fetch of UnpackBEVDosePillar decide each value.  Nothing is stored between passes: the values
 // are recomputed for the max, the counts and the emission.
+//
+// One workgroup per beamlet left most of the device idle (a job has some 400 beamlets, their boxes up
+// to 150 chunks of rows each) and made every pass a chain of its chunks; the three passes took 0.93 ms
+// (one 5 mm beam, 128^3 water), 4.1 ms (thorax, 3 beams) and 110 us (32^3 water), by chunks 0.34 ms,
+// 1.31 ms and 37 us.
 
 struct ColArgs {
     const BatchDev* batches;
@@ -934,7 +939,10 @@ struct ColArgs {
     int nx, ny;        // full volume dims (keys)
     float thresh;
     uint32_t* stat;    // per beamlet {kept, dropped, max bits, 0}
-    uint16_t* rowcnt;  // kept entries of every (i, j) row of every beamlet's box (from the scan)
+    uint16_t* rowcnt;  // kept entries of every (i, j) row of every beamlet's box
+    uint32_t* chunkcnt;  // [beamlet][chunks]: kept entries of every chunk of 256 rows
+    int chunks;        // chunks of the largest box
+    int beamlet0;      // first beamlet of this launch
     const uint64_t* off;
     uint64_t* keys;
     float* vals;
@@ -979,17 +987,26 @@ __device__ __forceinline__ void pillar_row(const ColArgs& a, const BeamletDev& b
     }
 }
 
+// The chunk of rows of a workgroup: its beamlet (of the launch's), and the chunk's place in the box.
+// Chunks of a beamlet are neighbours, so they share an L2.
+__device__ __forceinline__ int row_chunk(const ColArgs& a, int& chunk) {
+    const uint32_t item = xcd_chunks(blockIdx.x, gridDim.x, 64);
+    const int q = (int)(item / (uint32_t)a.chunks);
+    chunk = (int)(item - (uint32_t)q * (uint32_t)a.chunks);
+    return a.beamlet0 + q;
+}
+
 // Per-beamlet column statistics of _sparsify (DoseCalcIO/sparse_io.cpp:22-58): max over the
-// column (zeros outside the pillar count), kept (v > t * max) and dropped (0 < v <= t * max).
-__global__ void __launch_bounds__(256) bl_colscan_kernel(ColArgs a) {
-    __shared__ float s_max[4];
-    __shared__ uint32_t s_k[4], s_d[4];
-    const BeamletDev& bl = a.beamlets[blockIdx.x];
+// column (zeros outside the pillar count), kept (v > t * max) and dropped (0 < v <= t * max).  Pass 1:
+// the maximum (the bits of a non-negative float order as integers).
+__global__ void __launch_bounds__(256) bl_colmax_kernel(ColArgs a) {
+    int chunk;
+    const int b = row_chunk(a, chunk);
+    const BeamletDev& bl = a.beamlets[b];
     const BatchDev& B = a.batches[bl.batch];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int rows = bl.boxn[0] * bl.boxn[1];
+    const int rows = bl.boxn[0] * bl.boxn[1], r = chunk * 256 + (int)threadIdx.x;
     float mx = 0.f;
-    for (int r = t; r < rows; r += 256) {
+    if (r < rows) {
         const int i = r / bl.boxn[1], j = r - i * bl.boxn[1];
         int k0, k1;
         pillar_row(a, bl, B, bl.box0[0] + i, bl.box0[1] + j, k0, k1);
@@ -997,35 +1014,43 @@ __global__ void __launch_bounds__(256) bl_colscan_kernel(ColArgs a) {
             mx = fmaxf(mx, pillar_value(a, bl, B, bl.box0[0] + i, bl.box0[1] + j, bl.box0[2] + k));
     }
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if (lane == 0) s_max[w] = mx;
-    __syncthreads();
-    const float cmax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-    const float cut = a.thresh * cmax;
+    if ((threadIdx.x & 63) == 0 && mx > 0.f) atomicMax(a.stat + 4 * b + 2, __float_as_uint(mx));
+}
+
+// Pass 2: the counts, of every row, chunk and beamlet.
+__global__ void __launch_bounds__(256) bl_colcount_kernel(ColArgs a) {
+    __shared__ uint32_t s_k[4], s_d[4];
+    int chunk;
+    const int b = row_chunk(a, chunk);
+    const BeamletDev& bl = a.beamlets[b];
+    const BatchDev& B = a.batches[bl.batch];
+    const int rows = bl.boxn[0] * bl.boxn[1], r = chunk * 256 + (int)threadIdx.x;
+    if (chunk * 256 >= rows) return;
+    const float cut = a.thresh * __uint_as_float(a.stat[4 * b + 2]);
     uint32_t kept = 0, dropped = 0;
-    for (int r = t; r < rows; r += 256) {
+    if (r < rows) {
         const int i = r / bl.boxn[1], j = r - i * bl.boxn[1];
         int k0, k1;
         pillar_row(a, bl, B, bl.box0[0] + i, bl.box0[1] + j, k0, k1);
-        uint32_t rk = 0;
         for (int k = k0; k < k1; k++) {
             const float v = pillar_value(a, bl, B, bl.box0[0] + i, bl.box0[1] + j, bl.box0[2] + k);
-            if (v > cut) rk++;
+            if (v > cut) kept++;
             else if (v > 0.f) dropped++;
         }
-        kept += rk;
-        a.rowcnt[(size_t)bl.row0 + (size_t)r] = (uint16_t)rk;
+        a.rowcnt[(size_t)bl.row0 + (size_t)r] = (uint16_t)kept;
     }
     for (int o = 32; o > 0; o >>= 1) {
         kept += __shfl_xor(kept, o, 64);
         dropped += __shfl_xor(dropped, o, 64);
     }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (lane == 0) { s_k[w] = kept; s_d[w] = dropped; }
     __syncthreads();
-    if (t == 0) {
-        a.stat[4 * blockIdx.x + 0] = s_k[0] + s_k[1] + s_k[2] + s_k[3];
-        a.stat[4 * blockIdx.x + 1] = s_d[0] + s_d[1] + s_d[2] + s_d[3];
-        a.stat[4 * blockIdx.x + 2] = __float_as_uint(cmax);
-        a.stat[4 * blockIdx.x + 3] = 0;
+    if (threadIdx.x == 0) {
+        const uint32_t tk = s_k[0] + s_k[1] + s_k[2] + s_k[3], td = s_d[0] + s_d[1] + s_d[2] + s_d[3];
+        a.chunkcnt[(size_t)b * a.chunks + chunk] = tk;
+        if (tk) atomicAdd(a.stat + 4 * b + 0, tk);
+        if (td) atomicAdd(a.stat + 4 * b + 1, td);
     }
 }
 
@@ -1051,72 +1076,75 @@ __global__ void __launch_bounds__(1024) bl_offsets_kernel(uint32_t* __restrict__
     if (threadIdx.x == 0) off[n] = carry;
 }
 
-// Writes each beamlet's kept entries at its offset (one workgroup per beamlet), key = full-volume
-// linear index, value = dose, in the emission order of _sparsify.  The rows go in chunks of 256,
-// one per thread, with their kept counts from the column scan; each wave's 64 rows form one
-// contiguous range of the output.  A wave fills that range window by window: every lane evaluates
-// its row's values once, in k order, and stages the kept entries that fall in the window in LDS;
-// then the wave copies the window out with whole-wave, contiguous stores.
+// Writes each beamlet's kept entries at its offset, key = full-volume linear index, value = dose, in the
+// emission order of _sparsify.  A workgroup takes one chunk of 256 rows, one per thread, with their
+// kept counts from the count pass; each wave's 64 rows form one contiguous range of the output.  A wave
+// fills that range window by window: every lane evaluates its row's values once, in k order, and stages
+// the kept entries that fall in the window in LDS; then the wave copies the window out with
+// whole-wave, contiguous stores.
 constexpr uint32_t kEmitWindow = 512;  // staged entries per wave and round (6 KB)
 __global__ void __launch_bounds__(256) bl_emit_kernel(ColArgs a) {
     __shared__ uint64_t s_key[4][kEmitWindow];
     __shared__ float s_val[4][kEmitWindow];
-    __shared__ uint32_t s_w[4];
-    const BeamletDev& bl = a.beamlets[blockIdx.x];
+    __shared__ uint32_t s_w[4], s_b[4];
+    int chunk;
+    const int b = row_chunk(a, chunk);
+    const BeamletDev& bl = a.beamlets[b];
     const BatchDev& B = a.batches[bl.batch];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const uint32_t* cc = a.chunkcnt + (size_t)b * a.chunks;
     const int rows = bl.boxn[0] * bl.boxn[1];
-    const float cut = a.thresh * __uint_as_float(a.stat[4 * blockIdx.x + 2]);
-    uint64_t pos = a.off[blockIdx.x];
-    for (int base = 0; base < rows; base += 256) {
-        const int r = base + t;
-        const uint32_t n = r < rows ? (uint32_t)a.rowcnt[(size_t)bl.row0 + (size_t)r] : 0u;
-        // inclusive scan of n over the wave, and the waves' totals
-        uint32_t inc = n;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += u;
-        }
-        if (lane == 63) s_w[w] = inc;
-        __syncthreads();
-        uint32_t before = 0, total = 0, most = 0;
-        for (int q = 0; q < 4; q++) {
-            before += q < w ? s_w[q] : 0u;
-            total += s_w[q];
-            most = max(most, s_w[q]);
-        }
-        const uint32_t W = s_w[w];
-        __syncthreads();
-        int X = 0, Y = 0, k = 0, k1 = 0;
-        if (n) {
-            const int i = r / bl.boxn[1], j = r - i * bl.boxn[1];
-            pillar_row(a, bl, B, bl.box0[0] + i, bl.box0[1] + j, k, k1);
-            X = bl.box0[0] + i;
-            Y = bl.box0[1] + j;
-        }
-        uint32_t p = inc - n;  // next output of this lane, relative to the wave's range
-        const uint64_t wout = pos + before;
-        // the same number of rounds in every wave (the barriers), enough for the fullest wave
-        for (uint32_t wb = 0; wb < most; wb += kEmitWindow) {
-            const uint32_t we = min(W, wb + kEmitWindow);
-            while (p < inc && p < we && k < k1) {
-                const float v = pillar_value(a, bl, B, X, Y, bl.box0[2] + k);
-                if (v > cut) {
-                    s_key[w][p - wb] = ((uint64_t)(bl.box0[2] + k + a.bbs[2]) * (uint64_t)a.ny +
-                                        (uint64_t)(Y + a.bbs[1])) * (uint64_t)a.nx + (uint64_t)(X + a.bbs[0]);
-                    s_val[w][p - wb] = v;
-                    p++;
-                }
-                k++;
+    if (chunk * 256 >= rows || cc[chunk] == 0u) return;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const float cut = a.thresh * __uint_as_float(a.stat[4 * b + 2]);
+    // entries of the beamlet's earlier chunks
+    uint32_t earlier = 0;
+    for (int c = t; c < chunk; c += 256) earlier += cc[c];
+    for (int o = 32; o > 0; o >>= 1) earlier += __shfl_xor(earlier, o, 64);
+    const int r = chunk * 256 + t;
+    const uint32_t n = r < rows ? (uint32_t)a.rowcnt[(size_t)bl.row0 + (size_t)r] : 0u;
+    // inclusive scan of n over the wave, and the waves' totals
+    uint32_t inc = n;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+    }
+    if (lane == 63) s_w[w] = inc;
+    if (lane == 0) s_b[w] = earlier;
+    __syncthreads();
+    uint64_t wout = a.off[b];
+    uint32_t most = 0;
+    for (int q = 0; q < 4; q++) {
+        wout += s_b[q] + (q < w ? s_w[q] : 0u);
+        most = max(most, s_w[q]);
+    }
+    const uint32_t W = s_w[w];
+    int X = 0, Y = 0, k = 0, k1 = 0;
+    if (n) {
+        const int i = r / bl.boxn[1], j = r - i * bl.boxn[1];
+        pillar_row(a, bl, B, bl.box0[0] + i, bl.box0[1] + j, k, k1);
+        X = bl.box0[0] + i;
+        Y = bl.box0[1] + j;
+    }
+    uint32_t p = inc - n;  // next output of this lane, relative to the wave's range
+    // the same number of rounds in every wave (the barriers), enough for the fullest wave
+    for (uint32_t wb = 0; wb < most; wb += kEmitWindow) {
+        const uint32_t we = min(W, wb + kEmitWindow);
+        while (p < inc && p < we && k < k1) {
+            const float v = pillar_value(a, bl, B, X, Y, bl.box0[2] + k);
+            if (v > cut) {
+                s_key[w][p - wb] = ((uint64_t)(bl.box0[2] + k + a.bbs[2]) * (uint64_t)a.ny +
+                                    (uint64_t)(Y + a.bbs[1])) * (uint64_t)a.nx + (uint64_t)(X + a.bbs[0]);
+                s_val[w][p - wb] = v;
+                p++;
             }
-            __syncthreads();
-            for (uint32_t e = wb + (uint32_t)lane; e < we; e += 64) {
-                a.keys[wout + e] = s_key[w][e - wb];
-                a.vals[wout + e] = s_val[w][e - wb];
-            }
-            __syncthreads();
+            k++;
         }
-        pos += total;
+        __syncthreads();
+        for (uint32_t e = wb + (uint32_t)lane; e < we; e += 64) {
+            a.keys[wout + e] = s_key[w][e - wb];
+            a.vals[wout + e] = s_val[w][e - wb];
+        }
+        __syncthreads();
     }
 }
 
@@ -2457,9 +2485,16 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         // the previous job's columns reach the sink while this job's cone passes run on the device
         CCCS_TRY(run_job_cones(ctx, J, deliver));
         const int nbl = (int)J.beamlets.size();
-        CCCS_TRY(ctx->bl_cnt.ensure(sizeof(uint32_t) * 4 * nbl + sizeof(uint64_t) * (nbl + 1) + 256));
+        int max_rows = 1;
+        for (const BeamletDev& bl : J.beamlets) max_rows = std::max(max_rows, bl.boxn[0] * bl.boxn[1]);
+        const int chunks = (max_rows + 255) / 256;
+        const uint64_t units = (uint64_t)nbl * (uint64_t)chunks;
+        if (units > 0x7fffffffULL) return set_error(CCCS_EGEOM, "too many beamlet rows in one job");
+        const size_t o_off = (sizeof(uint32_t) * 4 * nbl + 255) & ~size_t(255);
+        const size_t o_chunk = (o_off + sizeof(uint64_t) * (nbl + 1) + 255) & ~size_t(255);
+        CCCS_TRY(ctx->bl_cnt.ensure(o_chunk + sizeof(uint32_t) * units));
         uint32_t* stat = ctx->bl_cnt.as<uint32_t>();
-        uint64_t* offs = reinterpret_cast<uint64_t*>(ctx->bl_cnt.as<uint8_t>() + ((sizeof(uint32_t) * 4 * nbl + 255) & ~size_t(255)));
+        uint64_t* offs = reinterpret_cast<uint64_t*>(ctx->bl_cnt.as<uint8_t>() + o_off);
         const size_t sz_b = sizeof(BatchDev) * J.batches.size();
         ColArgs ca;
         ca.batches = ctx->bl_tab.as<BatchDev>();
@@ -2476,12 +2511,18 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         ca.stat = stat;
         CCCS_TRY(ctx->bl_rowcnt.ensure(sizeof(uint16_t) * std::max<uint64_t>(1, J.rows)));
         ca.rowcnt = ctx->bl_rowcnt.as<uint16_t>();
+        ca.chunkcnt = reinterpret_cast<uint32_t*>(ctx->bl_cnt.as<uint8_t>() + o_chunk);
+        ca.chunks = chunks;
+        ca.beamlet0 = 0;
         ca.off = offs;
         ca.keys = nullptr;
         ca.vals = nullptr;
         if (copy_done) CCCS_HIP(hipStreamWaitEvent(ctx->stream, copy_done, 0));
         int tok = prof_begin(ctx, K_BL_UNPACK);
-        hipLaunchKernelGGL(bl_colscan_kernel, dim3(nbl), dim3(256), 0, ctx->stream, ca);
+        hipLaunchKernelGGL(bl_fill_kernel, dim3(grid_for(4 * (uint64_t)nbl, 256)), dim3(256), 0, ctx->stream,
+                           reinterpret_cast<float*>(stat), 4 * (uint64_t)nbl, 0.f);
+        hipLaunchKernelGGL(bl_colmax_kernel, dim3((unsigned)units), dim3(256), 0, ctx->stream, ca);
+        hipLaunchKernelGGL(bl_colcount_kernel, dim3((unsigned)units), dim3(256), 0, ctx->stream, ca);
         prof_end(ctx, tok, 0.0, 0.0, (uint64_t)nbl);
         hipLaunchKernelGGL(bl_offsets_kernel, dim3(1), dim3(1024), 0, ctx->stream, stat, nbl, offs);
         CCCS_HIP(hipGetLastError());
@@ -2495,7 +2536,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         ca.keys = ctx->bl_keys.as<uint64_t>();
         ca.vals = ctx->bl_vals.as<float>();
         int tk = prof_begin(ctx, K_BL_COMPACT);
-        hipLaunchKernelGGL(bl_emit_kernel, dim3(nbl), dim3(256), 0, ctx->stream, ca);
+        hipLaunchKernelGGL(bl_emit_kernel, dim3((unsigned)units), dim3(256), 0, ctx->stream, ca);
         // algorithmic traffic: the kept entries (8 B key + 4 B value)
         prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
         CCCS_HIP(hipGetLastError());
