@@ -1509,11 +1509,13 @@ void pillar_box(const cccs_problem& p, const cccs_beam& b, const BeamletPlan& o,
 // A finished job's sparse columns in pinned host memory, and the event that marks them copied.
 struct Delivery {
     bool live = false;
-    hipEvent_t ev = nullptr;
+    int nparts = 0;
+    hipEvent_t ev[kColParts] = {};  // the copy of each part's columns
+    size_t end[kColParts] = {};     // one past the last column of each part
     uint64_t* keys = nullptr;
     float* vals = nullptr;
-    uint32_t* stat = nullptr;  // per column: kept, dropped, (two unused)
-    uint32_t* rcnt = nullptr;  // per column and ROI: kept entries (ROI reduction)
+    const uint32_t* stat = nullptr;  // per column: kept, dropped, (two unused)
+    const uint32_t* rcnt = nullptr;  // per column and ROI: kept entries (ROI reduction)
     int nroi = 0;
     std::vector<std::pair<int, int>> cols;  // (request beam, fluence index) per column
 };
@@ -2144,6 +2146,7 @@ struct RoiArgs {
     const uint64_t* roff;        // [column][roi] first reduced entry (exclusive scan of cnt)
     uint64_t* rkeys;
     float* rvals;
+    int col0;                    // first column of this launch
 };
 
 // ROI rank of CT voxel `key` in ROI r (or -1).
@@ -2157,7 +2160,7 @@ __device__ __forceinline__ int32_t roi_rank(const RoiArgs& a, const RoiDev& R, i
 // chunk and ROI).
 __global__ void __launch_bounds__(256) roi_count_kernel(RoiArgs a) {
     __shared__ uint32_t s_c[kMaxRoi];
-    const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int q = a.col0 + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     for (int r = tid; r < a.nroi; r += 256) s_c[r] = 0u;
     __syncthreads();
     const uint64_t e0 = a.off[q], e1 = a.off[q + 1];
@@ -2185,7 +2188,7 @@ __global__ void __launch_bounds__(256) roi_count_kernel(RoiArgs a) {
 // order-preserving compaction per 256-entry chunk), keyed mark + rank.
 __global__ void __launch_bounds__(256) roi_emit_kernel(RoiArgs a) {
     __shared__ uint32_t s_w[4];
-    const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int q = a.col0 + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const uint64_t e0 = a.off[q], e1 = a.off[q + 1];
     const uint64_t plane = (uint64_t)a.nx * (uint64_t)a.ny;
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -2402,7 +2405,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         return CCCS_OK;
     }
     const size_t nvox = (size_t)p.bbox_size[0] * p.bbox_size[1] * p.bbox_size[2];
-    const size_t budget = size_t(ctx->sched.bl_job_gb) << 30;  // device bytes per job
+    const uint64_t budget_max = uint64_t(ctx->sched.bl_job_gb) << 30;  // device bytes per job
     const int nset = std::min(std::max(ctx->sched.bl_streams, 1), kRaySets);
     size_t next = 0;
     // device footprint of each batch, additive per cone direction: a job needs its batches' packed
@@ -2413,24 +2416,39 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
     std::vector<uint64_t> b_fixed(refs.size());
     for (size_t i = 0; i < refs.size(); i++)
         CCCS_TRY(batch_footprint(ctx, plans, refs[i], b_rev[i], b_lines[i], b_fixed[i]));
+    // device bytes of the batches [k0, k1) as one job: every direction in flight holds its own REV
+    // store, half steps and line table
+    auto job_bytes = [&](size_t k0, size_t k1) {
+        uint64_t mr = 0, ml = 0, fixed = 0;
+        for (int r = 0; r < nrays; r++) {
+            uint64_t rev = 0, lines = 0;
+            for (size_t i = k0; i < k1; i++) { rev += b_rev[i][r]; lines += b_lines[i][r]; }
+            mr = std::max(mr, rev);
+            ml = std::max(ml, lines);
+        }
+        for (size_t i = k0; i < k1; i++) fixed += b_fixed[i];
+        return fixed + (uint64_t)nset * (sizeof(float) * 2 * mr + sizeof(LineMeta) * ml);
+    };
+    constexpr uint64_t kMinJob = uint64_t(1) << 30;
+    constexpr uint64_t kPartEntries = 1 << 18;  // entries a part of the columns is worth (3 MiB, 60 us of copy)
     // columns of the last finished job, waiting in pinned host memory for the sink
-    for (hipEvent_t& e : ctx->stage_ev)
-        if (!e) CCCS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if (sink && !ctx->cstream) {
-        CCCS_HIP(hipStreamCreateWithFlags(&ctx->cstream, hipStreamNonBlocking));
-        CCCS_HIP(hipEventCreateWithFlags(&ctx->copy_ev, hipEventDisableTiming));
+    if (sink) {
+        if (!ctx->cstream) CCCS_HIP(hipStreamCreateWithFlags(&ctx->cstream, hipStreamNonBlocking));
+        for (hipEvent_t& e : ctx->col_ev)
+            if (!e) CCCS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-    hipEvent_t copy_done = nullptr;  // the last job's column copy (its buffers are rewritten after it)
+    hipEvent_t copy_done = nullptr;  // the last job's last column copy (its buffers are rewritten after it)
     Delivery pending;
     int njob = 0;
     auto deliver = [&]() -> int {
         if (!pending.live) return CCCS_OK;
         pending.live = false;
-        CCCS_HIP(hipEventSynchronize(pending.ev));
         const int nroi = pending.nroi;
         std::vector<uint64_t> blocks((size_t)nroi);
         uint64_t pos = 0;
+        int part = -1;
         for (size_t q = 0; q < pending.cols.size(); q++) {
+            while (part < 0 || q >= pending.end[part]) CCCS_HIP(hipEventSynchronize(pending.ev[++part]));
             const uint32_t* st = pending.stat + 4 * q;
             cccs_sparse_column col{};
             col.beam_index = pending.cols[q].first;
@@ -2452,15 +2470,26 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             col.keys = pending.keys + pos;
             col.values = pending.vals + pos;
             pos += col.nnz;
-            if (sink(user, &col) != 0) return set_error(CCCS_EIO, "sparse sink aborted the call");
+            if (sink(user, &col) != 0) {
+                (void)hipStreamSynchronize(ctx->cstream);  // the parts still on their way
+                return set_error(CCCS_EIO, "sparse sink aborted the call");
+            }
         }
         return CCCS_OK;
     };
     while (next < refs.size()) {
-        // grow the job batch by batch while it fits the budget
+        // grow the job batch by batch while it fits the budget and, where columns go to a sink, seven
+        // tenths of what is left: the sink takes a job's columns while the next job computes, so the
+        // last job, whose columns nothing hides, should be small, and the one before it about as long
+        // as the sink takes over its predecessor (a third of the compute time or less).  Jobs below
+        // kMinJob do not fill the device, so a rest of that size stays whole.  Whole calls with the
+        // 12 GiB budget alone and with this rule: 63.8 and 55.3 ms (two fine 4pi beams), 54.5 and
+        // 49.2 ms (thorax, 3 beams).
         std::vector<uint64_t> rev(nrays, 0), lines(nrays, 0);
         uint64_t fixed = 0;
         size_t k = next;
+        const uint64_t left = job_bytes(next, refs.size());
+        const uint64_t budget = !sink ? budget_max : std::min<uint64_t>(budget_max, std::max(kMinJob, left / 10 * 7));
         while (k < refs.size()) {
             uint64_t mr = 0, ml = 0;
             for (int r = 0; r < nrays; r++) {
@@ -2526,31 +2555,41 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         prof_end(ctx, tok, 0.0, 0.0, (uint64_t)nbl);
         hipLaunchKernelGGL(bl_offsets_kernel, dim3(1), dim3(1024), 0, ctx->stream, stat, nbl, offs);
         CCCS_HIP(hipGetLastError());
-        // totals decide the output size
-        uint64_t nnz_total = 0;
-        CCCS_HIP(hipMemcpyAsync(ctx->h_small.p, offs + nbl, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+        // totals decide the output size; the counts and offsets of every column follow them to the host
+        // (two sets in turn: the sink may still read the last job's)
+        HostBuf& hst = ctx->h_bl_st[njob & 1];
+        const int nroi = ctx->nroi;
+        const size_t ncr = (size_t)nbl * (size_t)nroi;
+        const size_t cbytes = (sizeof(uint32_t) * ncr + 255) & ~size_t(255);
+        CCCS_TRY(hst.ensure(o_chunk + cbytes + sizeof(uint64_t) * (ncr + 1)));
+        uint8_t* hs = hst.as<uint8_t>();
+        const uint64_t* hoff = reinterpret_cast<const uint64_t*>(hs + o_off);
+        CCCS_HIP(hipMemcpyAsync(hs, stat, o_off + sizeof(uint64_t) * (nbl + 1), hipMemcpyDeviceToHost, ctx->stream));
         CCCS_HIP(hipStreamSynchronize(ctx->stream));
-        std::memcpy(&nnz_total, ctx->h_small.p, sizeof(uint64_t));
+        const uint64_t nnz_total = hoff[nbl];
         CCCS_TRY(ctx->bl_keys.ensure(sizeof(uint64_t) * std::max<uint64_t>(1, nnz_total)));
         CCCS_TRY(ctx->bl_vals.ensure(sizeof(float) * std::max<uint64_t>(1, nnz_total)));
         ca.keys = ctx->bl_keys.as<uint64_t>();
         ca.vals = ctx->bl_vals.as<float>();
-        int tk = prof_begin(ctx, K_BL_COMPACT);
-        hipLaunchKernelGGL(bl_emit_kernel, dim3((unsigned)units), dim3(256), 0, ctx->stream, ca);
-        // algorithmic traffic: the kept entries (8 B key + 4 B value)
-        prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
-        CCCS_HIP(hipGetLastError());
+        auto emit = [&](int b0, int b1) {
+            if (b1 <= b0) return;
+            ca.beamlet0 = b0;
+            hipLaunchKernelGGL(bl_emit_kernel, dim3((unsigned)((uint64_t)(b1 - b0) * chunks)), dim3(256), 0, ctx->stream,
+                               ca);
+        };
         // ROI reduction of the job's columns (count, scan, order-preserving emit)
-        const int nroi = ctx->nroi;
-        uint64_t rtotal = 0;
-        uint32_t* rcnt = nullptr;
+        RoiArgs ra;
+        const uint64_t* out_off = hoff;  // first output entry of every column
+        std::vector<uint64_t> roi_off;
         if (nroi > 0) {
-            const size_t ncr = (size_t)nbl * (size_t)nroi;
-            const size_t cbytes = (sizeof(uint32_t) * ncr + 255) & ~size_t(255);
+            int tk = prof_begin(ctx, K_BL_COMPACT);
+            emit(0, nbl);
+            // algorithmic traffic: the kept entries (8 B key + 4 B value)
+            prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
+            CCCS_HIP(hipGetLastError());
             CCCS_TRY(ctx->roi_cnt.ensure(cbytes + sizeof(uint64_t) * (ncr + 1)));
-            rcnt = ctx->roi_cnt.as<uint32_t>();
+            uint32_t* rcnt = ctx->roi_cnt.as<uint32_t>();
             uint64_t* roff = reinterpret_cast<uint64_t*>(ctx->roi_cnt.as<uint8_t>() + cbytes);
-            RoiArgs ra;
             ra.rois = ctx->roi_tab.as<RoiDev>();
             ra.rank = ctx->roi_rank.as<int32_t>();
             ra.nroi = nroi;
@@ -2563,56 +2602,79 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             ra.roff = roff;
             ra.rkeys = nullptr;
             ra.rvals = nullptr;
+            ra.col0 = 0;
             hipLaunchKernelGGL(roi_count_kernel, dim3(nbl), dim3(256), 0, ctx->stream, ra);
             hipLaunchKernelGGL(roi_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, (const uint32_t*)rcnt, ncr, roff);
             CCCS_HIP(hipGetLastError());
-            CCCS_HIP(hipMemcpyAsync(ctx->h_small.p, roff + ncr, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+            CCCS_HIP(hipMemcpyAsync(hs + o_chunk, rcnt, cbytes + sizeof(uint64_t) * (ncr + 1), hipMemcpyDeviceToHost,
+                                    ctx->stream));
             CCCS_HIP(hipStreamSynchronize(ctx->stream));
-            std::memcpy(&rtotal, ctx->h_small.p, sizeof(uint64_t));
-            CCCS_TRY(ctx->roi_keys.ensure(sizeof(uint64_t) * std::max<uint64_t>(1, rtotal)));
-            CCCS_TRY(ctx->roi_vals.ensure(sizeof(float) * std::max<uint64_t>(1, rtotal)));
+            const uint64_t* hroff = reinterpret_cast<const uint64_t*>(hs + o_chunk + cbytes);
+            roi_off.resize((size_t)nbl + 1);
+            for (int q = 0; q <= nbl; q++) roi_off[(size_t)q] = hroff[(size_t)q * (size_t)nroi];
+            out_off = roi_off.data();
+            CCCS_TRY(ctx->roi_keys.ensure(sizeof(uint64_t) * std::max<uint64_t>(1, out_off[nbl])));
+            CCCS_TRY(ctx->roi_vals.ensure(sizeof(float) * std::max<uint64_t>(1, out_off[nbl])));
             ra.rkeys = ctx->roi_keys.as<uint64_t>();
             ra.rvals = ctx->roi_vals.as<float>();
-            hipLaunchKernelGGL(roi_emit_kernel, dim3(nbl), dim3(256), 0, ctx->stream, ra);
-            CCCS_HIP(hipGetLastError());
         }
-        if (!sink) continue;  // columns stay on the device (overwritten by the next job)
+        const uint64_t nout = out_off[nbl];
         // columns to pinned host memory (full PCIe rate, one of two buffers in turn); the sink sees
-        // them in place, during the next job or at the end of the call
-        const uint64_t nout = nroi > 0 ? rtotal : nnz_total;
-        const size_t kbytes = sizeof(uint64_t) * nout, vbytes = sizeof(float) * nout;
-        const size_t sbytes = sizeof(uint32_t) * 4 * (size_t)nbl;
-        const size_t rbytes = sizeof(uint32_t) * (size_t)nbl * (size_t)nroi;
-        HostBuf& hbuf = (njob & 1) ? ctx->h_bl_out2 : ctx->h_bl_out;
-        CCCS_TRY(hbuf.ensure(kbytes + vbytes + sbytes + rbytes + 64));
-        uint8_t* hb = hbuf.as<uint8_t>();
+        // them in place, during the next job or at the end of the call.  They go in parts of about
+        // equal size: while the sink takes one part, the next ones are emitted and copied.  The copies
+        // run on their own stream: the next job's cone passes, queued behind this compaction, do not
+        // wait for them; the next compaction waits before rewriting the buffers.
+        const int nparts = !sink ? 1 : (int)std::min<uint64_t>(kColParts, std::max<uint64_t>(1, nout / kPartEntries));
         Delivery& D = pending;
-        D.keys = reinterpret_cast<uint64_t*>(hb);
-        D.vals = reinterpret_cast<float*>(hb + kbytes);
-        D.stat = reinterpret_cast<uint32_t*>(hb + kbytes + vbytes);
-        D.rcnt = D.stat + 4 * (size_t)nbl;
-        D.nroi = nroi;
-        D.cols.resize((size_t)nbl);
-        for (int q = 0; q < nbl; q++) {
-            const BeamletDev& d = J.beamlets[q];
-            D.cols[(size_t)q] = {plans[sel[d.batch].plan].beam, d.fidx};
+        if (sink) {
+            const size_t kbytes = sizeof(uint64_t) * nout;
+            HostBuf& hbuf = (njob & 1) ? ctx->h_bl_out2 : ctx->h_bl_out;
+            CCCS_TRY(hbuf.ensure(kbytes + sizeof(float) * nout + 64));
+            D.keys = hbuf.as<uint64_t>();
+            D.vals = reinterpret_cast<float*>(hbuf.as<uint8_t>() + kbytes);
+            D.stat = reinterpret_cast<const uint32_t*>(hs);
+            D.rcnt = reinterpret_cast<const uint32_t*>(hs + o_chunk);
+            D.nroi = nroi;
+            D.cols.resize((size_t)nbl);
+            for (int q = 0; q < nbl; q++) {
+                const BeamletDev& d = J.beamlets[q];
+                D.cols[(size_t)q] = {plans[sel[d.batch].plan].beam, d.fidx};
+            }
+            D.nparts = nparts;
         }
-        // the copies run on their own stream: the next job's cone passes, queued behind this
-        // compaction, do not wait for them; the next compaction waits before rewriting the buffers
-        hipStream_t cs = ctx->cstream;
-        CCCS_HIP(hipEventRecord(ctx->copy_ev, ctx->stream));
-        CCCS_HIP(hipStreamWaitEvent(cs, ctx->copy_ev, 0));
-        CCCS_HIP(hipMemcpyAsync(D.stat, stat, sbytes, hipMemcpyDeviceToHost, cs));
-        if (nroi > 0) CCCS_HIP(hipMemcpyAsync(D.rcnt, rcnt, rbytes, hipMemcpyDeviceToHost, cs));
-        if (nout) {
-            CCCS_HIP(hipMemcpyAsync(D.keys, nroi > 0 ? ctx->roi_keys.p : ctx->bl_keys.p, kbytes, hipMemcpyDeviceToHost,
-                                    cs));
-            CCCS_HIP(hipMemcpyAsync(D.vals, nroi > 0 ? ctx->roi_vals.p : ctx->bl_vals.p, vbytes, hipMemcpyDeviceToHost,
-                                    cs));
+        int tk = nroi > 0 ? -1 : prof_begin(ctx, K_BL_COMPACT);
+        for (int part = 0, b0 = 0; part < nparts; part++) {
+            int b1 = nbl;
+            if (part + 1 < nparts)
+                b1 = (int)(std::lower_bound(out_off + b0, out_off + nbl, nout / nparts * (part + 1)) - out_off);
+            if (nroi > 0) {
+                ra.col0 = b0;
+                if (b1 > b0) hipLaunchKernelGGL(roi_emit_kernel, dim3(b1 - b0), dim3(256), 0, ctx->stream, ra);
+            } else {
+                emit(b0, b1);
+            }
+            CCCS_HIP(hipGetLastError());
+            if (sink) {
+                hipStream_t cs = ctx->cstream;
+                hipEvent_t ev = ctx->col_ev[(njob & 1) * kColParts + part];
+                const uint64_t e0 = out_off[b0], n = out_off[b1] - e0;
+                CCCS_HIP(hipEventRecord(ev, ctx->stream));
+                CCCS_HIP(hipStreamWaitEvent(cs, ev, 0));
+                if (n) {
+                    const uint64_t* sk = (nroi > 0 ? ctx->roi_keys : ctx->bl_keys).as<uint64_t>();
+                    const float* sv = (nroi > 0 ? ctx->roi_vals : ctx->bl_vals).as<float>();
+                    CCCS_HIP(hipMemcpyAsync(D.keys + e0, sk + e0, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, cs));
+                    CCCS_HIP(hipMemcpyAsync(D.vals + e0, sv + e0, sizeof(float) * n, hipMemcpyDeviceToHost, cs));
+                }
+                CCCS_HIP(hipEventRecord(ev, cs));
+                D.ev[part] = ev;
+                D.end[part] = (size_t)b1;
+                copy_done = ev;
+            }
+            b0 = b1;
         }
-        CCCS_HIP(hipEventRecord(ctx->stage_ev[njob & 1], cs));
-        D.ev = ctx->stage_ev[njob & 1];
-        copy_done = D.ev;
+        if (nroi == 0) prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
+        if (!sink) continue;  // columns stay on the device (overwritten by the next job)
         D.live = true;
         njob++;
     }

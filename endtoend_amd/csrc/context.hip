@@ -349,12 +349,14 @@ extern "C" int cccs_ctx_destroy(cccs_ctx* c) {
     c->h_small.release(); c->h_cones.release(); c->h_stage.release();
     for (hipEvent_t& e : c->stage_ev)
         if (e) (void)hipEventDestroy(e);
-    if (c->copy_ev) (void)hipEventDestroy(c->copy_ev);
+    for (hipEvent_t& e : c->col_ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->cstream) (void)hipStreamDestroy(c->cstream);
     c->bl_tab.release(); c->bl_pdose.release(); c->bl_lcone.release(); c->bl_rowcnt.release(); c->bl_arena.release();
     c->bl_cnt.release(); c->bl_keys.release(); c->bl_vals.release(); c->bl_fmap.release();
     c->bl_h.release(); c->bl_queue.release(); c->bl_qcnt.release(); c->bl_tiles.release();
     c->h_bl.release(); c->h_bl_out.release(); c->h_bl_out2.release();
+    for (HostBuf& h : c->h_bl_st) h.release();
     c->roi_tab.release(); c->roi_rank.release(); c->roi_cnt.release(); c->roi_keys.release(); c->roi_vals.release();
     for (hipEvent_t e : c->prof.pool) (void)hipEventDestroy(e);
     for (uint32_t* p : c->prof.chunks) (void)hipFree(p);

@@ -99,6 +99,7 @@ struct LineMeta;
 
 namespace cccs {
 constexpr int kConeClasses = 4;
+constexpr int kColParts = 8;  // parts in which a job's beamlet columns go to the host
 constexpr int kRaySets = 4;  // most cone directions of the beamlet pipeline in flight
 // Launch-schedule knobs (cccs_ctx_set_schedule).  They change how the work is scheduled, never
 // which samples contribute.
@@ -163,11 +164,12 @@ struct cccs_ctx {
     cccs::HostBuf h_small, h_cones, h_stage;  // h_stage: pinned double buffer of download_staged
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     hipStream_t cstream = nullptr;  // beamlet columns to pinned host memory, beside the next job
-    hipEvent_t copy_ev = nullptr;
+    hipEvent_t col_ev[2 * cccs::kColParts] = {};  // the parts of a job's columns, alternate jobs in turn
     // beamlet path: job tables, packed grids, column arena, sparse output, line grids
     cccs::DevBuf bl_tab, bl_pdose, bl_arena, bl_cnt, bl_keys, bl_vals, bl_fmap, bl_h, bl_queue, bl_qcnt, bl_tiles,
         bl_lcone, bl_rowcnt;
-    cccs::HostBuf h_bl, h_bl_out, h_bl_out2;  // h_bl_out/h_bl_out2: sparse columns of alternate jobs
+    // h_bl_out/h_bl_out2 and h_bl_st: sparse columns of alternate jobs, and their counts and offsets
+    cccs::HostBuf h_bl, h_bl_out, h_bl_out2, h_bl_st[2];
     std::vector<uint8_t> scratch_host;
     cccs::Profiler prof;
     cccs::Schedule sched;
