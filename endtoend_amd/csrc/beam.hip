@@ -130,9 +130,14 @@ __global__ void __launch_bounds__(256) terma_kernel(TermaArgs a) {
         // in which a resident unit-TERMA grid of the same source gives the same value
         const v3 p = terma_point(a, X, Y, Z);
         const float fl = point_fluence(p, a.fmap, a.beam, a.beamletnum);
-        int it = 0;
-        acc = fl > 0.f ? fl * unit_point_terma(p, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, &it) : 0.f;
-        steps = (uint32_t)it;
+        if (!(fl > 0.f)) {
+        } else if (a.counts) {
+            int it = 0;
+            acc = fl * unit_point_terma(p, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, &it);
+            steps = (uint32_t)it;
+        } else {
+            acc = fl * unit_point_terma(p, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, nullptr);
+        }
     }
     if (in) a.terma[(size_t)X + (size_t)a.bx * ((size_t)Y + (size_t)a.by * Z)] = acc;
     if (a.counts) block_count(steps, a.counts, blockIdx.x);

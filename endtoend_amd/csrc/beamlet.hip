@@ -610,10 +610,19 @@ __global__ void __launch_bounds__(256) bl_siddon_kernel(BlArgs a, const TermaReq
         if (r.slot == kNoSlot) continue;
         const BeamletDev& bl = a.beamlets[r.beamlet];
         const BatchDev& B = a.batches[bl.batch];
-        int it = 0;
-        a.rev[r.slot] = point_terma_rpl(mk3(r.x, r.y, r.z), B.fmap, B.beam, a.spec, a.vd, a.ivoxel, a.dens, a.bhc, bl.fidx,
-                                        &it);
-        steps += (uint32_t)it;
+        // (the request's point lies in its beamlet's cell: the sample stage tested it)
+        const float fluence = B.fmap[bl.fidx];
+        const v3 p = mk3(r.x, r.y, r.z);
+        float v = 0.f;
+        if (fluence <= 0.f) {
+        } else if (counts) {
+            int it = 0;
+            v = fluence_terma_rpl(p, fluence, B.beam, a.spec, a.vd, a.ivoxel, a.dens, a.bhc, &it);
+            steps += (uint32_t)it;
+        } else {
+            v = fluence_terma_rpl(p, fluence, B.beam, a.spec, a.vd, a.ivoxel, a.dens, a.bhc, nullptr);
+        }
+        a.rev[r.slot] = v;
     }
     if (counts) block_count(steps, counts, blockIdx.x);
 }
