@@ -1577,7 +1577,7 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     CCCS_HIP(hipGetLastError());
     uint32_t* d_scan = nullptr;
     CCCS_TRY(S.get(ctx->scan, line_scan_words(g.total_lines), &d_scan));
-    CCCS_TRY(launch_line_scan(ctx, ca.lines, g.total_lines, d_scan));
+    CCCS_TRY(launch_line_scan(ctx, ca.lines, g.total_lines, d_scan, 0));
     // stored-length classes: one launch each, with LDS for the class's longest line, so that the
     // many short lines are not held to the occupancy of the longest
     uint32_t maxn = 1;

@@ -27,6 +27,7 @@
 namespace cccs {
 
 constexpr int kWall = 2;        // pillar wall, REV samples (PILLAR_GRID, io_data_structs.h:139-160)
+constexpr int kLineZeros = 2;   // zero samples kept before and behind every stored REV line (BlArgs::zeros)
 constexpr int kBuffer = 2;      // pillar rim excluded from unpacking (same struct)
 constexpr int kMaxBatches = 100;  // batch-count retry limit of the reference (host.cu:692-834)
 constexpr uint32_t kSubQueues = 64;  // TERMA sub-queues per cone direction
@@ -76,6 +77,8 @@ struct BatchDev {
     uint64_t pdose;        // float offset of its packed dose grid ([pX][pZ][pY], pY fastest)
     uint32_t tile0;        // first gather tile
     int tiles[3];          // gather tiles along pY (16), pZ (4), pX (4)
+    uint32_t tdiv[2];      // t / tiles[k] == umulhi(t, tdiv[k]) for the batch's tiles (0: divide)
+    float ipd[3];          // 1 / pd
     float fc[2];           // beamlet axis in pillar sample coordinates (x, z)
     float fw;              // bound on the footprint half-width [samples]: farther samples get no TERMA
     float cb[8];           // footprint bounds linear in depth (footprint_cull): x lo, x hi, z lo, z hi
@@ -100,6 +103,7 @@ struct BlConeDev {
     v3 minc;         // REV grid origin [cm]
     int nx, ny, nz;  // line length, lines along y, lines along z
     int batch;
+    float hx, hz, hb;  // gather: |dx hz - dz hx| <= hb for a pillar axis that the voxel's lines can reach
     uint64_t line0;  // first line of this grid among the launch's lines
 };
 
@@ -124,6 +128,9 @@ struct BlArgs {
     uint32_t* line_cone;        // grid (= batch) of every line, written by the interval pass
     uint32_t* counts;
     const uint32_t* tile_batch; // batch of every gather tile (nullptr: a single batch)
+    // stored lines have kLineZeros zero samples on both sides, empty lines' offset points at zeros, and
+    // the store has fewer than 2^30 samples: the gather's short form applies
+    bool zeros;
 };
 
 CCCS_HD int find_cone(const BlConeDev* __restrict__ c, int n, uint64_t line) {
@@ -169,6 +176,8 @@ CCCS_HD LineMeta line_interval(const BlArgs& a, const BlConeDev& c, const BatchD
 
 __global__ void __launch_bounds__(256) bl_interval_kernel(BlArgs a) {
     const uint64_t line = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    // what empty lines (offset 0) read; the walk writes the zeros around the others
+    if (a.zeros && line < 2 * kLineZeros) a.rev[(int64_t)line - kLineZeros] = 0.f;
     if (line >= a.nlines) return;
     const int ci = find_cone(a.cones, a.nbatch, line);
     a.line_cone[line] = (uint32_t)ci;
@@ -346,7 +355,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             const BlConeDev c = uniform_copy(pc);
             const BatchDev B = uniform_copy(pB);
             const v3 dl = mk3(c.kinv_m.m[1], c.kinv_m.m[4], c.kinv_m.m[7]);
-            const float pdx = (float)B.pd[0], pdz = (float)B.pd[2], ipdx = 1.f / pdx, ipdz = 1.f / pdz;
+            const float pdx = (float)B.pd[0], pdz = (float)B.pd[2], ipdx = B.ipd[0], ipdz = B.ipd[2];
             const float cull = B.fw + 0.05f;
             // the distance from the nearest beamlet axis in pillars (0.05 samples wider than the cull)
             const float dux = dl.x * ipdx, duz = dl.z * ipdz, cx = (cull + 0.05f) * ipdx, cz = (cull + 0.05f) * ipdz;
@@ -385,13 +394,13 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
                 }
             }
         }
-        if ((lines_in & ~with_cand) >> tid & 1ull) a.lines[my_line].len = 0;
+        if ((lines_in & ~with_cand) >> tid & 1ull) a.lines[my_line] = LineMeta{0u, 0, 0};
         __syncthreads();
         // pass A.2: exact pillar mapping and fluence-cell test of the candidates, full waves
         if (ncand > 0) {
             const BlConeDev c = uniform_copy(pc);
             const BatchDev B = uniform_copy(pB);
-            const v3 ipd = mk3(1.f / (float)B.pd[0], 1.f / (float)B.pd[1], 1.f / (float)B.pd[2]);
+            const v3 ipd = mk3(B.ipd[0], B.ipd[1], B.ipd[2]);
             for (int r = 0; r < ncand; r += 64) {
                 const bool in = r + tid < ncand;
                 const int e = in ? (int)s_cand[r + tid] : 0, k = e >> 10;
@@ -421,7 +430,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             for (int e = c0; e < c1; e += 64)
                 nfoot += (uint32_t)__popcll(__ballot(e + tid < c1 && s_cpil[e + tid] != kNoPil));
             if (nfoot == 0) {
-                if (tid == 0) a.lines[line].len = 0;
+                if (tid == 0) a.lines[line] = LineMeta{0u, 0, 0};
                 continue;
             }
             // a line's TERMA requests go to one of kSubQueues queues, chosen by its run of 64
@@ -478,7 +487,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             float* Hl = H + moff;
             int nex = 0;
             {
-                const float ipdx = 1.f / (float)B.pd[0], ipdz = 1.f / (float)B.pd[2];
+                const float ipdx = B.ipd[0], ipdz = B.ipd[2];
                 const float ux0 = lane_f(my_p0.x, k) * ipdx, uz0 = lane_f(my_p0.z, k) * ipdz;
                 const float dux = c.kinv_m.m[1] * ipdx, duz = c.kinv_m.m[7] * ipdz;
                 // (inside the pillar by 0.05 samples on each side)
@@ -504,7 +513,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             }
             const uint32_t qbase = (uint32_t)lane_i((int)qres, 0);
             if (nex == 0) {  // every sample is a wall: no dose on this line, and the reservation stays empty
-                if (tid == 0) a.lines[line].len = 0;
+                if (tid == 0) a.lines[line] = LineMeta{0u, 0, 0};
                 for (uint32_t e = (uint32_t)tid; e < nfoot; e += 64)
                     if (qbase + e < subcap) qs[qbase + e].slot = kNoSlot;
                 __syncthreads();
@@ -525,7 +534,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             int first = -1, last = -1;  // first and last listed sample that is not a wall
             uint32_t qdone = 0;
             const int tY = lane_i(my_y, k), tZ = lane_i(my_z, k);
-            const v3 ipd = mk3(1.f / (float)B.pd[0], 1.f / (float)B.pd[1], 1.f / (float)B.pd[2]);
+            const v3 ipd = mk3(B.ipd[0], B.ipd[1], B.ipd[2]);
             for (int r = 0; r < nex; r += 64) {
                 bool ok = false, need = false;
                 int j = 0, pidx = 0;
@@ -582,11 +591,8 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             // gives a wall).
             const int nlo = first < 0 ? m : (int)s_list[first], nhi = last < 0 ? -1 : (int)s_list[last];
             if (tid == 0 && (nlo > 0 || nhi < m - 1)) {
-                LineMeta t;
-                t.off = nhi < nlo ? moff : moff + (uint32_t)nlo;
-                t.i0 = nhi < nlo ? (int16_t)i0 : (int16_t)(i0 + nlo);
-                t.len = nhi < nlo ? (int16_t)0 : (int16_t)(nhi - nlo + 1);
-                a.lines[line] = t;
+                a.lines[line] = nhi < nlo ? LineMeta{0u, 0, 0}
+                                          : LineMeta{moff + (uint32_t)nlo, (int16_t)(i0 + nlo), (int16_t)(nhi - nlo + 1)};
             }
             __syncthreads();  // the next line reuses the LDS arrays
         }
@@ -790,6 +796,7 @@ __global__ void __launch_bounds__(64) bl_walk_kernel(BlArgs a, const float* __re
             }
             T[j] = ej.x >= 0.f ? sum / nphi_f : 0.f;
         }
+        if (a.zeros && tid < 2 * kLineZeros) T[tid < kLineZeros ? tid - kLineZeros : m + tid - kLineZeros] = 0.f;
         __syncthreads();  // the next line reuses the LDS arrays
     }
     }
@@ -801,26 +808,32 @@ __global__ void __launch_bounds__(64) bl_walk_kernel(BlArgs a, const float* __re
 // farthest reach of the footprint bounds, itself <= fw).  The four lines a voxel reads lie within
 // sqrt(2) of the line through it, so if that line passes farther than sqrt(2)*(gw + 1) + 0.5 from
 // the axes of the voxel's pillar and of the neighbouring pillars it touches, the fetch is zero and
-// is skipped.  Depends on pX and pZ only.
-__device__ __forceinline__ bool bl_gather_hit(const BatchDev& B, const BlConeDev& c, int pX, int pZ) {
-    if (!(B.fw < 1e29f)) return true;
+// is skipped.  Depends on pX and pZ only.  The distance times the length of the line's direction in
+// the x-z plane, (hx, hz), is a cross product; a neighbour's differs from it by a pillar's width
+// (past the grid's last pillar the test is made all the same: the fetch is zero there).
+void gather_bound(const BatchDev& B, BlConeDev& c) {
     const float wx = c.kinv_m.m[1], wz = c.kinv_m.m[7];
-    const float wn = sqrtf(wx * wx + wz * wz);
+    const float wn = std::sqrt(wx * wx + wz * wz);
+    c.hx = wx;
+    c.hz = wz;
     const float bound = 1.41421356f * (B.gw + 1.f) + 0.5f;
-    const int pix = pX / B.pd[0], piy = pZ / B.pd[2];
-    const int rx = pX - pix * B.pd[0], rz = pZ - piy * B.pd[2];
-    const int sx = rx < 2 ? -1 : (rx >= B.pd[0] - 2 ? 1 : 0);
-    const int sz = rz < 2 ? -1 : (rz >= B.pd[2] - 2 ? 1 : 0);
-    bool hit = false;
-    for (int ox = 0; ox <= (sx != 0 ? 1 : 0) && !hit; ox++)
-        for (int oz = 0; oz <= (sz != 0 ? 1 : 0) && !hit; oz++) {
-            const int qx = pix + ox * sx, qz = piy + oz * sz;
-            if (qx < 0 || qz < 0 || qx >= B.npx || qz >= B.npy || qx + qz * B.npx >= B.n) continue;
-            const float dx = (float)(pX - qx * B.pd[0]) - B.fc[0], dz = (float)(pZ - qz * B.pd[2]) - B.fc[1];
-            const float dist = wn > 1e-6f ? fabsf(dx * wz - dz * wx) / wn : sqrtf(dx * dx + dz * dz);
-            hit = dist <= bound;
-        }
-    return hit;
+    // (negative: a line along the pillars, with the voxel's own distance)
+    c.hb = !(B.fw < 1e29f) ? INFINITY : wn > 1e-6f ? bound * wn * (1.f + 1e-5f) + 1e-4f : -bound;
+}
+__device__ __forceinline__ bool bl_gather_hit(const BatchDev& B, const BlConeDev& c, int pX, int pZ) {
+    const float pdx = (float)B.pd[0], pdz = (float)B.pd[2];
+    // (exact: pX and pZ are small integers, half a step away from the multiples of the pillar)
+    const float rx = (float)pX - floorf(((float)pX + 0.5f) * B.ipd[0]) * pdx;
+    const float rz = (float)pZ - floorf(((float)pZ + 0.5f) * B.ipd[2]) * pdz;
+    const float dx = rx - B.fc[0], dz = rz - B.fc[1], cross = dx * c.hz - dz * c.hx;
+    const float sx = rx < 2.f ? -pdx : (rx >= pdx - 2.f ? pdx : 0.f);
+    const float sz = rz < 2.f ? -pdz : (rz >= pdz - 2.f ? pdz : 0.f);
+    if (c.hb < 0.f) {
+        const float mx = fminf(fabsf(dx), fabsf(dx - sx)), mz = fminf(fabsf(dz), fabsf(dz - sz));
+        return sqrtf(mx * mx + mz * mz) <= -c.hb * (1.f + 1e-5f);
+    }
+    const float nx = sx * c.hz, nz = sz * c.hx;
+    return fminf(fminf(fabsf(cross), fabsf(cross - nx)), fminf(fabsf(cross + nz), fabsf(cross - nx + nz))) <= c.hb;
 }
 
 // PackedREVtoBEVdose (nvbbRayConvolve_device.cu:427-452) for one cone direction over every batch's
@@ -833,6 +846,16 @@ __device__ __forceinline__ bool bl_gather_hit(const BatchDev& B, const BlConeDev
 // issued before any of their stores, so a lane has four fetches in flight.
 constexpr int kGatherX = 4;  // the tile's depth along pX
 constexpr int kGatherY = 4;  // pY voxels per lane
+
+// The stored line of record (off, w) at sample i, interpolated at fraction x: the clamp takes samples
+// outside the line to its zeros.  rev0 is kLineZeros samples before the store.
+__device__ __forceinline__ float line_lerp(const char* __restrict__ rev0, uint32_t off, uint32_t w, int i, float x) {
+    const int d = i - (int)(int16_t)(w & 0xffffu), len = (int)w >> 16;
+    const int at = min(max(d, -kLineZeros), len) + (int)off;  // (v_med3)
+    const pair_f32 p = *reinterpret_cast<const pair_f32*>(rev0 + (uint32_t)(at + kLineZeros) * 4u);
+    return p.x + x * (p.y - p.x);
+}
+
 __global__ void __launch_bounds__(64) bl_gather_kernel(BlArgs a, uint32_t ntiles) {
     const uint32_t tile = xcd_chunks(blockIdx.x, gridDim.x, 64);
     if (tile >= ntiles) return;
@@ -840,29 +863,60 @@ __global__ void __launch_bounds__(64) bl_gather_kernel(BlArgs a, uint32_t ntiles
     const BatchDev& B = a.batches[lo];
     const BlConeDev& c = a.cones[lo];
     const uint32_t t = tile - B.tile0;
-    const int ty = (int)(t % (uint32_t)B.tiles[0]);
-    const int tz = (int)((t / (uint32_t)B.tiles[0]) % (uint32_t)B.tiles[1]);
-    const int tx = (int)(t / ((uint32_t)B.tiles[0] * (uint32_t)B.tiles[1]));
+    const uint32_t row = B.tdiv[0] ? __umulhi(t, B.tdiv[0]) : t / (uint32_t)B.tiles[0];
+    const uint32_t plane = B.tdiv[1] ? __umulhi(row, B.tdiv[1]) : row / (uint32_t)B.tiles[1];
+    const int ty = (int)(t - row * (uint32_t)B.tiles[0]), tz = (int)(row - plane * (uint32_t)B.tiles[1]), tx = (int)plane;
     const int tid = threadIdx.x;
     const int pY0 = ty * 16 + (tid & 3), pZ = tz * 4 + ((tid >> 2) & 3), pX = tx * kGatherX + (tid >> 4);
     if (pY0 >= B.gd[1] || pZ >= B.gd[2] || pX >= B.gd[0] || !bl_gather_hit(B, c, pX, pZ)) return;
     float old[kGatherY], dc[kGatherY];
     float* dst = a.pdose + B.pdose + (size_t)pY0 + (size_t)B.gd[1] * ((size_t)pZ + (size_t)B.gd[2] * pX);
+    v3 at[kGatherY];
+    bool inner = true;
 #pragma unroll
     for (int s = 0; s < kGatherY; s++) {
         const int pY = pY0 + 4 * s;
-        dc[s] = 0.f;
-        old[s] = 0.f;
-        if (pY >= B.gd[1]) continue;
         // continuous resampling: the matrix form of rotateKernel (the Rodrigues form differs only
         // in the last bits of the fetch coordinate)
         const v3 rk = c.kfwd_m(mk3((float)pX, (float)pY, (float)pZ));
-        const v3 ri = mk3(fmaf(-c.minc.x, a.rrv.x, rk.x), fmaf(-c.minc.y, a.rrv.y, rk.y),
-                          fmaf(-c.minc.z, a.rrv.z, rk.z));
+        // (sample, line y, line z), texel centres at +0.5 (rev_fetch)
+        at[s] = mk3(fmaf(-c.minc.y, a.rrv.y, rk.y) + 0.5f - 0.5f, fmaf(-c.minc.z, a.rrv.z, rk.z) + 0.5f - 0.5f,
+                    fmaf(-c.minc.x, a.rrv.x, rk.x) + 0.5f - 0.5f);
         // the voxel's packed dose is read before the fetch so that its latency overlaps the
         // fetch's (this lane alone writes the voxel in this launch)
-        old[s] = dst[4 * s];
-        dc[s] = rev_fetch(a.lines, a.rev, c.line0, c.nx, c.ny, c.nz, ri.y + 0.5f, ri.z + 0.5f, ri.x + 0.5f);
+        old[s] = pY < B.gd[1] ? dst[4 * s] : 0.f;
+        inner = inner && (pY >= B.gd[1] || (at[s].y >= 0.f && at[s].z >= 0.f && at[s].y < (float)(c.ny - 1) &&
+                                            at[s].z < (float)(c.nz - 1)));
+    }
+    if (a.zeros && __all(inner) && c.ny < (1 << 12) && c.nz < (1 << 12)) {
+        // every voxel of the tile has its four lines inside the grid: no test on lines or samples
+        const char* m0 = reinterpret_cast<const char*>(a.lines + c.line0);
+        const char* m1 = m0 + (size_t)c.ny * sizeof(LineMeta);
+        const char* rev0 = reinterpret_cast<const char*>(a.rev - kLineZeros);
+        pair_meta q0[kGatherY], q1[kGatherY];
+#pragma unroll
+        for (int s = 0; s < kGatherY; s++) {
+            // (rows past the grid's pY range stay inside the line table: their lane's own records)
+            const float y = fminf(fmaxf(at[s].y, 0.f), (float)(c.ny - 2)), z = fminf(fmaxf(at[s].z, 0.f), (float)(c.nz - 2));
+            const uint32_t l = mad24((uint32_t)(int)z, (uint32_t)c.ny, (uint32_t)(int)y) * (uint32_t)sizeof(LineMeta);
+            q0[s] = *reinterpret_cast<const pair_meta*>(m0 + l);
+            q1[s] = *reinterpret_cast<const pair_meta*>(m1 + l);
+        }
+#pragma unroll
+        for (int s = 0; s < kGatherY; s++) {
+            const float fu = floorf(at[s].x), x = at[s].x - fu, y = at[s].y - floorf(at[s].y), z = at[s].z - floorf(at[s].z);
+            const int i = (int)fu;
+            const float t0 = line_lerp(rev0, q0[s].x, q0[s].y, i, x), t1 = line_lerp(rev0, q0[s].z, q0[s].w, i, x);
+            const float t2 = line_lerp(rev0, q1[s].x, q1[s].y, i, x), t3 = line_lerp(rev0, q1[s].z, q1[s].w, i, x);
+            const float e0 = t0 + y * (t1 - t0), e1 = t2 + y * (t3 - t2);
+            dc[s] = pY0 + 4 * s < B.gd[1] ? e0 + z * (e1 - e0) : 0.f;
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < kGatherY; s++)
+            dc[s] = pY0 + 4 * s < B.gd[1]
+                        ? rev_fetch(a.lines, a.rev, c.line0, c.nx, c.ny, c.nz, at[s].x + 0.5f, at[s].y + 0.5f, at[s].z + 0.5f)
+                        : 0.f;
     }
 #pragma unroll
     for (int s = 0; s < kGatherY; s++)
@@ -1178,7 +1232,7 @@ __global__ void __launch_bounds__(256) plain_ray_kernel(BlArgs a, float* __restr
     float d = -1e-12f, t = 0.f;
     int pidx;
     v3 inp;
-    const v3 ipd = mk3(1.f / (float)B.pd[0], 1.f / (float)B.pd[1], 1.f / (float)B.pd[2]);
+    const v3 ipd = mk3(B.ipd[0], B.ipd[1], B.ipd[2]);
     if (bl_locate(a, c, B, ipd, tX, tY, tZ, pidx, inp)) {
         const PillarRec bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
         t = point_terma(bl_terma_point(a, B, bl, inp), B.fmap, B.beam, a.spec, a.vd, a.dens, a.bhc, bl.fidx, nullptr);
@@ -1562,6 +1616,11 @@ int build_job(cccs_ctx* ctx, const std::vector<BeamPlan>& plans, const std::vect
         B.tiles[0] = (B.gd[1] + 15) / 16;
         B.tiles[1] = (B.gd[2] + 3) / 4;
         B.tiles[2] = (B.gd[0] + kGatherX - 1) / kGatherX;
+        for (int k = 0; k < 2; k++) {  // (t * (d * ceil(2^32 / d) - 2^32) < 2^32 for every t below)
+            const uint64_t d = (uint64_t)B.tiles[k], n = (uint64_t)B.tiles[0] * B.tiles[1] * B.tiles[2];
+            B.tdiv[k] = d >= 2 && n * d < (uint64_t(1) << 32) ? (uint32_t)(((uint64_t(1) << 32) + d - 1) / d) : 0u;
+        }
+        for (int k = 0; k < 3; k++) B.ipd[k] = 1.f / (float)B.pd[k];
         B.tile0 = J.tiles;
         // footprint prefilter: the beamlet axis runs along the pillar's y axis through its x/z
         // centre; a sample farther from it than half the widest divergent beamlet (at the far end
@@ -1631,6 +1690,7 @@ int build_job(cccs_ctx* ctx, const std::vector<BeamPlan>& plans, const std::vect
             c.ny = (int)rv.size[1];
             c.nz = (int)rv.size[2];
             c.batch = bi;
+            gather_bound(B, c);
             c.line0 = J.ray_lines[r];
             J.ray_lines[r] += (uint64_t)c.ny * c.nz;
             ray_rev[r] += (uint64_t)c.nx * c.ny * c.nz;
@@ -1691,8 +1751,11 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     CCCS_HIP(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, ctx->stream));
     CCCS_TRY(ctx->bl_pdose.ensure(sizeof(float) * std::max<uint64_t>(1, J.pdose)));
     CCCS_TRY(ctx->lines.ensure(line_bytes(J.max_lines)));
-    CCCS_TRY(ctx->rev.ensure(rev_bytes(J.max_rev)));
-    CCCS_TRY(ctx->bl_h.ensure(sizeof(float) * std::max<uint64_t>(1, J.max_rev)));
+    // (the zeros around every line count as samples of the store)
+    const bool zeros = J.max_rev + (uint64_t)kLineZeros * J.max_lines + 2 * kRevPad < (uint64_t(1) << 30);
+    const uint64_t max_rev = J.max_rev + (zeros ? (uint64_t)kLineZeros * J.max_lines : 0);
+    CCCS_TRY(ctx->rev.ensure(rev_bytes(max_rev)));
+    CCCS_TRY(ctx->bl_h.ensure(sizeof(float) * std::max<uint64_t>(1, max_rev)));
     CCCS_TRY(ctx->bl_qcnt.ensure(sizeof(uint32_t) * (size_t)std::max(1, nrays)));
     CCCS_TRY(ctx->h_small.ensure(sizeof(uint32_t) * kMaxRays + 64));
     // TERMA queue: footprint samples are a few percent of the stored samples; the counts are
@@ -1707,6 +1770,7 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     a.rev = ctx->rev.as<float>() + kRevPad;
     a.pdose = ctx->bl_pdose.as<float>();
     a.nbatch = nb;
+    a.zeros = zeros;
     CCCS_TRY(ctx->bl_tiles.ensure(sizeof(uint32_t) * std::max<uint32_t>(1, J.tiles)));
     hipLaunchKernelGGL(bl_tile_batch_kernel, dim3(64, (unsigned)nb), dim3(256), 0, ctx->stream, a.batches,
                        ctx->bl_tiles.as<uint32_t>());
@@ -1734,8 +1798,8 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     for (int k = 0; k < nset; k++) CCCS_TRY(set_cone[k]->ensure(sizeof(uint32_t) * std::max<uint64_t>(1, J.max_lines)));
     for (int k = 1; k < nset; k++) {
         CCCS_TRY(set_lines[k]->ensure(line_bytes(J.max_lines)));
-        CCCS_TRY(set_rev[k]->ensure(rev_bytes(J.max_rev)));
-        CCCS_TRY(set_h[k]->ensure(sizeof(float) * std::max<uint64_t>(1, J.max_rev)));
+        CCCS_TRY(set_rev[k]->ensure(rev_bytes(max_rev)));
+        CCCS_TRY(set_h[k]->ensure(sizeof(float) * std::max<uint64_t>(1, max_rev)));
     }
     for (int attempt = 0; attempt < 3; attempt++) {
         subcap = std::min<uint64_t>(subcap, 0xffffffffULL / kSubQueues);
@@ -1772,7 +1836,7 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
                 hipLaunchKernelGGL(bl_interval_kernel, dim3((unsigned)((a.nlines + 255) / 256)), dim3(256), 0,
                                    ctx->stream, a);
                 if (hipGetLastError() != hipSuccess) { rc = set_error(CCCS_EDEVICE, "interval kernel"); break; }
-                if ((rc = launch_line_scan(ctx, a.lines, a.nlines)) != CCCS_OK) break;
+                if ((rc = launch_line_scan(ctx, a.lines, a.nlines, zeros ? kLineZeros : 0)) != CCCS_OK) break;
                 uint32_t maxn = 1;
                 for (int bi = 0; bi < nb; bi++) maxn = std::max(maxn, (uint32_t)J.cones[(size_t)r * nb + bi].nx);
                 const unsigned lw = (unsigned)std::min<uint64_t>(a.nlines, (uint64_t)ctx->sched.bl_sample_waves);
