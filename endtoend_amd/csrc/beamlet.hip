@@ -315,8 +315,6 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
     __shared__ uint32_t s_foot[kMaxLine / 32];    // one line's footprint samples
     __shared__ uint64_t s_exact[kMaxLine / 64];   // one line's samples on s_list
     __shared__ uint32_t s_pil[kPillarBits / 32];  // pillars with footprint samples on the line
-    __shared__ uint16_t s_rank[kPillarBits / 32]; // footprint pillars in the words before each word
-    __shared__ PillarRec s_rec[kStagePillars];    // their beamlet data, in pillar order
     constexpr uint16_t kNoPil = 0xffff;
     const int tid = threadIdx.x;
     const uint64_t lt = (1ull << tid) - 1ull;
@@ -456,26 +454,6 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
                 if (track) atomicOr(&s_pil[pil >> 5], 1u << (pil & 31u));
             }
             __syncthreads();
-            // the beamlet data of the footprint pillars into LDS (its loads overlap pass B.1): word w of
-            // s_pil is lane w's (w < 64) or lane w-64's; a pillar's slot is its rank among the set bits
-            if (track) {
-                uint32_t slot = 0;
-                for (int h = 0; h < 2; h++) {
-                    uint32_t w = s_pil[tid + 64 * h];
-                    uint32_t first = 0;
-                    for (uint64_t nz = __ballot(w != 0u); nz; nz &= nz - 1ull) {
-                        const int l = __builtin_ctzll(nz);
-                        if (tid == l) first = slot;
-                        slot += (uint32_t)__builtin_popcount((uint32_t)lane_i((int)w, l));
-                    }
-                    if (w) s_rank[tid + 64 * h] = (uint16_t)first;
-                    for (; w != 0u && first < (uint32_t)kStagePillars; first++) {
-                        const int b = __ffs(w) - 1;
-                        w &= w - 1u;
-                        s_rec[first] = pillar_rec(a.beamlets[B.beamlet0 + (tid + 64 * h) * 32 + b]);
-                    }
-                }
-            }
             // pass B.1: a pillar without footprint samples on this line gets no dose on it, so its
             // samples act as walls (a pillar crossing is exactly one segment of the walk).  Samples
             // confidently in such pillars (or outside the grid's pillars) are walls; the others go to
@@ -545,11 +523,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
                     if (bl_locate(a, c, B, ipd, i0 + j, tY, tZ, pidx, inp) &&
                         (!track || ((s_pil[pidx >> 5] >> (pidx & 31)) & 1u))) {
                         ok = true;
-                        const uint32_t slot = track ? (uint32_t)s_rank[pidx >> 5] +
-                                                          (uint32_t)__popc(s_pil[pidx >> 5] & ((1u << (pidx & 31)) - 1u))
-                                                    : (uint32_t)kStagePillars;
-                        if (slot < (uint32_t)kStagePillars) bl = s_rec[slot];
-                        else bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
+                        bl = pillar_rec(a.beamlets[B.beamlet0 + pidx]);
                         need = (s_foot[j >> 5] >> (j & 31)) & 1u;
                     }
                 }
