@@ -623,11 +623,18 @@ __device__ __forceinline__ double bperm_f64(int addr, double v) {
 // prefix sums (FP64), so each destination visits just the footprint samples of its segment, in the
 // reference's walk order, instead of every sample.
 //
-// Dynamic LDS: for up to maxn samples {half step, TERMA} (8 B), the radiological centre (FP64),
-// the segment bounds and the footprint list (3 x 2 B).
+// A line has some 40 samples and 4 footprint samples, so the time is the instructions around the
+// walks: the segment bounds and the place in the footprint list come from one ballot of the walls and
+// one of the footprint samples per 64 samples (bit scans instead of three wave scans and a search), and
+// a footprint sample next to the one before it takes its inner cumulative value from that one.
+//
+// Dynamic LDS: for up to maxn samples the radiological centre (FP64), {half step, TERMA} (8 B) and the
+// footprint list (2 B).
 __global__ void __launch_bounds__(64) bl_walk_kernel(BlArgs a, const float* __restrict__ H, int maxn, int len_lo) {
     extern __shared__ double s_dyn[];
     __shared__ float4 sTab[2][kMaxRadii];
+    __shared__ uint64_t s_wall[kMaxLine / 64], s_foot[kMaxLine / 64];  // walls and footprint samples
+    __shared__ int s_first[kMaxLine / 64];                             // footprint samples before each 64
     const int tid = threadIdx.x;
     const int nr = a.nradii;
     if (tid < nr) {
@@ -642,13 +649,13 @@ __global__ void __launch_bounds__(64) bl_walk_kernel(BlArgs a, const float* __re
     }
     double* sC = s_dyn;
     float2* sL = reinterpret_cast<float2*>(s_dyn + maxn);
-    short* s_lo = reinterpret_cast<short*>(sL + maxn);
-    short* s_hi = s_lo + maxn;
-    short* s_fp = s_hi + maxn;
+    short* s_fp = reinterpret_cast<short*>(sL + maxn);
     __syncthreads();
     const float rmax = sTab[0][nr - 1].w, rlast = sTab[0][nr - 2].w;
     const float nphi_f = (float)a.nphi;
     uint32_t iters = 0;
+    // a wave walks lines base, base + G, base + 2G, ..., so that neighbouring waves work on neighbouring
+    // lines at the same time, and takes the records of its next 64 lines at once, one per lane
     const uint64_t G = gridDim.x;
     for (uint64_t base = xcd_remap(blockIdx.x, gridDim.x); base < a.nlines; base += 64 * G) {
     LineMeta mine{};
@@ -656,119 +663,127 @@ __global__ void __launch_bounds__(64) bl_walk_kernel(BlArgs a, const float* __re
     // empty lines and other launches' lines are skipped here
     uint64_t todo = __ballot(mine.len >= len_lo && mine.len <= maxn);
     while (todo) {
-        const int kl = __ffsll((unsigned long long)todo) - 1;
+        const int kl = __builtin_ctzll(todo);
         todo &= todo - 1ull;
-        LineMeta meta = line_of_lane(mine, kl);
-        meta.off = __builtin_amdgcn_readfirstlane(meta.off);  // uniform: scalar registers
-        const int m = __builtin_amdgcn_readfirstlane((int)meta.len);
+        const uint32_t moff = (uint32_t)lane_i((int)mine.off, kl);
+        const int m = lane_i((int)mine.len, kl);
         // the scans' lane arithmetic is redone per line from an opaque lane id: hoisted out of
         // the line loop, it held some 20 VGPRs for the whole kernel
         int ln = tid;
         __asm__ volatile("" : "+v"(ln));
-        float* T = a.rev + meta.off;
-        const float* Hl = H + meta.off;
-        for (int j = tid; j < m; j += 64) sL[j] = make_float2(Hl[j], T[j]);
+        const uint64_t upto = (2ull << ln) - 1ull, below = upto >> 1;  // lanes up to and below this one
+        float* T = a.rev + moff;
+        const float* Hl = H + moff;
+        int nfoot = 0;
+        for (int c = 0; 64 * c < m; c++) {
+            const int j = 64 * c + tid;
+            float2 e = make_float2(-1.f, 0.f);  // (behind the line: a wall)
+            if (j < m) {
+                e = make_float2(Hl[j], T[j]);
+                sL[j] = e;
+            }
+            const uint64_t W = __ballot(e.x < 0.f), F = __ballot(e.y != 0.f);
+            if (e.y != 0.f) s_fp[nfoot + __popcll(F & below)] = (short)j;
+            if (tid == 0) {
+                s_wall[c] = W;
+                s_foot[c] = F;
+                s_first[c] = nfoot;
+            }
+            nfoot += __popcll(F);
+        }
         __syncthreads();
-        // chunked scans: radiological prefix, nearest walls, footprint list
+        // radiological centres: a lane sums its run of samples, a wave scan carries the sums over
         const int per = (m + 63) / 64;
         const int ca = min(m, tid * per), cb = min(m, ca + per);
         double csum = 0.0;
-        int last_wall = -1, first_wall = m, nfp = 0;
         for (int k = ca; k < cb; k++) {
-            const float2 e = sL[k];
-            if (e.x < 0.f) last_wall = k;
-            else csum += 2.0 * (double)e.x;
-            if (e.y != 0.f) nfp++;
+            const float h = sL[k].x;
+            if (!(h < 0.f)) csum += 2.0 * (double)h;
         }
-        for (int k = cb - 1; k >= ca; k--)
-            if (sL[k].x < 0.f) first_wall = k;
         double pc = csum;
-        int pre = last_wall, suf = first_wall, pf = nfp;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int iu = max(ln - o, 0) << 2, id = min(ln + o, 63) << 2;
-            const double uc = bperm_f64(iu, pc);
-            const int up = __builtin_amdgcn_ds_bpermute(iu, pre);
-            const int uf = __builtin_amdgcn_ds_bpermute(iu, pf);
-            const int dn = __builtin_amdgcn_ds_bpermute(id, suf);
-            if (tid >= o) { pc += uc; pre = max(pre, up); pf += uf; }
-            if (tid + o < 64) suf = min(suf, dn);
+        for (int o = 1; o < 64 && o * per < m; o <<= 1) {  // (lanes behind the line's end add nothing)
+            const double uc = bperm_f64(max(ln - o, 0) << 2, pc);
+            if (tid >= o) pc += uc;
         }
         double cacc = pc - csum;
-        int left = __builtin_amdgcn_ds_bpermute(max(ln - 1, 0) << 2, pre);
-        int right = __builtin_amdgcn_ds_bpermute(min(ln + 1, 63) << 2, suf);
-        int fpos = pf - nfp;
-        const int nfoot = __builtin_amdgcn_readlane(pf, 63);
-        if (tid == 0) left = -1;
-        if (tid == 63) right = m;
         for (int k = ca; k < cb; k++) {
-            const float2 e = sL[k];
-            const double hh = e.x < 0.f ? 0.0 : (double)e.x;
+            const float h = sL[k].x;
+            const double hh = h < 0.f ? 0.0 : (double)h;
             sC[k] = cacc + hh;
             cacc += 2.0 * hh;
-            if (e.x < 0.f) left = k;
-            s_lo[k] = (short)(left + 1);
-            if (e.y != 0.f) s_fp[fpos++] = (short)k;
-        }
-        for (int k = cb - 1; k >= ca; k--) {
-            if (sL[k].x < 0.f) right = k;
-            s_hi[k] = (short)(right - 1);
         }
         __syncthreads();
-        for (int base = 0; base < m; base += 64) {
-            const int j = base + tid;
-            if (j >= m) break;
-            const float2 ej = sL[j];
-            float sum = 0.f;
-            if (ej.x >= 0.f && nfoot > 0) {
-                const int slo = s_lo[j], shi = s_hi[j];
-                const double cj = sC[j];
-                int lo = 0, hi = nfoot;  // first footprint entry >= j
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (s_fp[mid] < j) lo = mid + 1; else hi = mid;
+        int wall_before = -1;  // last wall of the samples before the current 64
+        for (int c = 0; 64 * c < m; c++) {
+            const int j = 64 * c + tid;
+            const uint64_t W = s_wall[c], F = s_foot[c];
+            int wall_behind = m;  // first wall of the samples behind the current 64
+            for (int n = c + 1; 64 * n < m; n++)
+                if (const uint64_t v = s_wall[n]) {
+                    wall_behind = 64 * n + __builtin_ctzll(v);
+                    break;
                 }
-                const int p = lo;
-                const float r0 = ej.x;
-                for (int d = 0; d < 2; d++) {
-                    const float4* tab = sTab[d];
-                    int s = 0;
-                    float4 iv = tab[0];
-                    if (!(r0 <= rmax)) continue;
-                    sum += kc_at(r0, tab, nr, s, iv) * ej.y;  // the self sample
-                    iters++;
-                    if (r0 > rlast) continue;
-                    if (d == 0) {
-                        for (int q = p - 1; q >= 0; q--) {
-                            const int k = s_fp[q];
-                            if (k < slo) break;
-                            const double ck = sC[k];
-                            const float rp = k + 1 == j ? r0 : (float)(cj - sC[k + 1]);
-                            if (rp > rlast) break;
-                            const float rk = (float)(cj - ck);
-                            if (rk > rmax) break;
-                            const float kp = kc_at(rp, tab, nr, s, iv);
-                            const float kk = kc_at(rk, tab, nr, s, iv);
-                            sum += (kk - kp) * sL[k].y;
-                            iters++;
-                        }
-                    } else {
-                        for (int q = (p < nfoot && s_fp[p] == j) ? p + 1 : p; q < nfoot; q++) {
-                            const int k = s_fp[q];
-                            if (k > shi) break;
-                            const double ck = sC[k];
-                            const float rp = k - 1 == j ? r0 : (float)(sC[k - 1] - cj);
-                            if (rp > rlast) break;
-                            const float rk = (float)(ck - cj);
-                            if (rk > rmax) break;
-                            const float kp = kc_at(rp, tab, nr, s, iv);
-                            const float kk = kc_at(rk, tab, nr, s, iv);
-                            sum += (kk - kp) * sL[k].y;
-                            iters++;
+            if (j < m) {
+                const float2 ej = sL[j];
+                float sum = 0.f;
+                if (ej.x >= 0.f && nfoot > 0) {
+                    const uint64_t wl = W & below, wr = W & ~upto;
+                    const int slo = (wl ? 64 * c + 63 - __builtin_clzll(wl) : wall_before) + 1;
+                    const int shi = (wr ? 64 * c + __builtin_ctzll(wr) : wall_behind) - 1;
+                    const double cj = sC[j];
+                    const int p = s_first[c] + __popcll(F & below);  // first footprint entry >= j
+                    const float r0 = ej.x;
+                    for (int d = 0; d < 2; d++) {
+                        const float4* tab = sTab[d];
+                        int s = 0;
+                        float4 iv = tab[0];
+                        if (!(r0 <= rmax)) continue;
+                        float klast = kc_at(r0, tab, nr, s, iv);
+                        sum += klast * ej.y;  // the self sample
+                        iters++;
+                        if (r0 > rlast) continue;
+                        float rl = r0;  // distance to the outer face of the last sample, whose value is klast
+                        int kl2 = j;
+                        if (d == 0) {
+                            for (int q = p - 1; q >= 0; q--) {
+                                const int k = s_fp[q];
+                                if (k < slo) break;
+                                const bool next = k + 1 == kl2;
+                                if (!next) rl = (float)(cj - sC[k + 1]);
+                                if (rl > rlast) break;
+                                const float rk = (float)(cj - sC[k]);
+                                if (rk > rmax) break;
+                                if (!next) klast = kc_at(rl, tab, nr, s, iv);
+                                const float kk = kc_at(rk, tab, nr, s, iv);
+                                sum += (kk - klast) * sL[k].y;
+                                klast = kk;
+                                rl = rk;
+                                kl2 = k;
+                                iters++;
+                            }
+                        } else {
+                            for (int q = p + (int)(F >> ln & 1ull); q < nfoot; q++) {
+                                const int k = s_fp[q];
+                                if (k > shi) break;
+                                const bool next = k - 1 == kl2;
+                                if (!next) rl = (float)(sC[k - 1] - cj);
+                                if (rl > rlast) break;
+                                const float rk = (float)(sC[k] - cj);
+                                if (rk > rmax) break;
+                                if (!next) klast = kc_at(rl, tab, nr, s, iv);
+                                const float kk = kc_at(rk, tab, nr, s, iv);
+                                sum += (kk - klast) * sL[k].y;
+                                klast = kk;
+                                rl = rk;
+                                kl2 = k;
+                                iters++;
+                            }
                         }
                     }
                 }
+                T[j] = ej.x >= 0.f ? sum / nphi_f : 0.f;
             }
-            T[j] = ej.x >= 0.f ? sum / nphi_f : 0.f;
+            if (W) wall_before = 64 * c + 63 - __builtin_clzll(W);
         }
         if (a.zeros && tid < 2 * kLineZeros) T[tid < kLineZeros ? tid - kLineZeros : m + tid - kLineZeros] = 0.f;
         __syncthreads();  // the next line reuses the LDS arrays
@@ -1838,7 +1853,7 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
                 int nclass = 0;
                 for (uint32_t hi = split; split > 0 && hi < maxn && nclass < 11; hi *= 2) bounds[nclass++] = hi;
                 bounds[nclass++] = maxn;
-                const size_t per = sizeof(double) + sizeof(float2) + 3 * sizeof(short);
+                const size_t per = sizeof(double) + sizeof(float2) + sizeof(short);
                 uint32_t* wc = prof_counter(ctx, (size_t)nclass * ww);
                 int tw = prof_begin(ctx, K_BL_WALK);
                 for (int ci = 0; ci < nclass; ci++) {

@@ -32,13 +32,13 @@ __device__ __forceinline__ uint32_t xcd_chunks(uint32_t b, uint32_t nb, uint32_t
     return s0 + (r % 8) * chunk + r / 8;
 }
 
-// Sums one uint32 per thread over the workgroup (LDS tree, <= 256 threads) into part[slot].
 // Sums one uint32 per lane over a 64-lane workgroup into part[slot] (no LDS).
 __device__ __forceinline__ void wave_count(uint32_t v, uint32_t* __restrict__ part, size_t slot) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if (threadIdx.x == 0) part[slot] = v;
 }
 
+// Sums one uint32 per thread over the workgroup (LDS tree, <= 256 threads) into part[slot].
 __device__ __forceinline__ void block_count(uint32_t v, uint32_t* __restrict__ part, size_t slot) {
     __shared__ uint32_t s_cnt[256];
     const int t = threadIdx.x + threadIdx.y * blockDim.x + threadIdx.z * blockDim.x * blockDim.y;
@@ -68,20 +68,6 @@ struct LineMeta {
     int16_t len;   // stored samples
 };
 static_assert(sizeof(LineMeta) == 8, "line table entries are 8 bytes");
-
-// Persistent per-line kernels walk lines base, base + G, base + 2G, ... (G = grid size), so that
-// neighbouring waves work on neighbouring lines at the same time.  A wave loads the records of
-// its next 64 lines at once, one per lane (lane k: line base + k*G), and takes each from its lane:
-// one round trip per 64 lines instead of one per line, and lines it skips cost no memory access.
-__device__ __forceinline__ LineMeta line_of_lane(const LineMeta& m, int lane) {
-    const uint32_t w = (uint32_t)(uint16_t)m.i0 | ((uint32_t)(uint16_t)m.len << 16);
-    const uint32_t ow = (uint32_t)__shfl((int)w, lane, 64);
-    LineMeta r;
-    r.off = (uint32_t)__shfl((int)m.off, lane, 64);
-    r.i0 = (int16_t)(ow & 0xffffu);
-    r.len = (int16_t)(ow >> 16);
-    return r;
-}
 
 // Entries kept before and after a line table and a REV store, so that a pair load at an end stays
 // inside the allocation (128 bytes of the store: lines keep their alignment).
