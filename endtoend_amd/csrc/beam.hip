@@ -21,6 +21,7 @@
 #include <cstdio>
 #include <cstring>
 #include <array>
+#include <functional>
 #include <limits>
 #include <map>
 #include <memory>
@@ -235,6 +236,38 @@ __global__ void __launch_bounds__(256) crop_partial_kernel(const float* __restri
     if (t < 7) part[(size_t)blockIdx.x * 8 + t] = s[t][0];
 }
 
+// Small boxes in one workgroup: the launch that combines the partials costs more than the pass.
+constexpr size_t kCropSmall = size_t(1) << 16;  // voxels
+__global__ void __launch_bounds__(1024) crop_small_kernel(const float* __restrict__ terma, int bx, int by, int bz, Rot2 rot,
+                                                          float* __restrict__ out) {
+    __shared__ float s[16][7];
+    float v[7] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX, 0.f};
+    const uint32_t n = (uint32_t)bx * (uint32_t)by * (uint32_t)bz, t = threadIdx.x;
+#pragma unroll 4
+    for (uint32_t i = t; i < n; i += 1024) {
+        if (terma[i] == 0.f) continue;
+        const uint32_t row = i / (uint32_t)bx, z = row / (uint32_t)by;
+        const v3 b = rot_fwd(rot, mk3((float)(i - row * (uint32_t)bx), (float)(row - z * (uint32_t)by), (float)z));
+        v[0] = fminf(v[0], b.x); v[1] = fminf(v[1], b.y); v[2] = fminf(v[2], b.z);
+        v[3] = fmaxf(v[3], b.x); v[4] = fmaxf(v[4], b.y); v[5] = fmaxf(v[5], b.z);
+        v[6] += 1.f;
+    }
+#pragma unroll
+    for (int q = 0; q < 7; q++)
+        for (int o = 32; o > 0; o >>= 1) {
+            const float u = __shfl_xor(v[q], o, 64);
+            v[q] = q < 3 ? fminf(v[q], u) : q < 6 ? fmaxf(v[q], u) : v[q] + u;
+        }
+    if ((t & 63) == 0)
+        for (int q = 0; q < 7; q++) s[t >> 6][q] = v[q];
+    __syncthreads();
+    if (t < 7) {
+        float r = s[0][t];
+        for (int w = 1; w < 16; w++) r = t < 3 ? fminf(r, s[w][t]) : t < 6 ? fmaxf(r, s[w][t]) : r + s[w][t];
+        out[t] = r;
+    }
+}
+
 __global__ void __launch_bounds__(256) crop_final_kernel(const float* __restrict__ part, int nblocks, float* __restrict__ out) {
     __shared__ float s[7][256];
     const int t = threadIdx.x;
@@ -285,6 +318,7 @@ struct ConeArgs {
     int ramp_min;             // valid segments at least this long use the segment-sum walk
     int maxn;                 // longest stored line of this launch (LDS sizing)
     const ConeLine* list;     // the lines of this launch, one workgroup each
+    const uint32_t* count;    // their number, where the launch's grid is a bound (or nullptr)
     VolDesc vd;
     m33 binv;                 // PVCS <- BEV rotation (index units)
     v3 off;                   // (bevStart - start) / voxel
@@ -548,22 +582,6 @@ inline size_t cone_lds_bytes(uint32_t maxn, bool ramp) {
     return 2 * sizeof(double) * n1 + sizeof(float) * nc + sizeof(float2) * maxn + std::max(sizeof(uint16_t) * (2 * (size_t)maxn + 4), rows);
 }
 
-// Pass 1 of the cone pipeline: the stored interval of every REV line (offsets come from a scan).
-__global__ void __launch_bounds__(256) line_interval_kernel(ConeArgs a) {
-    const uint64_t line = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (line >= a.nlines) return;
-    const int q = cone_of_line(a.cones, a.ncones, line);
-    const ConeDev& c = a.cones[q];
-    const uint64_t l = line - c.line0;
-    int i0, i1;
-    line_interval(a, c, (int)(l % (uint64_t)c.ny), (int)(l / (uint64_t)c.ny), i0, i1);
-    LineMeta m;
-    m.i0 = (int16_t)i0;
-    m.len = (int16_t)(i1 - i0);
-    m.off = 0;
-    a.lines[line] = m;
-}
-
 // v moved across lanes by a DPP control; lanes outside the rows of the mask or without a source get 0.
 template <int kCtrl, int kRows>
 __device__ __forceinline__ double dpp_f64(double v) {
@@ -679,6 +697,7 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     __shared__ int s_red[NW][3];
     __shared__ uint32_t s_cnt[NW];
     const uint32_t slot = xcd_chunks(blockIdx.x, gridDim.x, 64);
+    if (a.count && slot >= *a.count) return;
     const uniform_ptr<ConeLine> en = as_uniform(a.list) + slot;
     const uint32_t off = en->off, tyz = en->tyz, seg = en->seg, last = en->last;
     const int i0 = (int)(seg & 1023u), m = (int)(seg >> 10 & 1023u) + 1, ja = (int)(seg >> 20);
@@ -1352,7 +1371,9 @@ int context_scratch(cccs_ctx* ctx, BeamScratch& S) {
     return CCCS_OK;
 }
 
-int run_crop(BeamScratch& S, const float* d_terma, const cccs_beam& b, float* red_host) {
+// `before_wait` (may be empty) enqueues work that needs the TERMA alone, before the host waits.
+int run_crop(BeamScratch& S, const float* d_terma, const cccs_beam& b, float* red_host,
+             const std::function<int()>& before_wait) {
     cccs_ctx* ctx = S.ctx;
     float* part = nullptr;
     const size_t used = S.used;
@@ -1362,33 +1383,43 @@ int run_crop(BeamScratch& S, const float* d_terma, const cccs_beam& b, float* re
     const cccs_problem& p = ctx->prob;
     size_t n = bbox_voxels(ctx);
     int blocks = (int)std::min<size_t>(kCropBlocks, (n + 255) / 256);
+    // the result goes straight to pinned host memory (the fixed array's caller has none)
+    float* out = S.arena ? part + kCropBlocks * 8 : S.host_small;
     int tok = prof_begin(ctx, K_CROP);
+    if (n <= kCropSmall) {
+        hipLaunchKernelGGL(crop_small_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_terma, (int)p.bbox_size[0],
+                           (int)p.bbox_size[1], (int)p.bbox_size[2], rot, out);
+    } else {
     hipLaunchKernelGGL(crop_partial_kernel, dim3(blocks), dim3(256), 0, ctx->stream, d_terma, (int)p.bbox_size[0],
                        (int)p.bbox_size[1], (int)p.bbox_size[2], rot, part);
-    hipLaunchKernelGGL(crop_final_kernel, dim3(1), dim3(256), 0, ctx->stream, part, blocks, part + kCropBlocks * 8);
+        hipLaunchKernelGGL(crop_final_kernel, dim3(1), dim3(256), 0, ctx->stream, part, blocks, out);
+    }
     prof_end(ctx, tok, 4.0 * (double)n, 0.0, n);
     CCCS_HIP(hipGetLastError());
-    CCCS_HIP(hipMemcpyAsync(S.host_small, part + kCropBlocks * 8, 7 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+    if (S.arena)
+        CCCS_HIP(hipMemcpyAsync(S.host_small, out, 7 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+    if (before_wait) CCCS_TRY(before_wait());
     CCCS_HIP(hipStreamSynchronize(ctx->stream));
     std::memcpy(red_host, S.host_small, 7 * sizeof(float));
     return CCCS_OK;
 }
 
-// Everything after TERMA: geometry, cones, PVCS accumulation into d_dose.
-// ---- per-class line lists -----------------------------------------------------------------------
+// ---- line table and per-class line lists ---------------------------------------------------------
 // The cone kernel runs one launch per stored-length class (LDS sized for the class's longest line).
 // Each launch takes the list of its own lines, in line order, so that no workgroup is spent on an
-// empty line or on a line of another class.  Three passes: per-block class counts, one block that
-// turns them into list offsets (class by class), and a stable scatter of the line indices.
+// empty line or on a line of another class.  Three passes: the stored interval of every line with the
+// stored samples and class counts of every 1024 lines, one workgroup that turns those into offsets
+// (seven passes, of 3 to 23 us each, when intervals, offsets and lists had their own), and the
+// lines' offsets and list entries.
 constexpr int kClassBlock = 1024;
+constexpr int kClassCols = kConeClasses + 1;  // lines per class, stored samples
 
 struct ClassArgs {
-    const LineMeta* lines;
-    uint64_t n;
     int hi[kConeClasses];  // longest stored line of each class (ascending)
     int ncls;
-    uint32_t* bcnt;        // [blocks][kConeClasses]: counts, then the blocks' list offsets
-    uint32_t* tot;         // [kConeClasses]: lines per class
+    uint32_t* bcnt;        // [blocks][kClassCols]: counts, then the blocks' offsets (classes: in their list)
+    uint32_t* tot;         // [kClassCols]: lines per class, stored samples
+    uint32_t* host;        // the same in pinned host memory, or nullptr
     ConeLine* list;        // the lines' entries, class by class
     uint32_t* counts;      // profiling: the slots of empty lines are zeroed here (or nullptr)
 };
@@ -1400,56 +1431,91 @@ __device__ __forceinline__ int class_of_line(const ClassArgs& a, int len) {
     return a.ncls - 1;
 }
 
-__global__ void __launch_bounds__(kClassBlock) class_count_kernel(ClassArgs a) {
-    __shared__ uint32_t s[kClassBlock / 64][kConeClasses];
+__device__ __forceinline__ uint32_t wave_incl_u32(uint32_t v) {
+    const int lane = threadIdx.x & 63;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
+__global__ void __launch_bounds__(kClassBlock) line_interval_kernel(ConeArgs ca, ClassArgs a) {
+    __shared__ uint32_t s[kClassBlock / 64][kClassCols];
     const uint64_t i = (uint64_t)blockIdx.x * kClassBlock + threadIdx.x;
-    const int cls = i < a.n ? class_of_line(a, a.lines[i].len) : -1;
-    if (a.counts && i < a.n && cls < 0) a.counts[i] = 0;
+    int len = 0;
+    if (i < ca.nlines) {
+        const ConeDev& c = ca.cones[cone_of_line(ca.cones, ca.ncones, i)];
+        const uint32_t l = (uint32_t)(i - c.line0), tz = l / (uint32_t)c.ny, ty = l - tz * (uint32_t)c.ny;
+        int i0, i1;
+        line_interval(ca, c, (int)ty, (int)tz, i0, i1);
+        len = (int)(int16_t)(i1 - i0);
+        ca.lines[i] = LineMeta{0u, (int16_t)i0, (int16_t)len};
+    }
+    const int cls = class_of_line(a, len);
+    if (a.counts && i < ca.nlines && cls < 0) a.counts[i] = 0;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int c = 0; c < kConeClasses; c++) {
         const uint64_t m = __ballot(cls == c);
         if (lane == 0) s[w][c] = (uint32_t)__popcll(m);
     }
+    uint32_t sum = (uint32_t)len;
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if (lane == 0) s[w][kConeClasses] = sum;
     __syncthreads();
-    if (threadIdx.x < kConeClasses) {
+    if (threadIdx.x < kClassCols) {
         uint32_t t = 0;
         for (int q = 0; q < kClassBlock / 64; q++) t += s[q][threadIdx.x];
-        a.bcnt[(size_t)blockIdx.x * kConeClasses + threadIdx.x] = t;
+        a.bcnt[(size_t)blockIdx.x * kClassCols + threadIdx.x] = t;
     }
 }
 
-// One workgroup: exclusive scan of the block counts of each class, the classes one after another.
+// One workgroup: exclusive scan of the block counts, column by column.
 __global__ void __launch_bounds__(kClassBlock) class_scan_kernel(ClassArgs a, uint32_t nb) {
-    __shared__ uint32_t s[kClassBlock];
-    const int t = threadIdx.x;
-    uint32_t base = 0;
-    for (int c = 0; c < kConeClasses; c++) {
-        const uint32_t start = base;
-        for (uint32_t b0 = 0; b0 < nb; b0 += kClassBlock) {
-            const uint32_t b = b0 + t;
-            const uint32_t v = b < nb ? a.bcnt[(size_t)b * kConeClasses + c] : 0u;
-            s[t] = v;
-            __syncthreads();
-            for (int off = 1; off < kClassBlock; off <<= 1) {
-                const uint32_t add = t >= off ? s[t - off] : 0u;
-                __syncthreads();
-                s[t] += add;
-                __syncthreads();
-            }
-            if (b < nb) a.bcnt[(size_t)b * kConeClasses + c] = base + s[t] - v;
-            base += s[kClassBlock - 1];
-            __syncthreads();
+    __shared__ uint32_t s[kClassCols][kClassBlock / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    uint32_t carry[kClassCols] = {};
+    for (uint32_t b0 = 0; b0 < nb; b0 += kClassBlock) {
+        uint32_t* row = a.bcnt + (size_t)(b0 + t) * kClassCols;
+        uint32_t v[kClassCols], inc[kClassCols];
+#pragma unroll
+        for (int q = 0; q < kClassCols; q++) v[q] = b0 + t < nb ? row[q] : 0u;
+#pragma unroll
+        for (int q = 0; q < kClassCols; q++) {
+            inc[q] = wave_incl_u32(v[q]);
+            if (lane == 63) s[q][w] = inc[q];
         }
-        if (t == 0) a.tot[c] = base - start;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kClassCols; q++) {
+            uint32_t before = 0, total = 0;
+            for (int k = 0; k < kClassBlock / 64; k++) {
+                before += k < w ? s[q][k] : 0u;
+                total += s[q][k];
+            }
+            if (b0 + t < nb) row[q] = carry[q] + before + inc[q] - v[q];
+            carry[q] += total;
+        }
+        __syncthreads();
     }
+#pragma unroll
+    for (int q = 0; q < kClassCols; q++)
+        if (t == q) {
+            a.tot[q] = carry[q];
+            if (a.host) a.host[q] = carry[q];
+        }
 }
 
 __global__ void __launch_bounds__(kClassBlock) class_scatter_kernel(ClassArgs a, ConeArgs ca) {
-    __shared__ uint32_t s[kClassBlock / 64][kConeClasses];
+    __shared__ uint32_t s[kClassBlock / 64][kClassCols];
     const uint64_t i = (uint64_t)blockIdx.x * kClassBlock + threadIdx.x;
-    const int cls = i < a.n ? class_of_line(a, a.lines[i].len) : -1;
+    LineMeta meta{};
+    if (i < ca.nlines) meta = ca.lines[i];
+    const int cls = class_of_line(a, meta.len);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint64_t below = (uint64_t(1) << lane) - 1;
+    const uint32_t inc = wave_incl_u32((uint32_t)meta.len);
+    if (lane == 63) s[w][kConeClasses] = inc;
     uint32_t rank = 0;
     for (int c = 0; c < kConeClasses; c++) {
         const uint64_t m = __ballot(cls == c);
@@ -1457,10 +1523,14 @@ __global__ void __launch_bounds__(kClassBlock) class_scatter_kernel(ClassArgs a,
         if (cls == c) rank = (uint32_t)__popcll(m & below);
     }
     __syncthreads();
+    const uint32_t* block = a.bcnt + (size_t)blockIdx.x * kClassCols;
+    meta.off = block[kConeClasses] + inc - (uint32_t)meta.len;
+    for (int q = 0; q < w; q++) meta.off += s[q][kConeClasses];
+    if (i < ca.nlines) ca.lines[i] = meta;
     if (cls >= 0) {
-        uint32_t off = a.bcnt[(size_t)blockIdx.x * kConeClasses + cls] + rank;
+        uint32_t off = block[cls] + rank;
+        for (int c = 0; c < cls; c++) off += a.tot[c];
         for (int q = 0; q < w; q++) off += s[q][cls];
-        const LineMeta meta = a.lines[i];
         const int q = cone_of_line(ca.cones, ca.ncones, i);
         const ConeDev& c = ca.cones[q];
         const uint32_t l = (uint32_t)(i - c.line0), tz = l / (uint32_t)c.ny, ty = l - tz * (uint32_t)c.ny;
@@ -1483,10 +1553,27 @@ void launch_cone(int threads, dim3 grid, size_t lds, hipStream_t st, const ConeA
     }
 }
 
+// Everything after TERMA: geometry, cones, PVCS accumulation into d_dose.
 int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d_dose, BeamGeom* gout) {
     cccs_ctx* ctx = S.ctx;
     float red[7];
-    CCCS_TRY(run_crop(S, d_terma, b, red));
+    const size_t nvox = vol_voxels(ctx);
+    float2* d_dt = nullptr;
+    auto pack = [&]() -> int {
+        const cccs_problem& p = ctx->prob;
+        dim3 blk(64, 4, 1), grd((unsigned)((p.size[0] + 63) / 64), (unsigned)((p.size[1] + 3) / 4), p.size[2]);
+        hipLaunchKernelGGL(pack_dt_kernel, grd, blk, 0, ctx->stream, (const float*)ctx->d_dens, d_terma,
+                           (int)p.size[0], (int)p.size[1], (int)p.size[2], (int)p.bbox_start[0],
+                           (int)p.bbox_start[1], (int)p.bbox_start[2], (int)p.bbox_size[0], (int)p.bbox_size[1],
+                           (int)p.bbox_size[2], d_dt);
+        CCCS_HIP(hipGetLastError());
+        return CCCS_OK;
+    };
+    // the interleaved volume needs the TERMA alone: it is packed while the host waits for the crop box
+    // (the fixed array's pieces keep their order)
+    const bool pack_early = d_dose && !S.arena && nvox < (size_t(1) << 31);
+    if (pack_early) CCCS_TRY(S.get(ctx->dt, nvox, &d_dt));
+    CCCS_TRY(run_crop(S, d_terma, b, red, pack_early ? std::function<int()>(pack) : std::function<int()>()));
     BeamGeom g;
     CCCS_TRY(beam_geometry(ctx, b, red, g));
     if (gout) *gout = g;
@@ -1537,10 +1624,8 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     CCCS_HIP(hipMemcpyAsync(d_cones, hc, sizeof(ConeDev) * g.nrays, hipMemcpyHostToDevice, ctx->stream));
     // the host staging may be the caller's stack (no-allocation entry point): the copy completes first
     if (S.arena) CCCS_HIP(hipStreamSynchronize(ctx->stream));
-    const size_t nvox = vol_voxels(ctx);
     if (nvox >= (size_t(1) << 31)) return set_error(CCCS_EGEOM, "CT grid beyond 2^31 voxels");
-    float2* d_dt = nullptr;
-    CCCS_TRY(S.get(ctx->dt, nvox, &d_dt));
+    if (!pack_early) CCCS_TRY(S.get(ctx->dt, nvox, &d_dt));
     ConeArgs ca;
     ca.list = nullptr;
     ca.dt = d_dt;
@@ -1563,21 +1648,7 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     ca.bb0 = ldu3(p.bbox_start);
     ca.bb1 = ca.bb0 + ldu3(p.bbox_size);
     if (g.total_lines == 0) return CCCS_OK;
-    {
-        dim3 blk(64, 4, 1), grd((unsigned)((p.size[0] + 63) / 64), (unsigned)((p.size[1] + 3) / 4), p.size[2]);
-        hipLaunchKernelGGL(pack_dt_kernel, grd, blk, 0, ctx->stream, (const float*)ctx->d_dens, d_terma,
-                           (int)p.size[0], (int)p.size[1], (int)p.size[2], (int)p.bbox_start[0],
-                           (int)p.bbox_start[1], (int)p.bbox_start[2], (int)p.bbox_size[0], (int)p.bbox_size[1],
-                           (int)p.bbox_size[2], d_dt);
-        CCCS_HIP(hipGetLastError());
-    }
-    // pass 1: stored interval of every line, then offsets into the compact store
-    hipLaunchKernelGGL(line_interval_kernel, dim3((unsigned)((g.total_lines + 255) / 256)), dim3(256), 0, ctx->stream,
-                       ca);
-    CCCS_HIP(hipGetLastError());
-    uint32_t* d_scan = nullptr;
-    CCCS_TRY(S.get(ctx->scan, line_scan_words(g.total_lines), &d_scan));
-    CCCS_TRY(launch_line_scan(ctx, ca.lines, g.total_lines, d_scan, 0));
+    if (!pack_early) CCCS_TRY(pack());
     // stored-length classes: one launch each, with LDS for the class's longest line, so that the
     // many short lines are not held to the occupancy of the longest
     uint32_t maxn = 1;
@@ -1593,29 +1664,37 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     }
     ca.counts = prof_counter(ctx, g.total_lines);
     ClassArgs cl;
-    cl.lines = ca.lines;
-    cl.n = g.total_lines;
     for (int c = 0; c < kConeClasses; c++) cl.hi[c] = c < ncls ? cls_hi[c] : 0;
     cl.ncls = ncls;
     cl.counts = ca.counts;
     const uint64_t ncb = (g.total_lines + kClassBlock - 1) / kClassBlock;
-    CCCS_TRY(S.get(ctx->cls_cnt, (size_t)ncb * kConeClasses + kConeClasses, &cl.bcnt));
-    cl.tot = cl.bcnt + (size_t)ncb * kConeClasses;
+    CCCS_TRY(S.get(ctx->cls_cnt, (size_t)ncb * kClassCols + kClassCols, &cl.bcnt));
+    cl.tot = cl.bcnt + (size_t)ncb * kClassCols;
+    // The launches and the store are sized from the totals on the host.  Small beams take the bounds
+    // instead (empty workgroups and some megabytes cost less than the wait: 32^3 water beam 115 against
+    // 124 us);
+    // their cone launch reads its count on the device.
+    const bool wait = S.arena || ctx->prof.on || ncls != 1 || g.total_lines > 32768 || g.total_rev > (uint64_t(1) << 24);
+    uint32_t* totals = reinterpret_cast<uint32_t*>(S.host_small + 8);
+    cl.host = wait && !S.arena ? totals : nullptr;
     CCCS_TRY(S.get(ctx->cls_list, g.total_lines, &cl.list));
-    hipLaunchKernelGGL(class_count_kernel, dim3((unsigned)ncb), dim3(kClassBlock), 0, ctx->stream, cl);
+    hipLaunchKernelGGL(line_interval_kernel, dim3((unsigned)ncb), dim3(kClassBlock), 0, ctx->stream, ca, cl);
     hipLaunchKernelGGL(class_scan_kernel, dim3(1), dim3(kClassBlock), 0, ctx->stream, cl, (uint32_t)ncb);
     hipLaunchKernelGGL(class_scatter_kernel, dim3((unsigned)ncb), dim3(kClassBlock), 0, ctx->stream, cl, ca);
     CCCS_HIP(hipGetLastError());
-    CCCS_HIP(hipMemcpyAsync(S.host_small, ca.lines + (g.total_lines - 1), sizeof(LineMeta), hipMemcpyDeviceToHost,
-                            ctx->stream));
-    CCCS_HIP(hipMemcpyAsync(S.host_small + 4, cl.tot, sizeof(uint32_t) * kConeClasses, hipMemcpyDeviceToHost,
-                            ctx->stream));
-    CCCS_HIP(hipStreamSynchronize(ctx->stream));
-    LineMeta last;
-    std::memcpy(&last, S.host_small, sizeof(LineMeta));
-    uint32_t cls_n[kConeClasses];
-    std::memcpy(cls_n, S.host_small + 4, sizeof(cls_n));
-    const uint64_t stored = (uint64_t)last.off + (uint64_t)last.len;
+    uint32_t cls_n[kConeClasses] = {};
+    uint64_t stored = g.total_rev;
+    ca.count = nullptr;
+    if (wait) {
+        if (S.arena)
+            CCCS_HIP(hipMemcpyAsync(totals, cl.tot, sizeof(uint32_t) * kClassCols, hipMemcpyDeviceToHost, ctx->stream));
+        CCCS_HIP(hipStreamSynchronize(ctx->stream));
+        std::memcpy(cls_n, totals, sizeof(cls_n));
+        stored = totals[kConeClasses];
+    } else {
+        cls_n[0] = (uint32_t)g.total_lines;
+        ca.count = cl.tot;
+    }
     CCCS_TRY(S.get(ctx->rev, stored + 2 * kRevPad, &ca.rev));
     ca.rev += kRevPad;
     // pass 2: per-line resample + walks into the compact store, one workgroup per listed line

@@ -120,7 +120,7 @@ struct Schedule {
     // streams' Siddon, walk and gather waves run beside it (its own 5-wave occupancy would take
     // every register of the SIMD)
     int bl_sample_waves = 3072;
-    int bl_walk_waves = 32768;
+    int bl_walk_waves = 16384;
     // device memory of one beamlet job [GiB]: batches join a job while its packed grids, output
     // bounds and per-direction buffers fit; fewer, larger jobs drain the direction pipeline less often
     int bl_job_gb = 12;
