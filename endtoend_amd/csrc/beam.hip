@@ -1431,15 +1431,6 @@ __device__ __forceinline__ int class_of_line(const ClassArgs& a, int len) {
     return a.ncls - 1;
 }
 
-__device__ __forceinline__ uint32_t wave_incl_u32(uint32_t v) {
-    const int lane = threadIdx.x & 63;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(v, o, 64);
-        if (lane >= o) v += u;
-    }
-    return v;
-}
-
 __global__ void __launch_bounds__(kClassBlock) line_interval_kernel(ConeArgs ca, ClassArgs a) {
     __shared__ uint32_t s[kClassBlock / 64][kClassCols];
     const uint64_t i = (uint64_t)blockIdx.x * kClassBlock + threadIdx.x;
@@ -1672,8 +1663,7 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     cl.tot = cl.bcnt + (size_t)ncb * kClassCols;
     // The launches and the store are sized from the totals on the host.  Small beams take the bounds
     // instead (empty workgroups and some megabytes cost less than the wait: 32^3 water beam 115 against
-    // 124 us);
-    // their cone launch reads its count on the device.
+    // 124 us); their cone launch reads its count on the device.
     const bool wait = S.arena || ctx->prof.on || ncls != 1 || g.total_lines > 32768 || g.total_rev > (uint64_t(1) << 24);
     uint32_t* totals = reinterpret_cast<uint32_t*>(S.host_small + 8);
     cl.host = wait && !S.arena ? totals : nullptr;

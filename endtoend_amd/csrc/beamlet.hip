@@ -126,6 +126,7 @@ struct BlArgs {
     SpecDev spec;
     float bhc;
     uint32_t* line_cone;        // grid (= batch) of every line, written by the interval pass
+    uint32_t* blocks;           // stored samples of every kLineBlock lines, or their exclusive scan
     uint32_t* counts;
     const uint32_t* tile_batch; // batch of every gather tile (nullptr: a single batch)
     // stored lines have kLineZeros zero samples on both sides, empty lines' offset points at zeros, and
@@ -174,14 +175,57 @@ CCCS_HD LineMeta line_interval(const BlArgs& a, const BlConeDev& c, const BatchD
     return m;
 }
 
-__global__ void __launch_bounds__(256) bl_interval_kernel(BlArgs a) {
-    const uint64_t line = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+// Offsets into the REV store: every stored line is preceded by kLineZeros samples of its own where
+// BlArgs::zeros holds, and empty lines get offset 0 there.  The interval pass leaves offsets within
+// blocks of kLineBlock lines and the blocks' totals; the sample stage, which reads every record first
+// and writes it back, adds the blocks before, from the totals themselves up to 64 blocks and from their
+// scan beyond (three scan launches of their own cost a 32^3 job a tenth of its time).
+constexpr int kLineBlock = 256;
+constexpr uint32_t kWaveBlocks = 64;  // blocks whose totals one wave scans
+
+__global__ void __launch_bounds__(kLineBlock) bl_interval_kernel(BlArgs a) {
+    __shared__ uint32_t s_w[kLineBlock / 64];
+    const uint64_t line = (uint64_t)blockIdx.x * kLineBlock + threadIdx.x;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     // what empty lines (offset 0) read; the walk writes the zeros around the others
     if (a.zeros && line < 2 * kLineZeros) a.rev[(int64_t)line - kLineZeros] = 0.f;
-    if (line >= a.nlines) return;
-    const int ci = find_cone(a.cones, a.nbatch, line);
-    a.line_cone[line] = (uint32_t)ci;
-    a.lines[line] = line_interval(a, a.cones[ci], a.batches[ci], line);
+    LineMeta m{};
+    int ci = 0;
+    if (line < a.nlines) {
+        ci = find_cone(a.cones, a.nbatch, line);
+        m = line_interval(a, a.cones[ci], a.batches[ci], line);
+    }
+    const uint32_t pad = a.zeros && m.len > 0 ? (uint32_t)kLineZeros : 0u, take = (uint32_t)m.len + pad;
+    const uint32_t inc = wave_incl_u32(take);
+    if (lane == 63) s_w[w] = inc;
+    __syncthreads();
+    uint32_t before = inc - take;
+    for (int q = 0; q < w; q++) before += s_w[q];
+    m.off = m.len > 0 ? before + pad : 0u;
+    if (line < a.nlines) {
+        a.line_cone[line] = (uint32_t)ci;
+        a.lines[line] = m;
+    }
+    if (threadIdx.x == kLineBlock - 1) a.blocks[blockIdx.x] = before + take;
+}
+
+// One workgroup: exclusive scan of the block totals.
+__global__ void __launch_bounds__(kLineBlock) bl_block_scan_kernel(uint32_t* __restrict__ blocks, uint32_t nb) {
+    __shared__ uint32_t s_w[kLineBlock / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (uint32_t b0 = 0; b0 < nb; b0 += kLineBlock) {
+        const uint32_t b = b0 + threadIdx.x, v = b < nb ? blocks[b] : 0u, inc = wave_incl_u32(v);
+        if (lane == 63) s_w[w] = inc;
+        __syncthreads();
+        uint32_t before = carry;
+        for (int q = 0; q < kLineBlock / 64; q++) {
+            before += q < w ? s_w[q] : 0u;
+            carry += s_w[q];
+        }
+        if (b < nb) blocks[b] = before + inc - v;
+        __syncthreads();
+    }
 }
 
 // fmodf(x, y) for 0 <= x < 2^24 and a positive integer y <= 2^20: n*y is exact, x - n*y is exact,
@@ -325,6 +369,10 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
     // this lane's line
     const uint64_t my_line = base + (uint64_t)tid * G;
     LineMeta mine{};
+    // (the totals of up to kWaveBlocks blocks are scanned here)
+    const uint32_t nblocks = (uint32_t)((a.nlines + kLineBlock - 1) / kLineBlock);
+    uint32_t total = (uint32_t)tid < nblocks && nblocks <= kWaveBlocks ? a.blocks[tid] : 0u;
+    total = wave_incl_u32(total) - total;
     int my_ci = 0, my_y = 0, my_z = 0;
     v3 my_p0 = mk3(0.f, 0.f, 0.f);
     if (my_line < a.nlines) {
@@ -340,6 +388,12 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
         my_p0 = c.kinv_m(mk3(fmaf(c.minc.x, a.rrv.x, (float)my_z), c.minc.y * a.rrv.y,
                              fmaf(c.minc.z, a.rrv.z, (float)my_y))) + 0.5f;
         if (mine.len > 0) stored += (uint32_t)mine.len;  // summed over the wave's lanes by wave_count
+    }
+    {
+        const uint32_t b = (uint32_t)(my_line / kLineBlock);
+        const uint32_t before = nblocks <= kWaveBlocks ? (uint32_t)__shfl((int)total, (int)(b & 63u), 64)
+                                                       : (mine.len > 0 ? a.blocks[b] : 0u);
+        mine.off += before;
     }
     uint64_t todo = __ballot(mine.len > 0);
     while (todo) {
@@ -564,7 +618,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
             // skip them (the gather reads samples outside a line's interval as zero, the dose the walk
             // gives a wall).
             const int nlo = first < 0 ? m : (int)s_list[first], nhi = last < 0 ? -1 : (int)s_list[last];
-            if (tid == 0 && (nlo > 0 || nhi < m - 1)) {
+            if (tid == 0) {
                 a.lines[line] = nhi < nlo ? LineMeta{0u, 0, 0}
                                           : LineMeta{moff + (uint32_t)nlo, (int16_t)(i0 + nlo), (int16_t)(nhi - nlo + 1)};
             }
@@ -1822,10 +1876,13 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
             float* H = set_h[k]->as<float>();
             TermaReq* q = set_q[k]->as<TermaReq>();
             do {
-                hipLaunchKernelGGL(bl_interval_kernel, dim3((unsigned)((a.nlines + 255) / 256)), dim3(256), 0,
-                                   ctx->stream, a);
+                const uint32_t nblocks = (uint32_t)((a.nlines + kLineBlock - 1) / kLineBlock);
+                if ((rc = ctx->scan.ensure(sizeof(uint32_t) * nblocks)) != CCCS_OK) break;
+                a.blocks = ctx->scan.as<uint32_t>();
+                hipLaunchKernelGGL(bl_interval_kernel, dim3(nblocks), dim3(kLineBlock), 0, ctx->stream, a);
+                if (nblocks > kWaveBlocks)
+                    hipLaunchKernelGGL(bl_block_scan_kernel, dim3(1), dim3(kLineBlock), 0, ctx->stream, a.blocks, nblocks);
                 if (hipGetLastError() != hipSuccess) { rc = set_error(CCCS_EDEVICE, "interval kernel"); break; }
-                if ((rc = launch_line_scan(ctx, a.lines, a.nlines, zeros ? kLineZeros : 0)) != CCCS_OK) break;
                 uint32_t maxn = 1;
                 for (int bi = 0; bi < nb; bi++) maxn = std::max(maxn, (uint32_t)J.cones[(size_t)r * nb + bi].nx);
                 const unsigned lw = (unsigned)std::min<uint64_t>(a.nlines, (uint64_t)ctx->sched.bl_sample_waves);

@@ -140,73 +140,6 @@ int set_error(int code, const std::string& msg) {
 void clear_error() { g_last_error.clear(); }
 
 
-// ---- line-table scan ---------------------------------------------------------------------------
-constexpr int kScanBlock = 1024;
-
-__device__ __forceinline__ uint32_t block_inclusive_scan(uint32_t v, uint32_t* s) {
-    const int t = threadIdx.x;
-    s[t] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanBlock; off <<= 1) {
-        uint32_t add = t >= off ? s[t - off] : 0u;
-        __syncthreads();
-        s[t] += add;
-        __syncthreads();
-    }
-    return s[t];
-}
-
-__global__ void __launch_bounds__(kScanBlock) line_scan_local(LineMeta* __restrict__ meta, uint64_t n,
-                                                            uint32_t* __restrict__ bsum, uint32_t pad) {
-    __shared__ uint32_t s[kScanBlock];
-    const uint64_t i = (uint64_t)blockIdx.x * kScanBlock + threadIdx.x;
-    const uint32_t len = i < n ? (uint32_t)meta[i].len : 0u, take = len ? len + pad : 0u;
-    const uint32_t inc = block_inclusive_scan(take, s);
-    if (i < n) meta[i].off = inc - take + (len ? pad : 0u);
-    if (threadIdx.x == kScanBlock - 1) bsum[blockIdx.x] = inc;
-}
-
-__global__ void __launch_bounds__(kScanBlock) line_scan_blocks(uint32_t* __restrict__ bsum, uint32_t nb) {
-    __shared__ uint32_t s[kScanBlock];
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < nb; base += kScanBlock) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < nb ? bsum[i] : 0u;
-        const uint32_t inc = block_inclusive_scan(v, s);
-        if (i < nb) bsum[i] = carry + inc - v;
-        carry += s[kScanBlock - 1];
-        __syncthreads();
-    }
-}
-
-__global__ void __launch_bounds__(kScanBlock) line_scan_add(LineMeta* __restrict__ meta, uint64_t n,
-                                                          const uint32_t* __restrict__ bsum, uint32_t pad) {
-    const uint64_t i = (uint64_t)blockIdx.x * kScanBlock + threadIdx.x;
-    if (i < n) meta[i].off = pad && meta[i].len == 0 ? 0u : meta[i].off + bsum[blockIdx.x];
-}
-
-size_t line_scan_words(uint64_t n) { return (size_t)((n + kScanBlock - 1) / kScanBlock); }
-
-int launch_line_scan(cccs_ctx* c, LineMeta* meta, uint64_t n, int pad) {
-    if (n == 0) return CCCS_OK;
-    CCCS_TRY(c->scan.ensure(sizeof(uint32_t) * line_scan_words(n)));
-    return launch_line_scan(c, meta, n, c->scan.as<uint32_t>(), pad);
-}
-
-int launch_line_scan(cccs_ctx* c, LineMeta* meta, uint64_t n, uint32_t* bsum, int pad) {
-    if (n == 0) return CCCS_OK;
-    const uint64_t nb = line_scan_words(n);
-    if (nb > 0xffffffffULL) return set_error(CCCS_EGEOM, "too many REV lines");
-    hipLaunchKernelGGL(line_scan_local, dim3((unsigned)nb), dim3(kScanBlock), 0, c->stream, meta, n, bsum,
-                       (uint32_t)pad);
-    hipLaunchKernelGGL(line_scan_blocks, dim3(1), dim3(kScanBlock), 0, c->stream, bsum, (uint32_t)nb);
-    hipLaunchKernelGGL(line_scan_add, dim3((unsigned)nb), dim3(kScanBlock), 0, c->stream, meta, n,
-                       (const uint32_t*)bsum, (uint32_t)pad);
-    CCCS_HIP(hipGetLastError());
-    return CCCS_OK;
-}
-
-
 }  // namespace cccs
 
 using namespace cccs;

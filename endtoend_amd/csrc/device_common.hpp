@@ -60,6 +60,16 @@ __device__ __forceinline__ uniform_ptr<T> as_uniform(const T* p) {
     return (uniform_ptr<T>)p;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave.
+__device__ __forceinline__ uint32_t wave_incl_u32(uint32_t v) {
+    const int lane = threadIdx.x & 63;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
 // One REV line of a cone grid in the compact store: samples [i0, i0 + len) of the line are kept at
 // rev[off ...]; every other sample of the line is zero.
 struct LineMeta {
