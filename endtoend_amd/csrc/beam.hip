@@ -1158,28 +1158,44 @@ __global__ void __launch_bounds__(64 * kSubRays) projection_kernel(const float* 
 // ---- fluence-map convolution (the FCBB lateral step; no reference source) --------------------
 // out[y][x] = sum_j sum_i K[j][i] * F[y - (j - kh/2)][x - (i - kw/2)], zero outside the map, the
 // terms added j outer, i inner.  One lane per output of a 16x16 tile; the tile plus its halo and
-// the kernel sit in LDS.
+// the kernel sit in LDS.  The sum is one chain per lane, in order, so a row of the kernel is unrolled
+// (KW taps, every odd width up to 31): its LDS reads are under way together instead of one round trip
+// per tap (20 maps of 64x64, 15x15 kernel: 12.8 -> 7.9 us).
 constexpr int kConvTile = 16, kConvMaxK = 31;
 
+template <int KW>
 __global__ void __launch_bounds__(256) fluence_conv_kernel(const float* __restrict__ f, int w, int h,
-                                                           const float* __restrict__ k, int kw, int kh,
-                                                           float* __restrict__ out) {
+                                                           const float* __restrict__ k, int kh, float* __restrict__ out) {
+    constexpr int kw = KW;
     __shared__ float s_k[kConvMaxK * kConvMaxK];
-    __shared__ float s_f[(kConvTile + kConvMaxK - 1) * (kConvTile + kConvMaxK - 1)];
+    // rows 48 apart: a wave's four rows of 16 outputs then read 64 different banks
+    constexpr int stride = 48;
+    static_assert(kConvTile + kConvMaxK - 1 <= stride, "row of the tile");
+    __shared__ float s_f[(kConvTile + kConvMaxK - 1) * stride];
     const int map = blockIdx.z;
     const float* F = f + (size_t)map * w * h;
     const int x0 = blockIdx.x * kConvTile, y0 = blockIdx.y * kConvTile;
     const int rx = kw / 2, ry = kh / 2;
     const int sw = kConvTile + kw - 1, sh = kConvTile + kh - 1;
     const int tid = threadIdx.x;
-    for (int q = tid; q < kw * kh; q += 256) s_k[q] = k[q];
     // s_f[v][u] = F[y0 + ry - v][x0 + rx - u]: the flipped window, so output (tx, ty) reads
-    // s_f[ty + j][tx + i] for kernel tap (i, j)
-    for (int q = tid; q < sw * sh; q += 256) {
-        const int u = q % sw, v = q / sw;
-        const int xx = x0 + (kConvTile - 1) - u + rx, yy = y0 + (kConvTile - 1) - v + ry;
-        s_f[q] = (xx >= 0 && yy >= 0 && xx < w && yy < h) ? F[(size_t)yy * w + xx] : 0.f;
+    // s_f[ty + j][tx + i] for kernel tap (i, j); four loads of a lane are under way together, with the
+    // kernel's
+    const float k0 = tid < kw * kh ? k[tid] : 0.f;
+    for (int q0 = 0; q0 < sw * sh; q0 += 4 * 256) {
+        float r[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int q = q0 + 256 * e + tid, v = q / sw, u = q - v * sw;
+            const int xx = x0 + (kConvTile - 1) - u + rx, yy = y0 + (kConvTile - 1) - v + ry;
+            r[e] = (q < sw * sh && xx >= 0 && yy >= 0 && xx < w && yy < h) ? F[(size_t)yy * w + xx] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (const int q = q0 + 256 * e + tid; q < sw * sh) s_f[q / sw * stride + q % sw] = r[e];
     }
+    if (tid < kw * kh) s_k[tid] = k0;
+    for (int q = 256 + tid; q < kw * kh; q += 256) s_k[q] = k[q];
     __syncthreads();
     const int tx = tid % kConvTile, ty = tid / kConvTile;
     const int x = x0 + tx, y = y0 + ty;
@@ -1187,9 +1203,25 @@ __global__ void __launch_bounds__(256) fluence_conv_kernel(const float* __restri
     // output (x, y) needs F[y - j + ry][x - i + rx] = s_f[(kConvTile-1-ty) + j][(kConvTile-1-tx) + i]
     const int bu = kConvTile - 1 - tx, bv = kConvTile - 1 - ty;
     float acc = 0.f;
-    for (int j = 0; j < kh; j++)
-        for (int i = 0; i < kw; i++) acc += s_k[j * kw + i] * s_f[(bv + j) * sw + bu + i];
+    for (int j = 0; j < kh; j++) {
+        float a[KW], b[KW];
+#pragma unroll
+        for (int i = 0; i < KW; i++) {
+            a[i] = s_k[j * kw + i];
+            b[i] = s_f[(bv + j) * stride + bu + i];
+        }
+#pragma unroll
+        for (int i = 0; i < KW; i++) acc += a[i] * b[i];
+    }
     out[(size_t)map * w * h + (size_t)y * w + x] = acc;
+}
+
+template <int KW>
+void launch_conv(int kw, dim3 grid, hipStream_t st, const float* f, int w, int h, const float* k, int kh, float* out) {
+    if constexpr (KW <= kConvMaxK) {
+        if (kw == KW) hipLaunchKernelGGL(fluence_conv_kernel<KW>, grid, dim3(256), 0, st, f, w, h, k, kh, out);
+        else launch_conv<KW + 2>(kw, grid, st, f, w, h, k, kh, out);
+    }
 }
 
 __global__ void add_kernel(float* __restrict__ dst, const float* __restrict__ src, size_t n) {
@@ -2142,8 +2174,7 @@ extern "C" int cccs_fluence_convolve(cccs_ctx* ctx, const float* fluence, int nm
     CCCS_HIP(hipMemcpy(kb.p, kernel, sizeof(float) * (size_t)kw * kh, hipMemcpyHostToDevice));
     const dim3 grid((unsigned)((width + kConvTile - 1) / kConvTile), (unsigned)((height + kConvTile - 1) / kConvTile),
                     (unsigned)nmaps);
-    hipLaunchKernelGGL(fluence_conv_kernel, grid, dim3(256), 0, ctx->stream, (const float*)fb.as<float>(), width, height,
-                       (const float*)kb.as<float>(), kw, kh, ob.as<float>());
+    launch_conv<1>(kw, grid, ctx->stream, fb.as<float>(), width, height, kb.as<float>(), kh, ob.as<float>());
     CCCS_HIP(hipGetLastError());
     CCCS_HIP(hipStreamSynchronize(ctx->stream));
     CCCS_HIP(hipMemcpy(out, ob.p, sizeof(float) * n, hipMemcpyDeviceToHost));
