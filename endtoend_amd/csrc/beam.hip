@@ -73,6 +73,8 @@ struct TermaArgs {
     int ss;                  // supersampling factor
     float bhc;
     int beamletnum;
+    int depth, far_first;     // axis along which the beam runs mostly; start at its high end
+    float field2;             // squared tangent of a cone around the fluence map (infinite: unknown)
     uint32_t* counts;         // per-block Siddon step counts (profiling) or nullptr
 };
 
@@ -86,14 +88,36 @@ CCCS_HD v3 terma_point(const TermaArgs& a, int X, int Y, int Z) {
 // march runs inside the field only, a part of the box, so the workgroups have to be small along x for
 // their waves to be full or empty, and rows of them go to the XCDs in turn: with 64x4x1 workgroups
 // dealt out one by one, a box of 4 or 8 workgroups along x left whole XCDs without field.  Thorax
-// beam at 54 degrees 1133 -> 395 us, 128^3 water beam 217 -> 116 us.
+// beam at 54 degrees 1133 -> 395 us, 128^3 water beam 217 -> 116 us.  A ray is a serial chain as long as
+// its voxel is deep, so the deepest planes along the beam's main axis start first and the short
+// rays fill the end; workgroups with and without field mix, so at most kTermaResident share a CU and
+// the rest go where one ends.  Those two and the cheap test of the field below: thorax at 54, 90 and 3
+// degrees 400, 220 and 243 -> 380, 176 and 182 us, 128^3 water 118 -> 95 us (without the bound 102;
+// five a CU: 398, 196, 215 and 83).
+constexpr int kTermaResident = 6;
 __device__ __forceinline__ void terma_voxel(const TermaArgs& a, int& X, int& Y, int& Z) {
-    const uint32_t nx = (uint32_t)(a.bx + 15) / 16, ny = (uint32_t)(a.by + 3) / 4;
-    const uint32_t t = xcd_chunks(blockIdx.x, gridDim.x, nx), r = t / nx;
+    const uint32_t nx = (uint32_t)(a.bx + 15) / 16, ny = (uint32_t)(a.by + 3) / 4, nz = (uint32_t)(a.bz + 3) / 4;
+    const uint32_t inner = a.depth == 0 ? ny : nx, middle = a.depth == 2 ? ny : nz;
+    const uint32_t t = xcd_chunks(blockIdx.x, gridDim.x, inner), r = t / inner;
+    // (the rows turn from plane to plane, or a multiple of 8 rows would keep each on one XCD)
+    const uint32_t i = t - r * inner, w0 = r / middle, m0 = r - w0 * middle + (middle >= 8 ? 5 * w0 & 7u : 0u);
+    const uint32_t m = m0 >= middle ? m0 - middle : m0;
+    const uint32_t outer = a.depth == 0 ? nx : a.depth == 1 ? ny : nz, o = a.far_first ? outer - 1 - w0 : w0;
+    const uint32_t bx = a.depth == 0 ? o : i, by = a.depth == 0 ? i : a.depth == 1 ? o : m, bz = a.depth == 2 ? o : m;
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    X = (int)(t - r * nx) * 16 + w * 4 + (l & 3);
-    Y = (int)(r % ny) * 4 + ((l >> 2) & 3);
-    Z = (int)(r / ny) * 4 + (l >> 4);
+    X = (int)bx * 16 + w * 4 + (l & 3);
+    Y = (int)by * 4 + ((l >> 2) & 3);
+    Z = (int)bz * 4 + (l >> 4);
+}
+// Point certainly outside the fluence map: farther from the beam's axis than the map's corners (by
+// 0.5 %).  Most voxels of the box are, and the exact cell takes 200 instructions more.  (A point level
+// with the source is left to the exact cell.)
+__device__ __forceinline__ bool outside_field(const TermaArgs& a, v3 p) {
+    const v3 d = p - a.beam.src;
+    const float along = dot3(d, a.beam.dir_n), a2 = along * along;
+    const v3 r = d - along * a.beam.dir_n;
+    const float r2 = dot3(r, r);
+    return r2 > a.field2 * a2 && a2 > 1e-6f * r2;
 }
 inline uint64_t terma_blocks(const TermaArgs& a) {
     return (uint64_t)((a.bx + 15) / 16) * (uint64_t)((a.by + 3) / 4) * (uint64_t)((a.bz + 3) / 4);
@@ -103,6 +127,8 @@ inline uint64_t terma_blocks(const TermaArgs& a) {
 // (the rpl-only march: same crossings and segments as cudaSiddon, fetch coordinates formed with
 // reciprocal voxel sizes); neighbouring lanes follow near-parallel rays, so the density taps stay
 // in L1/L2.
+// Supersampling and the profiling counts have instances of their own: together they took 81 registers.
+template <bool kSuper, bool kCount>
 __global__ void __launch_bounds__(256) terma_kernel(TermaArgs a) {
     int X, Y, Z;
     terma_voxel(a, X, Y, Z);
@@ -110,38 +136,32 @@ __global__ void __launch_bounds__(256) terma_kernel(TermaArgs a) {
     uint32_t steps = 0;
     float acc = 0.f;
     const v3 ivox = mk3(1.f / a.vd.voxel.x, 1.f / a.vd.voxel.y, 1.f / a.vd.voxel.z);
+    int it = 0;
+    int* const iters = kCount ? &it : nullptr;
     if (!in) {
-    } else if (a.ss > 1) {
+    } else if (kSuper) {
         // supersampled: sub-voxel centres, summed in sub-voxel order then averaged
         const int nsub = a.ss * a.ss * a.ss;
         v3 subsz = mk3(a.vd.voxel.x / (float)a.ss, a.vd.voxel.y / (float)a.ss, a.vd.voxel.z / (float)a.ss);
-        acc = 0.f;
         for (int s = 0; s < nsub; s++) {
             int sx = s % a.ss, sy = (s / a.ss) % a.ss, sz = s / (a.ss * a.ss);
             v3 p = mk3(a.vd.start.x + ((float)a.ox + X - 0.5f) * a.vd.voxel.x + (sx + 0.5f) * subsz.x,
                        a.vd.start.y + ((float)a.oy + Y - 0.5f) * a.vd.voxel.y + (sy + 0.5f) * subsz.y,
                        a.vd.start.z + ((float)a.oz + Z - 0.5f) * a.vd.voxel.z + (sz + 0.5f) * subsz.z);
-            int it = 0;
-            acc += point_terma_rpl(p, a.fmap, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, a.beamletnum, &it);
-            steps += (uint32_t)it;
+            acc += point_terma_rpl(p, a.fmap, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, a.beamletnum, iters);
+            if (kCount) steps += (uint32_t)it;
         }
         acc /= (float)nsub;
     } else {
         // fluence times the unit-fluence TERMA (the Siddon march only inside the field), the order
         // in which a resident unit-TERMA grid of the same source gives the same value
         const v3 p = terma_point(a, X, Y, Z);
-        const float fl = point_fluence(p, a.fmap, a.beam, a.beamletnum);
-        if (!(fl > 0.f)) {
-        } else if (a.counts) {
-            int it = 0;
-            acc = fl * unit_point_terma(p, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, &it);
-            steps = (uint32_t)it;
-        } else {
-            acc = fl * unit_point_terma(p, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, nullptr);
-        }
+        const float fl = outside_field(a, p) ? 0.f : point_fluence(p, a.fmap, a.beam, a.beamletnum);
+        if (fl > 0.f) acc = fl * unit_point_terma(p, a.beam, a.spec, a.vd, ivox, a.dens, a.bhc, iters);
+        if (kCount) steps = (uint32_t)it;
     }
     if (in) a.terma[(size_t)X + (size_t)a.bx * ((size_t)Y + (size_t)a.by * Z)] = acc;
-    if (a.counts) block_count(steps, a.counts, blockIdx.x);
+    if (kCount) block_count(steps, a.counts, blockIdx.x);
 }
 
 // Unit-fluence TERMA of every calc_bbox voxel (the march runs for every voxel): one beam source's
@@ -162,7 +182,8 @@ __global__ void __launch_bounds__(256) terma_from_unit_kernel(TermaArgs a, const
     const int Z = blockIdx.z;
     if (X >= a.bx || Y >= a.by || Z >= a.bz) return;
     const size_t v = (size_t)X + (size_t)a.bx * ((size_t)Y + (size_t)a.by * Z);
-    const float fl = point_fluence(terma_point(a, X, Y, Z), a.fmap, a.beam, a.beamletnum);
+    const v3 p = terma_point(a, X, Y, Z);
+    const float fl = outside_field(a, p) ? 0.f : point_fluence(p, a.fmap, a.beam, a.beamletnum);
     a.terma[v] = fl > 0.f ? fl * unit[v] : 0.f;
 }
 
@@ -1254,6 +1275,18 @@ TermaArgs terma_args(cccs_ctx* ctx, const cccs_beam& b, const float* d_fmap, flo
     a.bhc = ctx->prob.beamhard_correct;
     a.beamletnum = beamletnum;
     a.counts = nullptr;
+    const v3 dir = a.beam.iso - a.beam.src;
+    const float dc[3] = {dir.x, dir.y, dir.z};
+    a.depth = 2;
+    for (int k = 1; k >= 0; k--)
+        if (std::fabs(dc[k]) > std::fabs(dc[a.depth])) a.depth = k;
+    a.far_first = dc[a.depth] > 0.f;
+    // the map's cone, where the beam's direction is the y axis of its frame as for beams made here
+    const v3 y = rot2(a.beam.beam_fwd, a.beam.dir_n);
+    const float hx = 0.5f * (float)a.beam.fmx * a.beam.bsx, hz = 0.5f * (float)a.beam.fmy * a.beam.bsy;
+    a.field2 = std::fabs(y.x) < 1e-3f && std::fabs(y.z) < 1e-3f && a.beam.iso_dist > 0.f
+                   ? 1.01f * (hx * hx + hz * hz) / (a.beam.iso_dist * a.beam.iso_dist)
+                   : INFINITY;
     return a;
 }
 
@@ -1265,7 +1298,11 @@ int launch_terma(cccs_ctx* ctx, const TermaArgs& a0) {
     const double nbb = (double)a.bx * a.by * a.bz;
     const double nct = (double)a.vd.nx * a.vd.ny * a.vd.nz;
     int tok = prof_begin(ctx, K_TERMA);
-    hipLaunchKernelGGL(terma_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a);
+    const auto kernel = a.ss > 1 ? (a.counts ? terma_kernel<true, true> : terma_kernel<true, false>)
+                                 : (a.counts ? terma_kernel<false, true> : terma_kernel<false, false>);
+    // (LDS it does not use bounds the workgroups of a CU)
+    const size_t lds = (size_t)(160 * 1024 / kTermaResident - 256);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, ctx->stream, a);
     prof_end(ctx, tok, 4.0 * nct + 4.0 * nbb, 0.0, (uint64_t)nbb);
     CCCS_HIP(hipGetLastError());
     return CCCS_OK;
