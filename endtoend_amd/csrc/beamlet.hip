@@ -27,7 +27,6 @@
 namespace cccs {
 
 constexpr int kWall = 2;        // pillar wall, REV samples (PILLAR_GRID, io_data_structs.h:139-160)
-constexpr int kLineZeros = 2;   // zero samples kept before and behind every stored REV line (BlArgs::zeros)
 constexpr int kBuffer = 2;      // pillar rim excluded from unpacking (same struct)
 constexpr int kMaxBatches = 100;  // batch-count retry limit of the reference (host.cu:692-834)
 constexpr uint32_t kSubQueues = 64;  // TERMA sub-queues per cone direction
@@ -889,15 +888,6 @@ __device__ __forceinline__ bool bl_gather_hit(const BatchDev& B, const BlConeDev
 // issued before any of their stores, so a lane has four fetches in flight.
 constexpr int kGatherX = 4;  // the tile's depth along pX
 constexpr int kGatherY = 4;  // pY voxels per lane
-
-// The stored line of record (off, w) at sample i, interpolated at fraction x: the clamp takes samples
-// outside the line to its zeros.  rev0 is kLineZeros samples before the store.
-__device__ __forceinline__ float line_lerp(const char* __restrict__ rev0, uint32_t off, uint32_t w, int i, float x) {
-    const int d = i - (int)(int16_t)(w & 0xffffu), len = (int)w >> 16;
-    const int at = min(max(d, -kLineZeros), len) + (int)off;  // (v_med3)
-    const pair_f32 p = *reinterpret_cast<const pair_f32*>(rev0 + (uint32_t)(at + kLineZeros) * 4u);
-    return p.x + x * (p.y - p.x);
-}
 
 __global__ void __launch_bounds__(64) bl_gather_kernel(BlArgs a, uint32_t ntiles) {
     const uint32_t tile = xcd_chunks(blockIdx.x, gridDim.x, 64);

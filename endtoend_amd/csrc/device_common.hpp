@@ -149,6 +149,22 @@ __device__ __forceinline__ float rev_fetch(const LineMeta* __restrict__ meta, co
     return e0 + c * (e1 - e0);
 }
 
+// Zero samples kept before and behind every stored line, where a launch's `zeros` says so (a store of fewer
+// than 2^30 samples; empty lines then have offset 0 and the store begins with as many zeros): a
+// select on the index replaces one on each sample.
+constexpr int kLineZeros = 2;
+
+// The stored line of record (off, w) at sample i, interpolated at fraction x; rev0 is kLineZeros samples
+// before the store.  Samples outside the line all read the store's first zeros: the load of a wave
+// costs its different cache lines, so those lanes share one (clamped to their own line's zeros
+// instead, two instructions less, the beamlet gather took 79 us a direction, not 70).
+__device__ __forceinline__ float line_lerp(const char* __restrict__ rev0, uint32_t off, uint32_t w, int i, float x) {
+    const int d = i - (int)(int16_t)(w & 0xffffu);
+    const uint32_t at = (uint32_t)(d + 1) <= w >> 16 ? (uint32_t)(d + kLineZeros) + off : 0u;
+    const pair_f32 p = *reinterpret_cast<const pair_f32*>(rev0 + at * 4u);
+    return p.x + x * (p.y - p.x);
+}
+
 // The line's samples live in LDS as {half step, TERMA}: x = 0.5*delr*density (negative marks a
 // sample outside the crop box or the calc_bbox), y = TERMA.
 //
