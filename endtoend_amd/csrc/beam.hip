@@ -6,12 +6,14 @@
 //   2. crop_partial/final  BEV-rotated extent of non-zero TERMA, reduced on the GPU instead of the
 //                        reference's D2H copy + host triple loop (:417-499); 28 bytes come back
 //   3. host geometry     crop box + one REV grid per cone (findREV :75-155)
-//   4. cone_kernel       one workgroup per REV line, all cones in one launch: resample density and
+//   4. line_interval / class_scan / class_scatter_kernel  stored interval, offset and class-list entry of
+//                        every REV line of every cone
+//   5. cone_kernel       one workgroup per listed line, one launch per length class: resample density and
 //                        TERMA along the line into LDS (cudaRaytrace, nvbbRayConvolve_device.cu:11-80)
 //                        then the collapsed-cone walk in both directions from LDS (RowConvolve
 //                        :87-218).  The REV grid is sized per cone; nothing is cleared per cone.
-//   5. pvcs_kernel       one pass over the PVCS voxels the crop box can reach, gathering every
-//                        cone's REV dose trilinearly and adding the sum once (REV2XYZdose
+//   6. pvcs_kernel       passes over the PVCS voxels the crop box can reach, gathering their
+//                        cones' REV dose trilinearly and adding the sum once (REV2XYZdose
 //                        :222-261 per cone in the reference).
 #include <hip/hip_runtime.h>
 
@@ -255,38 +257,6 @@ __global__ void __launch_bounds__(256) crop_partial_kernel(const float* __restri
         __syncthreads();
     }
     if (t < 7) part[(size_t)blockIdx.x * 8 + t] = s[t][0];
-}
-
-// Small boxes in one workgroup: the launch that combines the partials costs more than the pass.
-constexpr size_t kCropSmall = size_t(1) << 16;  // voxels
-__global__ void __launch_bounds__(1024) crop_small_kernel(const float* __restrict__ terma, int bx, int by, int bz, Rot2 rot,
-                                                          float* __restrict__ out) {
-    __shared__ float s[16][7];
-    float v[7] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX, 0.f};
-    const uint32_t n = (uint32_t)bx * (uint32_t)by * (uint32_t)bz, t = threadIdx.x;
-#pragma unroll 4
-    for (uint32_t i = t; i < n; i += 1024) {
-        if (terma[i] == 0.f) continue;
-        const uint32_t row = i / (uint32_t)bx, z = row / (uint32_t)by;
-        const v3 b = rot_fwd(rot, mk3((float)(i - row * (uint32_t)bx), (float)(row - z * (uint32_t)by), (float)z));
-        v[0] = fminf(v[0], b.x); v[1] = fminf(v[1], b.y); v[2] = fminf(v[2], b.z);
-        v[3] = fmaxf(v[3], b.x); v[4] = fmaxf(v[4], b.y); v[5] = fmaxf(v[5], b.z);
-        v[6] += 1.f;
-    }
-#pragma unroll
-    for (int q = 0; q < 7; q++)
-        for (int o = 32; o > 0; o >>= 1) {
-            const float u = __shfl_xor(v[q], o, 64);
-            v[q] = q < 3 ? fminf(v[q], u) : q < 6 ? fmaxf(v[q], u) : v[q] + u;
-        }
-    if ((t & 63) == 0)
-        for (int q = 0; q < 7; q++) s[t >> 6][q] = v[q];
-    __syncthreads();
-    if (t < 7) {
-        float r = s[0][t];
-        for (int w = 1; w < 16; w++) r = t < 3 ? fminf(r, s[w][t]) : t < 6 ? fmaxf(r, s[w][t]) : r + s[w][t];
-        out[t] = r;
-    }
 }
 
 __global__ void __launch_bounds__(256) crop_final_kernel(const float* __restrict__ part, int nblocks, float* __restrict__ out) {
@@ -1509,14 +1479,9 @@ int run_crop(BeamScratch& S, const float* d_terma, const cccs_beam& b, float* re
     // the result goes straight to pinned host memory (the fixed array's caller has none)
     float* out = S.arena ? part + kCropBlocks * 8 : S.host_small;
     int tok = prof_begin(ctx, K_CROP);
-    if (n <= kCropSmall) {
-        hipLaunchKernelGGL(crop_small_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_terma, (int)p.bbox_size[0],
-                           (int)p.bbox_size[1], (int)p.bbox_size[2], rot, out);
-    } else {
     hipLaunchKernelGGL(crop_partial_kernel, dim3(blocks), dim3(256), 0, ctx->stream, d_terma, (int)p.bbox_size[0],
                        (int)p.bbox_size[1], (int)p.bbox_size[2], rot, part);
-        hipLaunchKernelGGL(crop_final_kernel, dim3(1), dim3(256), 0, ctx->stream, part, blocks, out);
-    }
+    hipLaunchKernelGGL(crop_final_kernel, dim3(1), dim3(256), 0, ctx->stream, part, blocks, out);
     prof_end(ctx, tok, 4.0 * (double)n, 0.0, n);
     CCCS_HIP(hipGetLastError());
     if (S.arena)
