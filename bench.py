@@ -474,7 +474,7 @@ def main():
     ap.add_argument("--bl-streams", type=int, default=0,
                     help="cone directions in flight for the whole run (profiling runs: 1); 0 = the library default")
     ap.add_argument("--bl-sample-waves", type=int, default=0,
-                    help="sample-stage waves for the whole run (profiling runs: 262144, as in the one-stream "
+                    help="sample-stage waves for the whole run (profiling runs: 4096, as in the one-stream "
                          "pass); 0 = the library default")
     ap.add_argument("--copy-mib", type=int, default=0,
                     help="only run the streaming copy kernel on this many MiB (HBM counter calibration)")
@@ -532,11 +532,11 @@ def main():
     dt = t1 - t0
     # per-kernel times: one step with one cone direction in flight, so that no two kernels share
     # the device and the kernel times add up to no more than that step.  Alone on the device the
-    # sample stage runs at its standalone best, 4 waves per SIMD (262144 waves); the headline
+    # sample stage runs at its standalone best, 4 waves per SIMD (4096 waves); the headline
     # keeps it at 2 waves per SIMD so that the other directions' stages run beside it.
     nstreams = eng.get_schedule("bl_streams")
     swaves = eng.get_schedule("bl_sample_waves")
-    alone = {"bl_streams": 1, "bl_sample_waves": 262144}
+    alone = {"bl_streams": 1, "bl_sample_waves": 4096}
     for k, v in alone.items():
         eng.set_schedule(k, v)
     step()

@@ -883,9 +883,10 @@ __device__ __forceinline__ bool bl_gather_hit(const BatchDev& B, const BlConeDev
 // fastest), as four 4x4x4 cubes along pY: a load of a cube touches the fewest different REV lines
 // over all cone directions (projected area 24 against 42 voxels for a 16x4x1 slab), which is what
 // bounds the gather, and a lane keeps one (pX, pZ) for its four voxels, so the pillar test runs once
-// per lane instead of once per voxel (140 -> 133 us with the pair loads alone, 91 us with the cubes:
-// one 5 mm beam, 128^3 water, per direction alone on the device).  The four voxels' loads are all
-// issued before any of their stores, so a lane has four fetches in flight.
+// per lane instead of once per voxel.  The four voxels' loads are all issued before any of their
+// stores, so a lane has four fetches in flight.  One 5 mm beam, 128^3 water, per direction alone on
+// the device: 140 us with single-tap loads, 133 with pair loads, 91 with the cubes, 77 with lines that
+// end in zeros (half the instructions), 70 with one cache line for the lanes outside their lines.
 constexpr int kGatherX = 4;  // the tile's depth along pX
 constexpr int kGatherY = 4;  // pY voxels per lane
 
@@ -1857,7 +1858,7 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
             a.counts = nullptr;
             if (a.nlines == 0) continue;
             const int k = r % nset;
-            // the helpers (line scan, profiling events) enqueue on ctx->stream and use ctx->scan
+            // the profiling events enqueue on ctx->stream, and the block totals sit in ctx->scan
             ctx->stream = S[k];
             std::swap(ctx->scan, *set_scan[k]);
             a.lines = set_lines[k]->as<LineMeta>() + kRevPad;

@@ -137,7 +137,7 @@ int cccs_ctx_memory(const cccs_ctx* ctx, uint64_t* resident_bytes, uint64_t* scr
  * rounding).  Keys:
  *   "cone_ramp_min"  full-beam cone lines with at least this many valid samples use the
  *                    segment-sum walk, O(nradii) per sample, instead of the sequential walk,
- *                    O(line) per sample (default 64; a value above the longest line disables it).
+ *                    O(line) per sample (default 32; a value above the longest line disables it).
  *   "cone_class_len0".."cone_class_len2"
  *                    upper stored-line lengths of the first three cone-kernel launch classes
  *                    (defaults 96, 160, 320; the last class takes the longer lines).  Each class
@@ -146,11 +146,11 @@ int cccs_ctx_memory(const cccs_ctx* ctx, uint64_t* resident_bytes, uint64_t* scr
  *                    consecutive directions' sample, Siddon and walk overlap on their own
  *                    streams; the gathers stay in direction order).
  *   "bl_sample_waves", "bl_walk_waves"
- *                    waves of the beamlet path's persistent per-line kernels (defaults 262144 and
- *                    32768; each wave takes a stride of lines).
+ *                    waves of the beamlet path's persistent per-line kernels (defaults 3072 and
+ *                    16384; each wave takes a stride of lines).
  *   "bl_walk_split"  the beamlet walk runs one launch per line-length class (up to this many
  *                    stored samples, up to twice that, ..., the rest), each with its LDS sized
- *                    for its own longest line (default 256; 0 = one launch).
+ *                    for its own longest line (default 128; 0 = one launch).
  *   "cone_class_threads0".."cone_class_threads3"
  *                    threads per cone line in each class: 64, 128 or 256 (defaults 64, 64, 128,
  *                    128). */
