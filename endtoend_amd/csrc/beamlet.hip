@@ -316,7 +316,7 @@ __device__ __forceinline__ float kc_at(float r, const float4* __restrict__ tab, 
     return iv.y + (r - iv.x) * iv.z;
 }
 
-constexpr int kStagePillars = 64;  // footprint pillars of one line whose beamlet data sits in LDS
+constexpr int kStagePillars = 64;  // footprint pillars of one line that the stage's CPU replay counts as usual
 
 __device__ __forceinline__ int lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ float lane_f(float v, int lane) {
