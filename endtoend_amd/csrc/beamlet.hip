@@ -2628,7 +2628,6 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         for (const BeamletDev& bl : J.beamlets) max_rows = std::max(max_rows, bl.boxn[0] * bl.boxn[1]);
         const int chunks = (max_rows + 255) / 256;
         const uint64_t units = (uint64_t)nbl * (uint64_t)chunks;
-        if (units > 0x7fffffffULL) return set_error(CCCS_EGEOM, "too many beamlet rows in one job");
         const size_t o_off = (sizeof(uint32_t) * 4 * nbl + 255) & ~size_t(255);
         const size_t o_chunk = (o_off + sizeof(uint64_t) * (nbl + 1) + 255) & ~size_t(255);
         CCCS_TRY(ctx->bl_cnt.ensure(o_chunk + sizeof(uint32_t) * units));
@@ -2660,8 +2659,17 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         int tok = prof_begin(ctx, K_BL_UNPACK);
         hipLaunchKernelGGL(bl_fill_kernel, dim3(grid_for(4 * (uint64_t)nbl, 256)), dim3(256), 0, ctx->stream,
                            reinterpret_cast<float*>(stat), 4 * (uint64_t)nbl, 0.f);
-        hipLaunchKernelGGL(bl_colmax_kernel, dim3((unsigned)units), dim3(256), 0, ctx->stream, ca);
-        hipLaunchKernelGGL(bl_colcount_kernel, dim3((unsigned)units), dim3(256), 0, ctx->stream, ca);
+        // one launch takes as many beamlets as its workgroups allow: jobs of many small boxes and a few huge
+        // ones have more than kMaxGroups chunks (a single box never does: it has fewer than 2^32 rows)
+        auto over = [&](int b0, int b1, void (*kernel)(ColArgs)) {
+            const int per = (int)std::max<uint32_t>(1, kMaxGroups / (uint32_t)chunks);
+            for (int b = b0; b < b1; b += per) {
+                ca.beamlet0 = b;
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(std::min(per, b1 - b) * chunks)), dim3(256), 0, ctx->stream, ca);
+            }
+        };
+        over(0, nbl, bl_colmax_kernel);
+        over(0, nbl, bl_colcount_kernel);
         prof_end(ctx, tok, 0.0, 0.0, (uint64_t)nbl);
         hipLaunchKernelGGL(bl_offsets_kernel, dim3(1), dim3(1024), 0, ctx->stream, stat, nbl, offs);
         CCCS_HIP(hipGetLastError());
@@ -2681,12 +2689,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         CCCS_TRY(ctx->bl_vals.ensure(sizeof(float) * std::max<uint64_t>(1, nnz_total)));
         ca.keys = ctx->bl_keys.as<uint64_t>();
         ca.vals = ctx->bl_vals.as<float>();
-        auto emit = [&](int b0, int b1) {
-            if (b1 <= b0) return;
-            ca.beamlet0 = b0;
-            hipLaunchKernelGGL(bl_emit_kernel, dim3((unsigned)((uint64_t)(b1 - b0) * chunks)), dim3(256), 0, ctx->stream,
-                               ca);
-        };
+        auto emit = [&](int b0, int b1) { over(b0, b1, bl_emit_kernel); };
         // ROI reduction of the job's columns (count, scan, order-preserving emit)
         RoiArgs ra;
         const uint64_t* out_off = hoff;  // first output entry of every column

@@ -32,6 +32,9 @@ __device__ __forceinline__ uint32_t xcd_chunks(uint32_t b, uint32_t nb, uint32_t
     return s0 + (r % 8) * chunk + r / 8;
 }
 
+// Workgroups of 256 threads in one launch: the threads along a launch dimension are counted in 32 bits.
+constexpr uint32_t kMaxGroups = (1u << 24) - 1;
+
 // Sums one uint32 per lane over a 64-lane workgroup into part[slot] (no LDS).
 __device__ __forceinline__ void wave_count(uint32_t v, uint32_t* __restrict__ part, size_t slot) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -1,0 +1,34 @@
+"""Calls whose kernels take more workgroups than one launch holds (2^24 - 1 of 256 threads): they run in
+several launches, and every part of the result is what a smaller call gives, bit for bit."""
+import numpy as np
+import pytest
+
+from endtoend_amd import engine as E
+from endtoend_amd import workloads as W
+from endtoend_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def test_columns_of_many_small_boxes_and_a_huge_one():
+    """One beamlet whose box spans a wide, flat grid beside 400 with narrow boxes: the column passes' chunks of
+    rows (those of the largest box for every beamlet) exceed one launch."""
+    n = 3300
+    ph = W.Phantom(np.full((4, n, n), 0.02, np.float32), 0.1)
+    spec = W.problem(ph, nphi=2, ntheta=4, spacing=0.5, kernel_extent=0.3, max_rev_size=(1024, 1024, 1024))
+    beams = [E.make_beam(45.0, 0.0, 0.0, sad=400.0, fmap_size=(1, 1), beamlet_size=(0.5, 0.5)),
+             E.make_beam(0.0, 0.0, 0.0, sad=400.0, fmap_size=(400, 1), beamlet_size=(0.5, 0.5))]
+    fmaps = [np.ones((1, 1), np.float32), np.ones((1, 400), np.float32)]
+    with Engine(spec) as eng:
+        eng.set_schedule("bl_streams", 1)  # (both beams then fit into one job)
+        print("[case] both beams", flush=True)
+        both = eng.beamlet_dose(beams, fmaps, threshold=1e-4)
+        print("[case] each beam alone", flush=True)
+        alone = [eng.beamlet_dose([b], [f], threshold=1e-4) for b, f in zip(beams, fmaps)]
+    rows = np.unique(both[0][2] // np.uint64(n) % np.uint64(n)).size
+    assert rows > 1500  # the diagonal beamlet's column reaches far over the grid
+    one = [(i, c[1], c[2], c[3]) for i, cols in enumerate(alone) for c in cols]
+    assert len(both) == len(one) == 401
+    for x, y in zip(both, one):
+        assert x[:2] == y[:2]
+        assert np.array_equal(x[2], y[2]) and np.array_equal(x[3].view(np.uint32), y[3].view(np.uint32))
