@@ -77,6 +77,7 @@ struct TermaArgs {
     int beamletnum;
     int depth, far_first;     // axis along which the beam runs mostly; start at its high end
     float field2;             // squared tangent of a cone around the fluence map (infinite: unknown)
+    uint32_t block0;          // first workgroup of this launch
     uint32_t* counts;         // per-block Siddon step counts (profiling) or nullptr
 };
 
@@ -100,7 +101,7 @@ constexpr int kTermaResident = 6;
 __device__ __forceinline__ void terma_voxel(const TermaArgs& a, int& X, int& Y, int& Z) {
     const uint32_t nx = (uint32_t)(a.bx + 15) / 16, ny = (uint32_t)(a.by + 3) / 4, nz = (uint32_t)(a.bz + 3) / 4;
     const uint32_t inner = a.depth == 0 ? ny : nx, middle = a.depth == 2 ? ny : nz;
-    const uint32_t t = xcd_chunks(blockIdx.x, gridDim.x, inner), r = t / inner;
+    const uint32_t t = a.block0 + xcd_chunks(blockIdx.x, gridDim.x, inner), r = t / inner;
     // (the rows turn from plane to plane, or a multiple of 8 rows would keep each on one XCD)
     const uint32_t i = t - r * inner, w0 = r / middle, m0 = r - w0 * middle + (middle >= 8 ? 5 * w0 & 7u : 0u);
     const uint32_t m = m0 >= middle ? m0 - middle : m0;
@@ -123,6 +124,17 @@ __device__ __forceinline__ bool outside_field(const TermaArgs& a, v3 p) {
 }
 inline uint64_t terma_blocks(const TermaArgs& a) {
     return (uint64_t)((a.bx + 15) / 16) * (uint64_t)((a.by + 3) / 4) * (uint64_t)((a.bz + 3) / 4);
+}
+
+// The workgroups of a calc_bbox, in as many launches as their number takes (boxes beyond 2^32 voxels of
+// whole workgroups: thin ones fill the last workgroup of a row badly).
+template <class Launch>
+void terma_launches(TermaArgs& a, Launch&& launch) {
+    const uint64_t n = terma_blocks(a);
+    for (uint64_t b = 0; b < n; b += kMaxGroups) {
+        a.block0 = (uint32_t)b;
+        launch(dim3((unsigned)std::min<uint64_t>(kMaxGroups, n - b)));
+    }
 }
 
 // One lane per calc_bbox voxel (x fastest => coalesced store).  Each lane marches its own ray
@@ -163,7 +175,7 @@ __global__ void __launch_bounds__(256) terma_kernel(TermaArgs a) {
         if (kCount) steps = (uint32_t)it;
     }
     if (in) a.terma[(size_t)X + (size_t)a.bx * ((size_t)Y + (size_t)a.by * Z)] = acc;
-    if (kCount) block_count(steps, a.counts, blockIdx.x);
+    if (kCount) block_count(steps, a.counts, a.block0 + blockIdx.x);
 }
 
 // Unit-fluence TERMA of every calc_bbox voxel (the march runs for every voxel): one beam source's
@@ -1300,6 +1312,7 @@ TermaArgs terma_args(cccs_ctx* ctx, const cccs_beam& b, const float* d_fmap, flo
     a.bhc = ctx->prob.beamhard_correct;
     a.beamletnum = beamletnum;
     a.counts = nullptr;
+    a.block0 = 0;
     const v3 dir = a.beam.iso - a.beam.src;
     const float dc[3] = {dir.x, dir.y, dir.z};
     a.depth = 2;
@@ -1327,7 +1340,7 @@ int launch_terma(cccs_ctx* ctx, const TermaArgs& a0) {
                                  : (a.counts ? terma_kernel<false, true> : terma_kernel<false, false>);
     // (LDS it does not use bounds the workgroups of a CU)
     const size_t lds = (size_t)(160 * 1024 / kTermaResident - 256);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, ctx->stream, a);
+    terma_launches(a, [&](dim3 grid) { hipLaunchKernelGGL(kernel, grid, dim3(256), lds, ctx->stream, a); });
     prof_end(ctx, tok, 4.0 * nct + 4.0 * nbb, 0.0, (uint64_t)nbb);
     CCCS_HIP(hipGetLastError());
     return CCCS_OK;
@@ -2007,8 +2020,9 @@ extern "C" int cccs_angle_cache_create(cccs_ctx* ctx, const cccs_beam* beams, in
             TermaArgs a = terma_args(ctx, beams[keep[e]], nullptr, nullptr, -1);
             const uint64_t blocks = terma_blocks(a);
             if (blocks <= 0x7fffffffULL)
-                hipLaunchKernelGGL(unit_terma_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a,
-                                   c->data + e * c->nbbox);
+                terma_launches(a, [&](dim3 grid) {
+                    hipLaunchKernelGGL(unit_terma_kernel, grid, dim3(256), 0, ctx->stream, a, c->data + e * c->nbbox);
+                });
             const hipError_t err = blocks <= 0x7fffffffULL ? hipGetLastError() : hipErrorInvalidValue;
             if (err != hipSuccess) {
                 (void)hipStreamSynchronize(ctx->stream);

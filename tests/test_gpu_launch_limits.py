@@ -32,3 +32,23 @@ def test_columns_of_many_small_boxes_and_a_huge_one():
     for x, y in zip(both, one):
         assert x[:2] == y[:2]
         assert np.array_equal(x[2], y[2]) and np.array_equal(x[3].view(np.uint32), y[3].view(np.uint32))
+
+
+def test_terma_of_a_thin_box():
+    """A calc_bbox one voxel thick along x fills a sixteenth of its workgroups' lanes."""
+    ny, nz = 16384, 16400
+    spec = W.problem(W.Phantom(np.ones((nz, ny, 1), np.float32), 0.01), nphi=2, ntheta=4, max_rev_size=(800, 800, 800))
+    beam = E.make_beam(0.0, 0.0, 0.0, iso=(0.0, 0.0, 0.0), sad=100.0, fmap_size=(3, 3), beamlet_size=(0.3, 0.3))
+    fmap = np.arange(1.0, 10.0, dtype=np.float32).reshape(3, 3)
+    with Engine(spec) as eng:
+        print("[case] whole box", flush=True)
+        whole = eng.beam_terma(beam, fmap)
+    z = np.nonzero(whole.any(axis=(1, 2)))[0]
+    assert z.size > 50
+    lo = int(z[0]) - 8
+    spec.bbox_start, spec.bbox_size = (0, 0, lo), (1, ny, int(z[-1]) + 8 - lo)
+    with Engine(spec) as eng:
+        print("[case] field only", flush=True)
+        part = eng.beam_terma(beam, fmap)
+    np.testing.assert_array_equal(whole[lo:lo + part.shape[0]].view(np.uint32), part.view(np.uint32))
+    assert not whole[:lo].any() and not whole[lo + part.shape[0]:].any()
