@@ -1185,10 +1185,11 @@ __device__ __forceinline__ bool mask_ray_hit(v3 sink, const VolDesc& vd, v3 ivox
 constexpr int kSubRays = 9;
 __global__ void __launch_bounds__(64 * kSubRays) projection_kernel(const float* __restrict__ mask, VolDesc vd, v3 ivoxel,
                                                         const int* __restrict__ box, const ProjBeam* __restrict__ beams,
-                                                        int nbeams, uint32_t total, float* __restrict__ out) {
+                                                        int nbeams, uint32_t block0, uint32_t total,
+                                                        float* __restrict__ out) {
     __shared__ uint32_t s_hit[64];
     const int lane = threadIdx.x & 63, sr = threadIdx.x >> 6;
-    const uint32_t t = blockIdx.x * 64 + lane;
+    const uint32_t t = (block0 + blockIdx.x) * 64 + lane;
     if (sr == 0) s_hit[lane] = 0u;
     __syncthreads();
     if (t < total && box[3] >= 0) {
@@ -2226,9 +2227,12 @@ extern "C" int cccs_fluence_projection(cccs_ctx* ctx, const uint8_t* mask, const
                        mf.as<float>(), nv, ctx->vol.nx, ctx->vol.ny, box);
     CCCS_HIP(hipGetLastError());
     const v3 vox = ctx->vol.voxel;
-    hipLaunchKernelGGL(projection_kernel, dim3((unsigned)((total + 63) / 64)), dim3(64 * kSubRays), 0, ctx->stream,
-                       (const float*)mf.as<float>(), ctx->vol, mk3(1.f / vox.x, 1.f / vox.y, 1.f / vox.z), (const int*)box,
-                       (const ProjBeam*)tb.as<ProjBeam>(), nbeams, (uint32_t)total, ob.as<float>());
+    // (a launch holds kMaxGroups workgroups of 256 threads; these have 576)
+    const uint32_t groups = (uint32_t)((total + 63) / 64), per = kMaxGroups / 3;
+    for (uint32_t b0 = 0; b0 < groups; b0 += per)
+        hipLaunchKernelGGL(projection_kernel, dim3(std::min(per, groups - b0)), dim3(64 * kSubRays), 0, ctx->stream,
+                           (const float*)mf.as<float>(), ctx->vol, mk3(1.f / vox.x, 1.f / vox.y, 1.f / vox.z),
+                           (const int*)box, (const ProjBeam*)tb.as<ProjBeam>(), nbeams, b0, (uint32_t)total, ob.as<float>());
     CCCS_HIP(hipGetLastError());
     CCCS_HIP(hipStreamSynchronize(ctx->stream));
     CCCS_HIP(hipMemcpy(fluence, ob.p, sizeof(float) * total, hipMemcpyDeviceToHost));

@@ -52,3 +52,19 @@ def test_terma_of_a_thin_box():
         part = eng.beam_terma(beam, fmap)
     np.testing.assert_array_equal(whole[lo:lo + part.shape[0]].view(np.uint32), part.view(np.uint32))
     assert not whole[:lo].any() and not whole[lo + part.shape[0]:].any()
+
+
+def test_projection_of_half_a_billion_beamlets():
+    n, m = 8, 8000
+    spec = W.problem(W.water_cube(16, 1.0), nphi=2, ntheta=4)
+    mask = np.zeros((16, 16, 16), np.uint8)
+    mask[4:11, 6:9, 5:12] = 1
+    beams = [E.make_beam(40.0 * i, 10.0 * i, 0.0, fmap_size=(m, m), beamlet_size=(0.002, 0.002)) for i in range(n)]
+    with Engine(spec) as eng:
+        print("[case] all beams", flush=True)
+        got = eng.fluence_projection(mask, beams)
+        for i in (0, n - 1):
+            print(f"[case] beam {i}", flush=True)
+            one = eng.fluence_projection(mask, [beams[i]])[0]
+            np.testing.assert_array_equal(got[i], one)
+            assert 0 < int(one.sum()) < m * m
