@@ -304,7 +304,8 @@ __device__ __forceinline__ float bl_density(const BlArgs& a, const MarchVol& vol
                                             v3 inp) {
     const v3 g2 = rot_inv(B.beam_inv, rot1(bl.inv, inp * a.rvs)) + bl.pst;
     const v3 gi = div_by(g2 - a.vd.start, a.vd.voxel, a.ivoxel);
-    return tex3_march(vol, gi.x + 0.5f, gi.y + 0.5f, gi.z + 0.5f);
+    const float s = gi.x + gi.y + gi.z;  // (div_by makes an infinite quotient NaN: outside, as the quotient)
+    return s == s ? tex3_march(vol, gi.x + 0.5f, gi.y + 0.5f, gi.z + 0.5f) : 0.f;
 }
 
 // Cumulative kernel of one row, linear between radii (the reference's clamped linear texture

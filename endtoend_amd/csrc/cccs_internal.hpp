@@ -270,7 +270,7 @@ CCCS_HD uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) {
 
 // A volume as the march's taps see it: the addresses of the four x rows of a cell, so that a tap
 // address is a uniform base and one 32-bit offset, formed with 24-bit products.  Volumes beyond that
-// (`small` false) take tex3_border's general addresses.
+// (`small` false), and coordinates that may not be numbers, take tex3_border's general addresses.
 struct MarchVol {
     const float* v;
     int nx, ny, nz;
@@ -291,7 +291,8 @@ CCCS_HD MarchVol march_vol(const float* v, int nx, int ny, int nz) {
     m.p11 = reinterpret_cast<const char*>(v + (size_t)nx * ny + nx);
     return m;
 }
-// tex3_border at (u, w, t): the same operations where all eight taps lie inside (two per load).
+// tex3_border at (u, w, t), which are numbers where `small` holds (one that is not would turn into index
+// 0): the same operations where all eight taps lie inside (two per load).
 CCCS_HD float tex3_march(const MarchVol& m, float u, float w, float t) {
     typedef float pair __attribute__((ext_vector_type(2), aligned(4)));
     const float xb = u - 0.5f, yb = w - 0.5f, zb = t - 0.5f;
@@ -332,12 +333,14 @@ CCCS_HD float siddon_rpl(v3 this_voxel, v3 start, v3 end, v3 voxel, v3 ivoxel, v
     float rpl = 0.0f;
     int iter = 0;
     if (!(a_min >= a_max)) {
-        const MarchVol vol = march_vol(dens, nx, ny, nz);
+        MarchVol vol = march_vol(dens, nx, ny, nz);
         float d12 = len3(diff);
         float step_x = fabsf(voxel.x / diff.x);
         float step_y = fabsf(voxel.y / diff.y);
         float step_z = fabsf(voxel.z / diff.z);
         const v3 o = (src - start) * ivoxel, dd = diff * ivoxel;
+        // (a voxel size whose reciprocal overflows: coordinates that are not numbers read 0)
+        vol.small = vol.small && ((o.x + o.y) + (o.z + dd.x) + (dd.y + dd.z)) * 0.f == 0.f;
         float alpha = a_min, ax = a_min, ay = a_min, az = a_min;
         for (int n = 1;; n++) {
             // the three plane tests run in sequence and each sees the alphas already advanced
