@@ -2549,6 +2549,15 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             if (!e) CCCS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     hipEvent_t copy_done = nullptr;  // the last job's last column copy (its buffers are rewritten after it)
+    // No return leaves a column copy on its way: the next call's fluence maps are staged in the buffer that
+    // the copies write.
+    struct Drain {
+        hipStream_t s;
+        bool queued;
+        ~Drain() {
+            if (queued) (void)hipStreamSynchronize(s);
+        }
+    } drain{ctx->cstream, false};
     Delivery pending;
     int njob = 0;
     auto deliver = [&]() -> int {
@@ -2581,10 +2590,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             col.keys = pending.keys + pos;
             col.values = pending.vals + pos;
             pos += col.nnz;
-            if (sink(user, &col) != 0) {
-                (void)hipStreamSynchronize(ctx->cstream);  // the parts still on their way
-                return set_error(CCCS_EIO, "sparse sink aborted the call");
-            }
+            if (sink(user, &col) != 0) return set_error(CCCS_EIO, "sparse sink aborted the call");
         }
         return CCCS_OK;
     };
@@ -2774,6 +2780,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
                 const uint64_t e0 = out_off[b0], n = out_off[b1] - e0;
                 CCCS_HIP(hipEventRecord(ev, ctx->stream));
                 CCCS_HIP(hipStreamWaitEvent(cs, ev, 0));
+                drain.queued = true;
                 if (n) {
                     const uint64_t* sk = (nroi > 0 ? ctx->roi_keys : ctx->bl_keys).as<uint64_t>();
                     const float* sv = (nroi > 0 ? ctx->roi_vals : ctx->bl_vals).as<float>();
@@ -2793,5 +2800,6 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         njob++;
     }
     CCCS_TRY(deliver());
+    drain.queued = false;  // (the last part has arrived)
     return CCCS_OK;
 }
