@@ -1810,13 +1810,11 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
         launch_cone(cls_threads[c], dim3(cls_n[c]), lds, ctx->stream, ca);
         CCCS_HIP(hipGetLastError());
     }
-    if (ca.zeros) {
-        const uint64_t lines = (uint64_t)cls_n[0] + cls_n[1] + cls_n[2] + cls_n[3];
-        if (lines == 0) return CCCS_OK;
-        stored -= (uint64_t)kLineZeros * lines;
-    }
+    const uint64_t lines = (uint64_t)cls_n[0] + cls_n[1] + cls_n[2] + cls_n[3];
+    if (ca.zeros) stored -= (uint64_t)kLineZeros * lines;
     // algorithmic traffic: density + TERMA in, cone dose out, per stored sample
     prof_end(ctx, tok, 12.0 * (double)stored, 0.0, stored);
+    if (ca.zeros && lines == 0) return CCCS_OK;  // (nothing wrote the zeros that the short form reads)
     PvcsArgs pa;
     pa.cones = d_cones;
     pa.lines = ca.lines;
