@@ -1762,6 +1762,19 @@ BlArgs base_args(cccs_ctx* ctx) {
 // Line table and REV store with the pads of rev_fetch's pair loads.
 inline size_t line_bytes(uint64_t n) { return sizeof(LineMeta) * (size_t)(n + 2 * kRevPad); }
 inline size_t rev_bytes(uint64_t n) { return sizeof(float) * (size_t)(n + 2 * kRevPad); }
+// Whether a store of `rev` samples in `lines` lines keeps the zeros around its lines, and the samples that it
+// then has.
+inline bool line_zeros(uint64_t rev, uint64_t lines) {
+    return rev + (uint64_t)kLineZeros * lines + 2 * kRevPad < (uint64_t(1) << 30);
+}
+inline uint64_t store_samples(uint64_t rev, uint64_t lines) {
+    return rev + (line_zeros(rev, lines) ? (uint64_t)kLineZeros * lines : 0);
+}
+// Device bytes of one cone direction in flight: REV store, half steps, line table and the lines' grids (the
+// pads apart).
+inline uint64_t direction_bytes(uint64_t rev, uint64_t lines) {
+    return 2 * sizeof(float) * store_samples(rev, lines) + (sizeof(LineMeta) + sizeof(uint32_t)) * lines;
+}
 
 inline unsigned grid_for(uint64_t n, unsigned block) { return (unsigned)std::min<uint64_t>((n + block - 1) / block, 1u << 20); }
 
@@ -1787,8 +1800,8 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     CCCS_TRY(ctx->bl_pdose.ensure(sizeof(float) * std::max<uint64_t>(1, J.pdose)));
     CCCS_TRY(ctx->lines.ensure(line_bytes(J.max_lines)));
     // (the zeros around every line count as samples of the store)
-    const bool zeros = J.max_rev + (uint64_t)kLineZeros * J.max_lines + 2 * kRevPad < (uint64_t(1) << 30);
-    const uint64_t max_rev = J.max_rev + (zeros ? (uint64_t)kLineZeros * J.max_lines : 0);
+    const bool zeros = line_zeros(J.max_rev, J.max_lines);
+    const uint64_t max_rev = store_samples(J.max_rev, J.max_lines);
     CCCS_TRY(ctx->rev.ensure(rev_bytes(max_rev)));
     CCCS_TRY(ctx->bl_h.ensure(sizeof(float) * std::max<uint64_t>(1, max_rev)));
     CCCS_TRY(ctx->bl_qcnt.ensure(sizeof(uint32_t) * (size_t)std::max(1, nrays)));
@@ -2425,7 +2438,7 @@ extern "C" int cccs_beamlet_footprint(const cccs_ctx* ctx, const cccs_beam* beam
     }
     uint64_t mr = 0, ml = 0;
     for (int r = 0; r < ctx->nrays; r++) { mr = std::max(mr, rev[r]); ml = std::max(ml, lines[r]); }
-    *bytes = fixed + sizeof(float) * 2 * mr + sizeof(LineMeta) * ml;
+    *bytes = fixed + direction_bytes(mr, ml);
     return CCCS_OK;
 }
 
@@ -2538,7 +2551,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             ml = std::max(ml, lines);
         }
         for (size_t i = k0; i < k1; i++) fixed += b_fixed[i];
-        return fixed + (uint64_t)nset * (sizeof(float) * 2 * mr + sizeof(LineMeta) * ml);
+        return fixed + (uint64_t)nset * direction_bytes(mr, ml);
     };
     constexpr uint64_t kMinJob = uint64_t(1) << 30;
     constexpr uint64_t kPartEntries = 1 << 18;  // entries a part of the columns is worth (3 MiB, 60 us of copy)
@@ -2614,8 +2627,7 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
                 ml = std::max(ml, lines[r] + b_lines[k][r]);
             }
             // every direction in flight holds its own REV store, half steps and line table
-            const uint64_t bytes =
-                fixed + b_fixed[k] + (uint64_t)nset * (sizeof(float) * 2 * mr + sizeof(LineMeta) * ml);
+            const uint64_t bytes = fixed + b_fixed[k] + (uint64_t)nset * direction_bytes(mr, ml);
             if (k > next && bytes > budget) break;
             for (int r = 0; r < nrays; r++) {
                 rev[r] += b_rev[k][r];

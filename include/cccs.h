@@ -266,8 +266,9 @@ int cccs_beamlet_dense(cccs_ctx* ctx, const cccs_beam* beam, const float* fluenc
                        float* out, int max_beamlets, int* nactive);
 
 /* Device bytes a cccs_beamlet_dose call for this one beam would hold while it runs (packed
- * grids, one cone direction's REV store, half steps and line table, sparse-output bound); host
- * planning only, no device work.  No counterpart in the reference. */
+ * grids, one cone direction's REV store and half steps with the zeros around their lines, line
+ * tables, sparse-output bound); host planning only, no device work.  No counterpart in the
+ * reference. */
 int cccs_beamlet_footprint(const cccs_ctx* ctx, const cccs_beam* beam, const float* fluence, uint64_t* bytes);
 
 /* ---- serving: a request loop over device-resident contexts ----------------------------------
