@@ -181,6 +181,8 @@ CCCS_HD LineMeta line_interval(const BlArgs& a, const BlConeDev& c, const BatchD
 // scan beyond (three scan launches of their own cost a 32^3 job a tenth of its time).
 constexpr int kLineBlock = 256;
 constexpr uint32_t kWaveBlocks = 64;  // blocks whose totals one wave scans
+// Samples of the store before a line's own, beside the lines before it.
+CCCS_HD uint32_t line_pad(bool zeros, int len) { return zeros && len > 0 ? (uint32_t)kLineZeros : 0u; }
 
 __global__ void __launch_bounds__(kLineBlock) bl_interval_kernel(BlArgs a) {
     __shared__ uint32_t s_w[kLineBlock / 64];
@@ -194,7 +196,7 @@ __global__ void __launch_bounds__(kLineBlock) bl_interval_kernel(BlArgs a) {
         ci = find_cone(a.cones, a.nbatch, line);
         m = line_interval(a, a.cones[ci], a.batches[ci], line);
     }
-    const uint32_t pad = a.zeros && m.len > 0 ? (uint32_t)kLineZeros : 0u, take = (uint32_t)m.len + pad;
+    const uint32_t pad = line_pad(a.zeros, m.len), take = (uint32_t)m.len + pad;
     const uint32_t inc = wave_incl_u32(take);
     if (lane == 63) s_w[w] = inc;
     __syncthreads();
@@ -308,6 +310,40 @@ __device__ __forceinline__ float bl_density(const BlArgs& a, const MarchVol& vol
     return s == s ? tex3_march(vol, gi.x + 0.5f, gi.y + 0.5f, gi.z + 0.5f) : 0.f;
 }
 
+// The affine form of the mapping, in the sample stage: the packed coordinate of sample t of line (tY, tZ) is
+// line_start + t * line_step (matrix rotation).  It only skips samples that are far from every footprint or
+// inside pillars without footprint samples, with margins far above its rounding; the exact mapping decides
+// every other sample.
+CCCS_HD v3 line_start(const BlArgs& a, const BlConeDev& c, int tY, int tZ) {
+    return c.kinv_m(mk3(fmaf(c.minc.x, a.rrv.x, (float)tZ), c.minc.y * a.rrv.y, fmaf(c.minc.z, a.rrv.z, (float)tY))) + 0.5f;
+}
+CCCS_HD v3 line_step(const BlConeDev& c) { return mk3(c.kinv_m.m[1], c.kinv_m.m[4], c.kinv_m.m[7]); }
+
+// Pass A.1's cull of one sample.  First the distance from the nearest beamlet axis, in pillars with the axis at
+// 0.5 (cx, cz: the second test's half-width and 0.05 samples).
+CCCS_HD bool near_axis(bool in, float ux, float uz, float cx, float cz) {
+    return in && fabsf((ux - floorf(ux)) - 0.5f) <= cx && fabsf((uz - floorf(uz)) - 0.5f) <= cz;
+}
+// Then the footprint half-width fw (cull: 0.05 samples wider) and the batch's depth-linear footprint bounds (cb).
+CCCS_HD bool in_foot_bounds(bool near, const BatchDev& B, float px, float py, float pz, float pdx, float pdz, float ipdx,
+                            float ipdz, float cull) {
+    const float xl = px - floorf(px * ipdx) * pdx, zl = pz - floorf(pz * ipdz) * pdz;
+    return near && fabsf(xl - B.fc[0]) <= cull && fabsf(zl - B.fc[1]) <= cull && xl >= B.cb[0] + B.cb[1] * py &&
+           xl <= B.cb[2] + B.cb[3] * py && zl >= B.cb[4] + B.cb[5] * py && zl <= B.cb[6] + B.cb[7] * py;
+}
+
+// Pass B.1: whether a sample at (ux, uz), in pillars, needs the exact mapping: not where it certainly lies in a
+// pillar without a bit in `pil` or outside the grid's pillars (by 0.05 samples; hx, hz: half a pillar less that).
+CCCS_HD bool may_take_dose(bool in, const BatchDev& B, float ux, float uz, float hx, float hz, const uint32_t* pil) {
+    const float fx = floorf(ux), fz = floorf(uz);
+    if (fabsf((ux - fx) - 0.5f) < hx && fabsf((uz - fz) - 0.5f) < hz) {
+        const int px = (int)fx, pa = px + (int)fz * B.npx;
+        const bool grid = (uint32_t)px < (uint32_t)B.npx && fz >= 0.f && pa < B.n;
+        in = in && grid && (pil[grid ? pa >> 5 : 0] >> (pa & 31)) & 1u;
+    }
+    return in;
+}
+
 // Cumulative kernel of one row, linear between radii (the reference's clamped linear texture
 // lookup, nvbbRayConvolve_device.cu:330-352).  Interval s of a row is {lo, K(lo), slope, hi}: the
 // value at r in (lo, hi] is K(lo) + (r - lo) * slope.  s tracks the first radius >= r and r must
@@ -317,7 +353,8 @@ __device__ __forceinline__ float kc_at(float r, const float4* __restrict__ tab, 
     return iv.y + (r - iv.x) * iv.z;
 }
 
-constexpr int kStagePillars = 64;  // footprint pillars of one line that the stage's CPU replay counts as usual
+// Footprint pillars of a line beyond which the host's index audit counts a line apart (the stage has no such limit).
+constexpr int kStagePillars = 64;
 
 __device__ __forceinline__ int lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ float lane_f(float v, int lane) {
@@ -382,11 +419,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
         const uint64_t l = my_line - c.line0;
         my_z = (int)(l / (uint64_t)c.ny);
         my_y = (int)(l - (uint64_t)my_z * (uint64_t)c.ny);
-        // affine form of the packed coordinate along the line (matrix rotation): used only to skip
-        // samples that are far from every footprint or inside pillars without footprint samples; the
-        // exact mapping decides every other sample
-        my_p0 = c.kinv_m(mk3(fmaf(c.minc.x, a.rrv.x, (float)my_z), c.minc.y * a.rrv.y,
-                             fmaf(c.minc.z, a.rrv.z, (float)my_y))) + 0.5f;
+        my_p0 = line_start(a, c, my_y, my_z);
         if (mine.len > 0) stored += (uint32_t)mine.len;  // summed over the wave's lanes by wave_count
     }
     {
@@ -406,10 +439,9 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
         {
             const BlConeDev c = uniform_copy(pc);
             const BatchDev B = uniform_copy(pB);
-            const v3 dl = mk3(c.kinv_m.m[1], c.kinv_m.m[4], c.kinv_m.m[7]);
+            const v3 dl = line_step(c);
             const float pdx = (float)B.pd[0], pdz = (float)B.pd[2], ipdx = B.ipd[0], ipdz = B.ipd[2];
             const float cull = B.fw + 0.05f;
-            // the distance from the nearest beamlet axis in pillars (0.05 samples wider than the cull)
             const float dux = dl.x * ipdx, duz = dl.z * ipdz, cx = (cull + 0.05f) * ipdx, cz = (cull + 0.05f) * ipdz;
             while (todo) {
                 const int k = __builtin_ctzll(todo);
@@ -424,15 +456,9 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
                 for (int j0 = 0; j0 < m; j0 += 64) {
                     const float t = t0 + (float)j0;
                     const float ux = fmaf(t, dux, ux0), uz = fmaf(t, duz, uz0);
-                    bool cand = tid < m - j0 && fabsf((ux - floorf(ux)) - 0.5f) <= cx &&
-                                fabsf((uz - floorf(uz)) - 0.5f) <= cz;
+                    bool cand = near_axis(tid < m - j0, ux, uz, cx, cz);
                     if (!__ballot(cand)) continue;
-                    // the footprint half-width fw and the batch's depth-linear footprint bounds (cb)
-                    const float px = px0 + t * dl.x, pz = pz0 + t * dl.z, py = py0 + t * dl.y;
-                    const float xl = px - floorf(px * ipdx) * pdx, zl = pz - floorf(pz * ipdz) * pdz;
-                    cand = cand && fabsf(xl - B.fc[0]) <= cull && fabsf(zl - B.fc[1]) <= cull &&
-                           xl >= B.cb[0] + B.cb[1] * py && xl <= B.cb[2] + B.cb[3] * py &&
-                           zl >= B.cb[4] + B.cb[5] * py && zl <= B.cb[6] + B.cb[7] * py;
+                    cand = in_foot_bounds(cand, B, px0 + t * dl.x, py0 + t * dl.y, pz0 + t * dl.z, pdx, pdz, ipdx, ipdz, cull);
                     const uint64_t mask = __ballot(cand);
                     if (cand) s_cand[ncand + __popcll(mask & lt)] = (uint16_t)(k << 10 | (j0 + tid));
                     ncand += __popcll(mask);
@@ -529,13 +555,7 @@ __global__ void __launch_bounds__(64) bl_sample_kernel(BlArgs a, float* __restri
                     bool exact = j < m;
                     if (track) {
                         const float t = (float)(i0 + j);
-                        const float ux = fmaf(t, dux, ux0), uz = fmaf(t, duz, uz0);
-                        const float fx = floorf(ux), fz = floorf(uz);
-                        if (fabsf((ux - fx) - 0.5f) < hx && fabsf((uz - fz) - 0.5f) < hz) {
-                            const int px = (int)fx, pa = px + (int)fz * B.npx;
-                            const bool grid = (uint32_t)px < (uint32_t)B.npx && fz >= 0.f && pa < B.n;
-                            exact = exact && grid && (s_pil[grid ? pa >> 5 : 0] >> (pa & 31)) & 1u;
-                        }
+                        exact = may_take_dose(exact, B, fmaf(t, dux, ux0), fmaf(t, duz, uz0), hx, hz, s_pil);
                     }
                     const uint64_t mask = __ballot(exact);
                     if (tid == 0) s_exact[j0 >> 6] = mask;
