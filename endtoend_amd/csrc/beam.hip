@@ -448,8 +448,9 @@ CCCS_HD int ramp_find(const RampLine& L, float y) {
     const RampPos p = ramp_probe<kUpper>(L, y);
     return p.more ? ramp_more<kUpper>(L, y, p) : p.k;
 }
-// Lines whose cells are too fine for FP32 lookups (the first half step dwarfs the rest of the line:
-// cells of less than 1/20 of the samples' mean share of c_{n-1}) keep one cell and search in it.
+// Cells per cm over [c_0, c_{n-1}].  c_0 is half of the first sample and c_{n-1} at least all of it, so two samples
+// or more span at least half of c_{n-1} and their 2n cells are never too fine for FP32 lookups; one sample, and a
+// line without density, keep one cell (a margin of ten below that half).
 CCCS_HD float ramp_cells(float c0, float cn, int U) { return cn - c0 > 0.05f * cn ? (float)U / (cn - c0) : 0.f; }
 
 // Lanes of a wave leave the walk together, so that its body runs without masks.
