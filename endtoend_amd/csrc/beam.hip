@@ -715,8 +715,8 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
     const int nr = a.nradii;
     uint32_t iters = 0;
     // the radial steps go to LDS past the resample, so their latency overlaps the gathers
-    RampStep step{};
-    if (tid < nr) step = a.steps[(size_t)rowf * nr + tid];
+    const RampStep* my_step = a.steps + ((size_t)rowf * nr + min(tid, nr - 1));
+    const double step_r = my_step->r, step_b = my_step->sigb, step_f = my_step->sigf;
     {
         const bool ramp_lds = a.ramp_min <= a.maxn;
         // LDS: [E | E2 | c | line | lb] with the segment-sum arrays, else [line]
@@ -782,7 +782,11 @@ __global__ void __launch_bounds__(NT) cone_kernel(ConeArgs a) {
             }
         }
         nvalid -= nbad;
-        if (tid < nr) s_steps[tid] = step;
+        if (tid < nr) {
+            s_steps[tid].r = step_r;
+            s_steps[tid].sigb = step_b;
+            s_steps[tid].sigf = step_f;
+        }
         if (NW > 1 && lane == 0) {
             s_red[wid][0] = vlo;
             s_red[wid][1] = vhi;
