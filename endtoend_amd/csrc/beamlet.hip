@@ -1045,8 +1045,12 @@ __global__ void __launch_bounds__(256) bl_unpack_kernel(UnpackArgs a) {
 //
 // One workgroup per beamlet left most of the device idle (a job has some 400 beamlets, their boxes up
 // to 150 chunks of rows each) and made every pass a chain of its chunks; the three passes took 0.93 ms
-// (one 5 mm beam, 128^3 water), 4.1 ms (thorax, 3 beams) and 110 us (32^3 water), by chunks 0.34 ms,
-// 1.31 ms and 37 us.
+// (one 5 mm beam, 128^3 water), 4.1 ms (thorax, 3 beams) and 110 us (32^3 water), by chunks 0.35 ms, 1.4 ms and
+// 36 us.  The max and count passes issue VALU in all of their cycles.  The emission's launch lasts as long as its
+// longest row, a serial chain of one lane (0.23 of VALU issue at one wave per SIMD for the one beam), so a job
+// emits all its columns in one launch: by parts of the columns, as they go to the host, it took 1.76 ms of
+// eight launches instead of 0.17 ms (one beam), 3.5 instead of 0.56 ms (thorax) and 6.1 instead of 0.88 ms (two
+// fine 4pi beams).
 
 struct ColArgs {
     const BatchDev* batches;
@@ -2290,7 +2294,6 @@ struct RoiArgs {
     const uint64_t* roff;        // [column][roi] first reduced entry (exclusive scan of cnt)
     uint64_t* rkeys;
     float* rvals;
-    int col0;                    // first column of this launch
 };
 
 // ROI rank of CT voxel `key` in ROI r (or -1).
@@ -2304,7 +2307,7 @@ __device__ __forceinline__ int32_t roi_rank(const RoiArgs& a, const RoiDev& R, i
 // chunk and ROI).
 __global__ void __launch_bounds__(256) roi_count_kernel(RoiArgs a) {
     __shared__ uint32_t s_c[kMaxRoi];
-    const int q = a.col0 + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int q = (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     for (int r = tid; r < a.nroi; r += 256) s_c[r] = 0u;
     __syncthreads();
     const uint64_t e0 = a.off[q], e1 = a.off[q + 1];
@@ -2332,7 +2335,7 @@ __global__ void __launch_bounds__(256) roi_count_kernel(RoiArgs a) {
 // order-preserving compaction per 256-entry chunk), keyed mark + rank.
 __global__ void __launch_bounds__(256) roi_emit_kernel(RoiArgs a) {
     __shared__ uint32_t s_w[4];
-    const int q = a.col0 + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int q = (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const uint64_t e0 = a.off[q], e1 = a.off[q + 1];
     const uint64_t plane = (uint64_t)a.nx * (uint64_t)a.ny;
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -2700,15 +2703,15 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
                            reinterpret_cast<float*>(stat), 4 * (uint64_t)nbl, 0.f);
         // one launch takes as many beamlets as its workgroups allow: jobs of many small boxes and a few huge
         // ones have more than kMaxGroups chunks (a single box never does: it has fewer than 2^32 rows)
-        auto over = [&](int b0, int b1, void (*kernel)(ColArgs)) {
+        auto over = [&](void (*kernel)(ColArgs)) {
             const int per = (int)std::max<uint32_t>(1, kMaxGroups / (uint32_t)chunks);
-            for (int b = b0; b < b1; b += per) {
+            for (int b = 0; b < nbl; b += per) {
                 ca.beamlet0 = b;
-                hipLaunchKernelGGL(kernel, dim3((unsigned)(std::min(per, b1 - b) * chunks)), dim3(256), 0, ctx->stream, ca);
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(std::min(per, nbl - b) * chunks)), dim3(256), 0, ctx->stream, ca);
             }
         };
-        over(0, nbl, bl_colmax_kernel);
-        over(0, nbl, bl_colcount_kernel);
+        over(bl_colmax_kernel);
+        over(bl_colcount_kernel);
         prof_end(ctx, tok, 0.0, 0.0, (uint64_t)nbl);
         hipLaunchKernelGGL(bl_offsets_kernel, dim3(1), dim3(1024), 0, ctx->stream, stat, nbl, offs);
         CCCS_HIP(hipGetLastError());
@@ -2728,14 +2731,13 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
         CCCS_TRY(ctx->bl_vals.ensure(sizeof(float) * std::max<uint64_t>(1, nnz_total)));
         ca.keys = ctx->bl_keys.as<uint64_t>();
         ca.vals = ctx->bl_vals.as<float>();
-        auto emit = [&](int b0, int b1) { over(b0, b1, bl_emit_kernel); };
         // ROI reduction of the job's columns (count, scan, order-preserving emit)
         RoiArgs ra;
         const uint64_t* out_off = hoff;  // first output entry of every column
         std::vector<uint64_t> roi_off;
         if (nroi > 0) {
             int tk = prof_begin(ctx, K_BL_COMPACT);
-            emit(0, nbl);
+            over(bl_emit_kernel);
             // algorithmic traffic: the kept entries (8 B key + 4 B value)
             prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
             CCCS_HIP(hipGetLastError());
@@ -2754,7 +2756,6 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             ra.roff = roff;
             ra.rkeys = nullptr;
             ra.rvals = nullptr;
-            ra.col0 = 0;
             hipLaunchKernelGGL(roi_count_kernel, dim3(nbl), dim3(256), 0, ctx->stream, ra);
             hipLaunchKernelGGL(roi_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, (const uint32_t*)rcnt, ncr, roff);
             CCCS_HIP(hipGetLastError());
@@ -2771,63 +2772,59 @@ extern "C" int cccs_beamlet_dose(cccs_ctx* ctx, const cccs_beam* beams, int nbea
             ra.rvals = ctx->roi_vals.as<float>();
         }
         const uint64_t nout = out_off[nbl];
-        // columns to pinned host memory (full PCIe rate, one of two buffers in turn); the sink sees
-        // them in place, during the next job or at the end of the call.  They go in parts of about
-        // equal size: while the sink takes one part, the next ones are emitted and copied.  The copies
-        // run on their own stream: the next job's cone passes, queued behind this compaction, do not
-        // wait for them; the next compaction waits before rewriting the buffers.
-        const int nparts = !sink ? 1 : (int)std::min<uint64_t>(kColParts, std::max<uint64_t>(1, nout / kPartEntries));
-        Delivery& D = pending;
-        if (sink) {
-            const size_t kbytes = sizeof(uint64_t) * nout;
-            HostBuf& hbuf = (njob & 1) ? ctx->h_bl_out2 : ctx->h_bl_out;
-            CCCS_TRY(hbuf.ensure(kbytes + sizeof(float) * nout + 64));
-            D.keys = hbuf.as<uint64_t>();
-            D.vals = reinterpret_cast<float*>(hbuf.as<uint8_t>() + kbytes);
-            D.stat = reinterpret_cast<const uint32_t*>(hs);
-            D.rcnt = reinterpret_cast<const uint32_t*>(hs + o_chunk);
-            D.nroi = nroi;
-            D.cols.resize((size_t)nbl);
-            for (int q = 0; q < nbl; q++) {
-                const BeamletDev& d = J.beamlets[q];
-                D.cols[(size_t)q] = {plans[sel[d.batch].plan].beam, d.fidx};
-            }
-            D.nparts = nparts;
-        }
+        // All columns in one launch: a launch lasts as long as its longest row, one lane's serial chain, however
+        // few columns it has.
         int tk = nroi > 0 ? -1 : prof_begin(ctx, K_BL_COMPACT);
+        if (nroi > 0) hipLaunchKernelGGL(roi_emit_kernel, dim3(nbl), dim3(256), 0, ctx->stream, ra);
+        else over(bl_emit_kernel);
+        if (nroi == 0) prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
+        CCCS_HIP(hipGetLastError());
+        if (!sink) continue;  // columns stay on the device (overwritten by the next job)
+        // Columns to pinned host memory (full PCIe rate, one of two buffers in turn); the sink sees them in
+        // place, during the next job or at the end of the call.  They go in parts of about equal size: while
+        // the sink takes one part, the next ones are copied.  The copies run on their own stream: the next
+        // job's cone passes, queued behind this compaction, do not wait for them; the next compaction waits
+        // before rewriting the buffers.
+        const int nparts = (int)std::min<uint64_t>(kColParts, std::max<uint64_t>(1, nout / kPartEntries));
+        const size_t kbytes = sizeof(uint64_t) * nout;
+        HostBuf& hbuf = (njob & 1) ? ctx->h_bl_out2 : ctx->h_bl_out;
+        CCCS_TRY(hbuf.ensure(kbytes + sizeof(float) * nout + 64));
+        Delivery& D = pending;
+        D.keys = hbuf.as<uint64_t>();
+        D.vals = reinterpret_cast<float*>(hbuf.as<uint8_t>() + kbytes);
+        D.stat = reinterpret_cast<const uint32_t*>(hs);
+        D.rcnt = reinterpret_cast<const uint32_t*>(hs + o_chunk);
+        D.nroi = nroi;
+        D.cols.resize((size_t)nbl);
+        for (int q = 0; q < nbl; q++) {
+            const BeamletDev& d = J.beamlets[q];
+            D.cols[(size_t)q] = {plans[sel[d.batch].plan].beam, d.fidx};
+        }
+        D.nparts = nparts;
+        const uint64_t* sk = (nroi > 0 ? ctx->roi_keys : ctx->bl_keys).as<uint64_t>();
+        const float* sv = (nroi > 0 ? ctx->roi_vals : ctx->bl_vals).as<float>();
+        hipStream_t cs = ctx->cstream;
         for (int part = 0, b0 = 0; part < nparts; part++) {
             int b1 = nbl;
             if (part + 1 < nparts)
                 b1 = (int)(std::lower_bound(out_off + b0, out_off + nbl, nout / nparts * (part + 1)) - out_off);
-            if (nroi > 0) {
-                ra.col0 = b0;
-                if (b1 > b0) hipLaunchKernelGGL(roi_emit_kernel, dim3(b1 - b0), dim3(256), 0, ctx->stream, ra);
-            } else {
-                emit(b0, b1);
-            }
-            CCCS_HIP(hipGetLastError());
-            if (sink) {
-                hipStream_t cs = ctx->cstream;
-                hipEvent_t ev = ctx->col_ev[(njob & 1) * kColParts + part];
-                const uint64_t e0 = out_off[b0], n = out_off[b1] - e0;
+            hipEvent_t ev = ctx->col_ev[(njob & 1) * kColParts + part];
+            if (part == 0) {
                 CCCS_HIP(hipEventRecord(ev, ctx->stream));
                 CCCS_HIP(hipStreamWaitEvent(cs, ev, 0));
                 drain.queued = true;
-                if (n) {
-                    const uint64_t* sk = (nroi > 0 ? ctx->roi_keys : ctx->bl_keys).as<uint64_t>();
-                    const float* sv = (nroi > 0 ? ctx->roi_vals : ctx->bl_vals).as<float>();
-                    CCCS_HIP(hipMemcpyAsync(D.keys + e0, sk + e0, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, cs));
-                    CCCS_HIP(hipMemcpyAsync(D.vals + e0, sv + e0, sizeof(float) * n, hipMemcpyDeviceToHost, cs));
-                }
-                CCCS_HIP(hipEventRecord(ev, cs));
-                D.ev[part] = ev;
-                D.end[part] = (size_t)b1;
-                copy_done = ev;
             }
+            const uint64_t e0 = out_off[b0], n = out_off[b1] - e0;
+            if (n) {
+                CCCS_HIP(hipMemcpyAsync(D.keys + e0, sk + e0, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, cs));
+                CCCS_HIP(hipMemcpyAsync(D.vals + e0, sv + e0, sizeof(float) * n, hipMemcpyDeviceToHost, cs));
+            }
+            CCCS_HIP(hipEventRecord(ev, cs));
+            D.ev[part] = ev;
+            D.end[part] = (size_t)b1;
+            copy_done = ev;
             b0 = b1;
         }
-        if (nroi == 0) prof_end(ctx, tk, 12.0 * (double)nnz_total, 0.0, nnz_total);
-        if (!sink) continue;  // columns stay on the device (overwritten by the next job)
         D.live = true;
         njob++;
     }
