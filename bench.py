@@ -177,7 +177,7 @@ def plain_beam_path(steps: int = 2, autotune: bool = False):
     return {"workload": "200x200x160 thorax @ 2 mm, 20 coplanar beams, 40x40 x 5 mm U[0,1] fluence masked "
                         "to the PTV, full-beam dose", "value": w.active_beamlets / dt, "unit": "beamlet-doses/s",
             "ms_per_plan": 1e3 * dt, "latency_ms": {"p50": _percentile(lat, 50), "p99": _percentile(lat, 99)},
-            "kernels": _kernels(prof), "roofline_cone": roofline_row(prof, "cone", "cone_64"), "schedule": tune}
+            "kernels": _kernels(prof), "roofline_cone": roofline_row(prof, "cone"), "schedule": tune}
 
 
 def full_4pi(stride: int = 12, rate: float = 20.0, requests: bool = True):
@@ -533,7 +533,7 @@ def main():
     # per-kernel times: one step with one cone direction in flight, so that no two kernels share
     # the device and the kernel times add up to no more than that step.  Alone on the device the
     # sample stage runs at its standalone best, 4 waves per SIMD (4096 waves); the headline
-    # keeps it at 2 waves per SIMD so that the other directions' stages run beside it.
+    # keeps it at 3 waves per SIMD (3072) so that the other directions' stages run beside it.
     nstreams = eng.get_schedule("bl_streams")
     swaves = eng.get_schedule("bl_sample_waves")
     alone = {"bl_streams": 1, "bl_sample_waves": 4096}

@@ -95,8 +95,10 @@ CCCS_HD v3 terma_point(const TermaArgs& a, int X, int Y, int Z) {
 // its voxel is deep, so the deepest planes along the beam's main axis start first and the short
 // rays fill the end; workgroups with and without field mix, so at most kTermaResident share a CU and
 // the rest go where one ends.  Those two and the cheap test of the field below: thorax at 54, 90 and 3
-// degrees 400, 220 and 243 -> 380, 176 and 182 us, 128^3 water 118 -> 95 us (without the bound 102;
-// five a CU: 398, 196, 215 and 83).
+// degrees 400, 220 and 243 -> 380, 176 and 182 us, 128^3 water 118 -> 95 us.  Four to eight a CU take 139,
+// 137, 136, 138 and 144 us a beam over the 20 beams of a thorax plan, 85, 85, 94, 108 and 154 us for the 128^3
+// water beam and 22 us each for a 32^3 one: six is the plan's best, by a hundredth, and water's runs of
+// full workgroups would have fewer.
 constexpr int kTermaResident = 6;
 __device__ __forceinline__ void terma_voxel(const TermaArgs& a, int& X, int& Y, int& Z) {
     const uint32_t nx = (uint32_t)(a.bx + 15) / 16, ny = (uint32_t)(a.by + 3) / 4, nz = (uint32_t)(a.bz + 3) / 4;
@@ -1777,8 +1779,10 @@ int run_cones(BeamScratch& S, const cccs_beam& b, const float* d_terma, float* d
     CCCS_TRY(S.get(ctx->cls_cnt, (size_t)ncb * kClassCols + kClassCols, &cl.bcnt));
     cl.tot = cl.bcnt + (size_t)ncb * kClassCols;
     // The launches and the store are sized from the totals on the host.  Small beams take the bounds
-    // instead (empty workgroups and some megabytes cost less than the wait: 32^3 water beam 115 against
-    // 124 us); their cone launch reads its count on the device.
+    // instead; their cone launch reads its count on the device.  The wait costs 10 to 12 us at every size
+    // measured (8 to 48 cones on grids of 16^3 to 64^3, 2500 to 115000 lines of up to 96 samples: 97 against 87 us
+    // the smallest, 338 against 327 the largest); the bounds below keep the empty workgroups below 32768 and the
+    // store, dense, at 64 MiB.
     const bool wait = S.arena || ctx->prof.on || ncls != 1 || g.total_lines > 32768 || g.total_rev > (uint64_t(1) << 24);
     uint32_t* totals = reinterpret_cast<uint32_t*>(S.host_small + 8);
     cl.host = wait && !S.arena ? totals : nullptr;

@@ -1,5 +1,5 @@
-// context.hip -- the resident device context (cccs_ctx), device buffers, per-kernel profiling,
-// the line-table scan shared by the cone pipelines, and the context/memory C-ABI.
+// context.hip -- the resident device context (cccs_ctx), device buffers, per-kernel profiling and the
+// context/memory C-ABI.
 // Replaces the per-device static arrays, textures and memory accounting of initCudaConstandTex /
 // freeCudaTexture (CCCS/dosecalc-beam/nvbbRayConvolve_host.cu:27-54, 158-293, 745-771;
 // CCCS/CudaUtilities/memory_manager.cu:7-68).

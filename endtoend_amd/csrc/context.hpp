@@ -114,9 +114,9 @@ struct Schedule {
     int cone_class_threads[kConeClasses] = {64, 64, 128, 128};
     // waves of the beamlet path's persistent per-line kernels (each takes a stride of lines).  The
     // sample stage holds 3 waves per SIMD: with several cone directions in flight, the other
-    // streams' Siddon, walk and gather waves run beside it (its own 5-wave occupancy would take
-    // every register of the SIMD).  The walk's waves share a table that each loads first: whole calls
-    // with 8192 to 16384 run 1 to 2 % faster than with 32768, with 2048 slower
+    // streams' Siddon, walk and gather waves run beside it (at its own occupancy of 4 waves, with 116
+    // VGPRs, it would take nearly every register of the SIMD).  The walk's waves share a table that each
+    // loads first: whole calls with 8192 to 16384 run 1 to 2 % faster than with 32768, with 2048 slower
     int bl_sample_waves = 3072;
     int bl_walk_waves = 16384;
     // device memory of one beamlet job [GiB]: batches join a job while its packed grids, output
