@@ -987,6 +987,12 @@ __global__ void __launch_bounds__(256) bl_tile_batch_kernel(const BatchDev* __re
     for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) tb[B.tile0 + t] = (uint32_t)b;
 }
 
+// A job's tables from pinned host memory.  (An upload would wait for its copy engine behind the columns of the job
+// before, some 6 ms of copies for 27 million entries, and the whole job behind it.)
+__global__ void __launch_bounds__(256) bl_table_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, uint32_t n) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
 __global__ void __launch_bounds__(256) bl_fill_kernel(float* __restrict__ p, uint64_t n, float v) {
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) p[i] = v;
 }
@@ -1046,11 +1052,11 @@ __global__ void __launch_bounds__(256) bl_unpack_kernel(UnpackArgs a) {
 // One workgroup per beamlet left most of the device idle (a job has some 400 beamlets, their boxes up
 // to 150 chunks of rows each) and made every pass a chain of its chunks; the three passes took 0.93 ms
 // (one 5 mm beam, 128^3 water), 4.1 ms (thorax, 3 beams) and 110 us (32^3 water), by chunks 0.35 ms, 1.4 ms and
-// 36 us.  The max and count passes issue VALU in all of their cycles.  The emission's launch lasts as long as its
-// longest row, a serial chain of one lane (0.23 of VALU issue at one wave per SIMD for the one beam), so a job
-// emits all its columns in one launch: by parts of the columns, as they go to the host, it took 1.76 ms of
-// eight launches instead of 0.17 ms (one beam), 3.5 instead of 0.56 ms (thorax) and 6.1 instead of 0.88 ms (two
-// fine 4pi beams).
+// 36 us.  The max and count passes issue VALU in all of their cycles, the emission in 0.77 (one beam) and 0.68
+// (thorax).  The emission's launch lasts no less than its longest row, a serial chain of one lane, so a job emits
+// all its columns in one launch: by parts of the columns, as they go to the host, it took 1.76 ms of eight
+// launches (0.23 of VALU issue) instead of 0.17 ms (one beam), 3.5 instead of 0.56 ms (thorax) and 6.1 instead of
+// 0.88 ms (two fine 4pi beams).
 
 struct ColArgs {
     const BatchDev* batches;
@@ -1811,7 +1817,7 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     const size_t sz_b = sizeof(BatchDev) * nb, sz_l = sizeof(BeamletDev) * J.beamlets.size(),
                  sz_c = sizeof(BlConeDev) * J.cones.size();
     const size_t o_l = (sz_b + 255) & ~size_t(255), o_c = (o_l + sz_l + 255) & ~size_t(255);
-    const size_t total = o_c + sz_c;
+    const size_t total = (o_c + sz_c + 15) & ~size_t(15);
     CCCS_TRY(ctx->bl_tab.ensure(total));
     CCCS_HIP(hipStreamSynchronize(ctx->stream));  // the pinned staging buffer may still be in use
     CCCS_TRY(ctx->h_bl.ensure(total));
@@ -1820,7 +1826,9 @@ int run_job_cones(cccs_ctx* ctx, const Job& J, const std::function<int()>& while
     std::memcpy(h + o_l, J.beamlets.data(), sz_l);
     std::memcpy(h + o_c, J.cones.data(), sz_c);
     uint8_t* d = ctx->bl_tab.as<uint8_t>();
-    CCCS_HIP(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(bl_table_kernel, dim3((unsigned)std::min<size_t>(1024, (total / 16 + 255) / 256)), dim3(256), 0,
+                       ctx->stream, reinterpret_cast<uint4*>(d), reinterpret_cast<const uint4*>(h), (uint32_t)(total / 16));
+    CCCS_HIP(hipGetLastError());
     CCCS_TRY(ctx->bl_pdose.ensure(sizeof(float) * std::max<uint64_t>(1, J.pdose)));
     CCCS_TRY(ctx->lines.ensure(line_bytes(J.max_lines)));
     // (the zeros around every line count as samples of the store)
